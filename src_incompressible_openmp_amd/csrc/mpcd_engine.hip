@@ -1143,73 +1143,44 @@ __device__ __forceinline__ void zone_finish_body(const ZoneArgs& a, const ZoneIn
     } else {
         zone_attach_state(z, st);
     }
-    if (kLds && hand) {
+    if (kLds) {
         unsigned char* p = lds;
-        IT* cnt = (IT*)p; p += (size_t)z.C * sizeof(IT);
-        IT* head = (IT*)p; p += (size_t)z.C * sizeof(IT);
-        IT* tail = (IT*)p; p += (size_t)z.C * sizeof(IT);
+        ZCell<IT>* cell = (ZCell<IT>*)p; p += (size_t)z.C * sizeof(ZCell<IT>);
         IT* k0 = (IT*)p; p += (size_t)z.C * sizeof(IT);
-        unsigned short* fl = (unsigned short*)p; p += (size_t)z.C * sizeof(unsigned short);
         p = lds + (((size_t)(p - lds) + 3) & ~(size_t)3);
         int* colL = (int*)p; p += (size_t)z.zw * sizeof(int);
         int* colG = (int*)p; p += (size_t)z.zw * sizeof(int);
         IT* links = (IT*)p;
         const long long room = (ldsBytes - (long long)(p - lds)) / (long long)sizeof(IT);
         const int nL = (int)(room < (long long)z.P ? (room > 0 ? room : 0) : z.P);
-        /* the passes' links k < hand->nL, behind their scratch, move down in
-         * chunks no longer than the distance they move, so a chunk overwrites
-         * only links earlier chunks have copied; the rest come from the
-         * zone's global link region */
-        const IT* src = (const IT*)(lds + zone_fixed_bytes<IT>(z.C, z.zw, z.zp.useLocal));
-        const int gap = (int)(src - links);
-        const int nP = hand->nL < nL ? hand->nL : nL;
-        for (int c0 = 0; c0 < nP; c0 += gap) {
-            const int c1 = c0 + gap < nP ? c0 + gap : nP;
-            for (int k = c0 + tid; k < c1; k += TPB) links[k] = src[k];
-            __syncthreads();
+        if (hand) {
+            /* the passes' links k < hand->nL, behind their scratch, move down in
+             * chunks no longer than the distance they move, so a chunk overwrites
+             * only links earlier chunks have copied; the rest come from the
+             * zone's global link region */
+            const IT* src = (const IT*)(lds + zone_fixed_bytes<IT>(z.C, z.zw, z.zp.useLocal));
+            const int gap = (int)(src - links);
+            const int nP = hand->nL < nL ? hand->nL : nL;
+            for (int c0 = 0; c0 < nP; c0 += gap) {
+                const int c1 = c0 + gap < nP ? c0 + gap : nP;
+                for (int k = c0 + tid; k < c1; k += TPB) links[k] = src[k];
+                __syncthreads();
+            }
+            for (int k = nP + tid; k < nL; k += TPB) links[k] = z.nxG[k];
+        } else {
+            /* the state and the first links to LDS */
+            for (int lc = tid; lc < z.C; lc += TPB) {
+                cell[lc] = st.cell[lc];
+                k0[lc] = st.k0[lc];
+            }
+            for (int c = tid; c < z.zw; c += TPB) {
+                colL[c] = st.colL[c];
+                colG[c] = st.colG[c];
+            }
+            for (int k = tid; k < nL; k += TPB) links[k] = z.nxG[k];
         }
-        for (int k = nP + tid; k < nL; k += TPB) links[k] = z.nxG[k];
-        z.cnt = cnt;
-        z.head = head;
-        z.tail = tail;
+        z.cell = cell;
         z.k0 = k0;
-        z.fl = fl;
-        z.colL = colL;
-        z.colG = colG;
-        z.nxL = links;
-        z.nL = nL;
-        __syncthreads();
-    } else if (kLds) {
-        /* the state and the first links to LDS */
-        unsigned char* p = lds;
-        IT* cnt = (IT*)p; p += (size_t)z.C * sizeof(IT);
-        IT* head = (IT*)p; p += (size_t)z.C * sizeof(IT);
-        IT* tail = (IT*)p; p += (size_t)z.C * sizeof(IT);
-        IT* k0 = (IT*)p; p += (size_t)z.C * sizeof(IT);
-        unsigned short* fl = (unsigned short*)p; p += (size_t)z.C * sizeof(unsigned short);
-        p = lds + (((size_t)(p - lds) + 3) & ~(size_t)3);
-        int* colL = (int*)p; p += (size_t)z.zw * sizeof(int);
-        int* colG = (int*)p; p += (size_t)z.zw * sizeof(int);
-        IT* links = (IT*)p;
-        const long long room = (ldsBytes - (long long)(p - lds)) / (long long)sizeof(IT);
-        const int nL = (int)(room < (long long)z.P ? (room > 0 ? room : 0) : z.P);
-        for (int lc = tid; lc < z.C; lc += TPB) {
-            cnt[lc] = st.cnt[lc];
-            head[lc] = st.head[lc];
-            tail[lc] = st.tail[lc];
-            k0[lc] = st.k0[lc];
-            fl[lc] = st.fl[lc];
-        }
-        for (int c = tid; c < z.zw; c += TPB) {
-            colL[c] = st.colL[c];
-            colG[c] = st.colG[c];
-        }
-        for (int k = tid; k < nL; k += TPB) links[k] = z.nxG[k];
-        z.cnt = cnt;
-        z.head = head;
-        z.tail = tail;
-        z.k0 = k0;
-        z.fl = fl;
         z.colL = colL;
         z.colG = colG;
         z.nxL = links;
@@ -2549,8 +2520,8 @@ struct mpcd_gpu_sim {
         const size_t fix16 = zone_fixed_bytes<uint16_t>(maxC, maxW, zp.useLocal);
         const bool fast = maxC < 65535 && fix16 + 2048 <= (size_t)ZONE_LDS_FAST;
         /* LDS staging of the correction: the cell arrays and the column map leave room for links */
-        const size_t cellB16 = (size_t)maxC * (4 * sizeof(uint16_t) + 2) + 8 * (size_t)maxW + 16;
-        const size_t cellB32 = (size_t)maxC * (4 * sizeof(int) + 2) + 8 * (size_t)maxW + 16;
+        const size_t cellB16 = (size_t)maxC * (sizeof(ZCell<uint16_t>) + sizeof(uint16_t)) + 8 * (size_t)maxW + 16;
+        const size_t cellB32 = (size_t)maxC * (sizeof(ZCell<int>) + sizeof(int)) + 8 * (size_t)maxW + 16;
         /* passes and correction in one kernel when the correction fits the passes' LDS */
         const bool fused = fast && cellB16 + 4096 <= (size_t)ZONE_LDS_FAST;
         if (fast) {

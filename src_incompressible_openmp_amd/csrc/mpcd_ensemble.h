@@ -599,7 +599,7 @@ struct mpcd_gpu_ensemble {
         narrow = maxN < (1 << 27) ? 1 : 0;
         /* the fused zone kernel on 16-bit working sets must take every zone */
         const size_t fix16 = zone_fixed_bytes<uint16_t>(maxC, maxW, anyLocal);
-        const size_t cellB16 = (size_t)maxC * (4 * sizeof(uint16_t) + 2) + 8 * (size_t)maxW + 16;
+        const size_t cellB16 = (size_t)maxC * (sizeof(ZCell<uint16_t>) + sizeof(uint16_t)) + 8 * (size_t)maxW + 16;
         if (!(maxC < 65535 && fix16 + 2048 <= (size_t)ZONE_LDS_FAST && cellB16 + 4096 <= (size_t)ZONE_LDS_FAST))
             throw ApiError(MPCD_E_INVALID, "ensemble zones must fit the fused zone kernel (zone tiles too large)");
         HIP_OK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));

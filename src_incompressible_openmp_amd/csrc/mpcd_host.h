@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -168,6 +169,17 @@ inline ZoneParams make_zone_params(const mpcd_params& p) {
             if (idx < 21) zp.binLo |= (unsigned long long)ib << (3 * idx);
             else zp.binHi |= (unsigned long long)ib << (3 * (idx - 21));
         }
+    int perBin[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int idx = 0; idx < 25; ++idx)
+        if (idx != 12) ++perBin[zone_bin(zp, idx)];
+    bool apart = true; /* the offsets of a bin differ in (Chebyshev, squared) distance */
+    for (int a = 0; a < 25; ++a)
+        for (int b = 0; b < a; ++b) {
+            if (a == 12 || b == 12 || zone_bin(zp, a) != zone_bin(zp, b)) continue;
+            const int ax = std::abs(a % 5 - 2), ay = std::abs(a / 5 - 2), bx = std::abs(b % 5 - 2), by = std::abs(b / 5 - 2);
+            if (std::max(ax, ay) == std::max(bx, by) && ax * ax + ay * ay == bx * bx + by * by) apart = false;
+        }
+    zp.quadBins = !zp.dedupe && apart && *std::max_element(perBin, perBin + 8) <= 3;
     return zp;
 }
 

@@ -37,11 +37,14 @@
  * zone covers; for cells several zones cover they go to vsx/vsy and are
  * copied back after the pass, so every zone reads inputs.
  *
- * Lists.  A cell's list stays implicit -- a run of consecutive local
- * indices head..tail, initially its input run -- while only its head is
- * popped; the first append or rewrite writes its links (ZF_MAT).  ZF_CHG
- * marks every cell whose list changed; the others cost nothing at the
- * correction.
+ * Lists.  A cell's list starts as its input run, consecutive local indices
+ * k0..run_end.  What is left of the run stays implicit (pops only move the
+ * head along it) and arrivals are linked behind it: the run's last entry
+ * links to the first arrival, each arrival to the next.  An append thus
+ * writes two links, however long the run is.  A list that is reordered (a
+ * sparse donor's), or that takes back a particle of its own run, has every
+ * link written (ZF_MAT).  ZF_CHG marks every cell whose list changed; the
+ * others cost nothing at the correction.
  */
 #pragma once
 
@@ -88,6 +91,10 @@ ZHD int wave_shfl_up_add(int v, int lane) {
 ZHD int wave_bcast(int v, int src) { return __shfl(v, src, 64); }
 /* value of lane l (l uniform across the wavefront) */
 ZHD int wave_readlane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+/* v with lane l's value replaced by s (s and l uniform): the compiler has the
+ * operation as an intrinsic without a builtin of its own */
+extern "C" __device__ int mpcd_intrin_writelane(int s, int l, int v) __asm("llvm.amdgcn.writelane.i32");
+__device__ inline __attribute__((always_inline)) int wave_writelane(int s, int l, int v) { return mpcd_intrin_writelane(s, l, v); }
 ZHD double wave_readlane_d(double v, int l) {
     const unsigned long long b = (unsigned long long)__double_as_longlong(v);
     const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
@@ -126,6 +133,8 @@ struct ZoneParams {
     double lowLoc1, highLoc1; /* empty-cell thresholds for fluid fraction 1 */
     int useLocal, maxPasses, corrEnabled;
     int dedupe; /* a periodic axis narrower than 5 cells: wrapped neighbours can repeat */
+    int quadBins; /* no dedupe, at most 3 neighbour offsets per angular bin, no two of a bin equally far: the
+                   * wavefront form's lane layout, in which no tie is left to a draw */
     /* angular bin (3 bits) of (dx,dy) in [-2,2]^2 at index (dy+2)*5+(dx+2):
      * indices 0..20 in binLo, 21..24 in binHi (registers, not an array that
      * a dynamic index would send to private memory) */
@@ -170,7 +179,7 @@ enum : unsigned short {
     ZF_RECV = 2,    /* received particles */
     ZF_BB = 4,      /* bulk-to-bulk transfer */
     ZF_SKIP = 8,    /* transfer touching a non-bulk cell */
-    ZF_MAT = 16,    /* list links written */
+    ZF_MAT = 16,    /* every list link written (else: what is left of the input run, then linked arrivals) */
     ZF_CORR = 32,   /* momentum correction applies */
     ZF_CHG = 64,    /* list changed */
     ZF_OWN = 128,   /* this zone owns the cell's input particles */
@@ -224,12 +233,29 @@ struct ZoneShared {
     double stats4, stats5;
 };
 
+/* A cell's live state: one 8-byte LDS access with 16-bit indices. */
+template <class IT>
+struct alignas(4 * sizeof(IT)) ZCell {
+    IT cnt, head, tail, fl;
+};
+
+/* The small scratch of the one-lane forms (and, idle, of the scheduled
+ * phases' list building). */
+template <class IT>
+struct ZScratch {
+    Cand cand[24];
+    double ordThr[24], nbTie[24], dsc[8], nsm4[4];
+    int ord[24], nbGc[24], rnk[24], recvT[48], dord[8], dord2[16];
+    IT tmpL[ZONE_TMP_L]; /* a donor list being shuffled */
+};
+
 template <class IT>
 struct ZoneCtxT {
     typedef IT idx_t;
     Geom g;
     ZoneParams zp;
     int xs, xe, ys, ye, zw, zh, C;
+    unsigned zhM; /* lc_col's factor, 0 for zh = 1 */
     int zid, P, nL;
     int allOwned; /* copied from the shared set-up result */
     uint64_t seed;
@@ -247,28 +273,15 @@ struct ZoneCtxT {
     double* duG; /* velocity change per cell (zone's global region, 2 per cell) */
     unsigned char* rec; /* last move of each particle by local index (zone's global region, 1 per particle) */
     /* cell arrays */
-    IT *cnt, *head, *tail, *dl, *k0;
+    ZCell<IT>* cell;
+    IT *dl, *k0;
     IT* ext; /* sparse phase: the counts it starts from, zone and ring, (zw+4) x (zh+4) column-major */
-    unsigned short* fl;
     int *colL, *colG; /* per column: first local index, start in the binning list */
     double *lowA, *highA; /* local fluid-fraction thresholds (only with useLocal) */
     IT* halo;             /* pass-input counts of the ring of width 2 around the zone */
-    /* small scratch */
-    Cand* cand;     /* 24 */
-    int* ord;       /* 24 */
-    double* ordThr; /* 24 */
-    int* nbGc;      /* 24 */
-    double* nbTie;  /* 24 */
-    int* rnk;       /* 24 */
-    int* recvT;     /* 24 */
-    double* dsc;    /* 8 */
-    int* dord;      /* 8 */
-    int* dord2;     /* 8 */
-    double* nsm4;   /* 4 */
-    int* mvk;          /* ZONE_MAX_MOVE: local indices of a materialised list's head run */
-    IT* tmpL;          /* tmpCap entries (ZONE_TMP_L, or a wavefront's share in the multi-wavefront sparse phase) */
-    IT* lix;           /* per cell: its index in the multi-wavefront sparse phase's list, or the type's maximum */
-    int tmpCap;
+    ZScratch<IT>* scr;
+    IT* lix; /* per cell: its index in the sparse phase's list (the type's maximum: none, or done); in the dense
+              * passes a dense cell's surplus and start bins */
     ZoneShared* sh;
 };
 
@@ -280,39 +293,39 @@ ZHD int iget(IT v) {
 }
 template <class Z>
 ZHD bool fget(const Z& z, int lc, unsigned short b) {
-    return (z.fl[lc] & b) != 0;
+    return ((unsigned)z.cell[lc].fl & b) != 0;
 }
 template <class Z>
 ZHD void fset(Z& z, int lc, unsigned short b) {
-    z.fl[lc] = (unsigned short)(z.fl[lc] | b);
+    z.cell[lc].fl = (typename Z::idx_t)((unsigned)z.cell[lc].fl | b);
 }
 template <class Z>
 ZHD void fclr(Z& z, int lc, unsigned short b) {
-    z.fl[lc] = (unsigned short)(z.fl[lc] & ~b);
+    z.cell[lc].fl = (typename Z::idx_t)((unsigned)z.cell[lc].fl & ~(unsigned)b);
 }
 template <class Z>
 ZHD int cnt_of(const Z& z, int lc) {
-    return (int)z.cnt[lc];
+    return (int)z.cell[lc].cnt;
 }
 template <class Z>
 ZHD void cnt_set(Z& z, int lc, int v) {
-    z.cnt[lc] = (typename Z::idx_t)v;
+    z.cell[lc].cnt = (typename Z::idx_t)v;
 }
 template <class Z>
 ZHD int head_of(const Z& z, int lc) {
-    return iget(z.head[lc]);
+    return iget(z.cell[lc].head);
 }
 template <class Z>
 ZHD int tail_of(const Z& z, int lc) {
-    return iget(z.tail[lc]);
+    return iget(z.cell[lc].tail);
 }
 template <class Z>
 ZHD void head_set(Z& z, int lc, int k) {
-    z.head[lc] = (typename Z::idx_t)k;
+    z.cell[lc].head = (typename Z::idx_t)k;
 }
 template <class Z>
 ZHD void tail_set(Z& z, int lc, int k) {
-    z.tail[lc] = (typename Z::idx_t)k;
+    z.cell[lc].tail = (typename Z::idx_t)k;
 }
 /* Accesses to the zone's global regions.  On the device they are
  * non-temporal operations: distinct from the working-set accesses, so the
@@ -351,13 +364,22 @@ ZHD int zone_lc(const Z& z, int gx, int gy) {
     if (gx >= z.xs && gx < z.xe && gy >= z.ys && gy < z.ye) return (gx - z.xs) * z.zh + (gy - z.ys);
     return -1;
 }
+/* lc / zh.  With 16-bit indices by a multiplication: zhM = floor((2^32-1)/zh) + 1
+ * exceeds 2^32/zh by e/zh with e <= zh, and lc e < 2^32, so the high word of
+ * lc zhM is the quotient (zh = 1 has no such factor in 32 bits). */
+template <class Z>
+ZHD int lc_col(const Z& z, int lc) {
+    if (sizeof(typename Z::idx_t) == 2)
+        return z.zhM ? (int)(((unsigned long long)(unsigned)lc * (unsigned long long)z.zhM) >> 32) : lc;
+    return lc / z.zh;
+}
 template <class Z>
 ZHD int lc_gx(const Z& z, int lc) {
-    return z.xs + lc / z.zh;
+    return z.xs + lc_col(z, lc);
 }
 template <class Z>
 ZHD int lc_gy(const Z& z, int lc) {
-    return z.ys + lc % z.zh;
+    return z.ys + lc - z.zh * lc_col(z, lc);
 }
 template <class Z>
 ZHD int lc_gc(const Z& z, int lc) {
@@ -377,6 +399,25 @@ ZHD int halo_slot(const Z& z, int dx, int dy) {
     if (hx < 2) return 4 * W4 + hx * z.zh + (hy - 2);
     if (hx >= z.zw + 2) return 4 * W4 + 2 * z.zh + (hx - z.zw - 2) * z.zh + (hy - 2);
     return -1;
+}
+/* extended coordinates (0 .. zw+3, 0 .. zh+3) of ring slot h */
+template <class Z>
+ZHD void halo_xy(const Z& z, int h, int& hx, int& hy) {
+    const int W4 = z.zw + 4;
+    if (h < 2 * W4) {
+        hx = h / 2;
+        hy = h % 2;
+    } else if (h < 4 * W4) {
+        hx = (h - 2 * W4) / 2;
+        hy = z.zh + 2 + (h - 2 * W4) % 2;
+    } else if (h < 4 * W4 + 2 * z.zh) {
+        hx = lc_col(z, h - 4 * W4);
+        hy = 2 + (h - 4 * W4) - hx * z.zh;
+    } else {
+        const int q = lc_col(z, h - 4 * W4 - 2 * z.zh);
+        hx = z.zw + 2 + q;
+        hy = 2 + (h - 4 * W4 - 2 * z.zh) - q * z.zh;
+    }
 }
 template <class Z>
 ZHD int halo_size(const Z& z) {
@@ -405,7 +446,7 @@ template <class Z>
 ZHD int count_at(const Z& z, int gx, int gy, int use_copy) {
     const int lc = zone_lc(z, gx, gy);
     if (lc >= 0) {
-        if (!use_copy) return (int)z.cnt[lc];
+        if (!use_copy) return (int)z.cell[lc].cnt;
         const int ix = lc / z.zh;
         return (int)z.ext[(ix + 2) * (z.zh + 4) + (lc - ix * z.zh) + 2];
     }
@@ -481,7 +522,7 @@ ZHD double nsm_ext(const Z& z, int gx, int gy) {
  * empty-cell values are constants, otherwise they are stored per cell. */
 template <class Z>
 ZHD void zone_maps(Z& z, int lc, int use_copy) {
-    const int bulk = z.cnt[lc] > 0;
+    const int bulk = z.cell[lc].cnt > 0;
     if (bulk) fset(z, lc, ZF_BULK0);
     else fclr(z, lc, ZF_BULK0);
     if (!z.zp.useLocal) return;
@@ -576,48 +617,63 @@ ZHD unsigned short own_bits(const Z& z, int k, int col) {
         if ((int)z.k0[mid] <= k) lo = mid;
         else hi = mid - 1;
     }
-    return (unsigned short)(z.fl[lo] & (ZF_OWN | ZF_COVER));
+    return (unsigned short)((unsigned)z.cell[lo].fl & (ZF_OWN | ZF_COVER));
+}
+
+/* last local index of cell lc's input run (k0[lc] - 1 when it is empty): the
+ * runs follow each other in lc order */
+template <class Z>
+ZHD int run_end(const Z& z, int lc) {
+    return (lc + 1 < z.C ? (int)z.k0[lc + 1] : z.P) - 1;
+}
+/* k belongs to cell lc's input run */
+template <class Z>
+ZHD bool in_run(const Z& z, int lc, int k) {
+    return k >= (int)z.k0[lc] && k <= run_end(z, lc);
+}
+/* entries of a list with head h that are still implicit: what is left of the
+ * input run (none once its links are written or the run is used up) */
+template <class Z>
+ZHD int run_left(const Z& z, int lc, int h) {
+    return (h >= 0 && !fget(z, lc, ZF_MAT) && in_run(z, lc, h)) ? run_end(z, lc) - h + 1 : 0;
 }
 
 /* successor of k in cell lc's list (implicit run or links) */
 template <class Z>
 ZHD int next_k(const Z& z, int lc, int k) {
-    return fget(z, lc, ZF_MAT) ? nx_get(z, k) : (k < tail_of(z, lc) ? k + 1 : -1);
+    if (!fget(z, lc, ZF_MAT)) {
+        if (k == tail_of(z, lc)) return -1;
+        if (k >= (int)z.k0[lc] && k < run_end(z, lc)) return k + 1;
+    }
+    return nx_get(z, k);
 }
 
-/* write the links of a still-implicit list before its first append */
+/* write the links of what is still implicit in cell lc's list */
 template <class Z>
 ZHD void ensure_mat(Z& z, int lc) {
     if (fget(z, lc, ZF_MAT)) return;
-    const int t = tail_of(z, lc);
-    for (int k = head_of(z, lc); k >= 0 && k <= t; ++k) nx_set(z, k, (k < t) ? k + 1 : -1);
+    const int h = head_of(z, lc), left = run_left(z, lc, h);
+    for (int q = 0; q + 1 < left; ++q) nx_set(z, h + q, h + q + 1);
+    if (left > 0 && tail_of(z, lc) == h + left - 1) nx_set(z, h + left - 1, -1);
     fset(z, lc, ZF_MAT);
 }
 
-/* ensure_mat by all lanes (lc the same on every lane) */
+/* A list that takes back a particle of its own input run cannot keep the run
+ * implicit: its links are written first (one lane). */
 template <class Z>
-ZHD void ensure_mat_lanes(Z& z, int lc, int lane, int nl) {
-    if (fget(z, lc, ZF_MAT)) return;
-    const int h = head_of(z, lc), t = tail_of(z, lc);
-    if (h >= 0)
-        for (int k = h + lane; k <= t; k += nl) nx_set(z, k, k < t ? k + 1 : -1);
-    ZBAR();
-    if (lane == 0) fset(z, lc, ZF_MAT);
-    ZBAR();
+ZHD void ensure_append(Z& z, int lc, int k) {
+    if (in_run(z, lc, k)) ensure_mat(z, lc);
 }
 
-/* requires a materialised list */
 template <class Z>
 ZHD void list_append(Z& z, int lc, int k) {
-    typedef typename Z::idx_t IT;
-    IT* const H = z.head;
-    IT* const T = z.tail;
+    ensure_append(z, lc, k);
     fset(z, lc, ZF_CHG);
     nx_set(z, k, -1);
-    const int t = iget(T[lc]);
-    if (t < 0) H[lc] = (IT)k;
+    const int t = tail_of(z, lc);
+    if (t < 0) head_set(z, lc, k);
     else nx_set(z, t, k);
-    T[lc] = (IT)k;
+    tail_set(z, lc, k);
 }
 
 /* A moved particle's new position (zone_pass.cpp:280-294: uniform in its
@@ -698,8 +754,8 @@ ZHD int zone_compact(Z& z, int lane, int nl, int mode) {
         const int lc = b0 + lane;
         bool f = false;
         if (lc < z.C) {
-            const double c = (double)z.cnt[lc];
-            f = (mode == ZC_DENSE) ? c > high_thr(z, lc) : (z.cnt[lc] > 0 && c < low_thr(z, lc));
+            const double c = (double)z.cell[lc].cnt;
+            f = (mode == ZC_DENSE) ? c > high_thr(z, lc) : (z.cell[lc].cnt > 0 && c < low_thr(z, lc));
             f = f && !fget(z, lc, ZF_OUT);
         }
         const unsigned long long msk = wave_ballot(f);
@@ -725,6 +781,33 @@ struct ShufDraw {
     }
 };
 
+#if defined(__HIP_DEVICE_COMPILE__)
+/* Fisher-Yates of the values v of lanes 0..m-1 (m <= 64) with lane i's
+ * partner j (in [0, i]) */
+__device__ inline __attribute__((always_inline)) int shuffle64(int v, int j, int m) {
+    int ii = m - 1;
+    for (; ii >= 8; ii -= 8) {
+        /* the partners of eight swaps first: off the swaps' own chain */
+        int jj[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) jj[t] = wave_readlane(j, ii - t);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const int vi = wave_readlane(v, ii - t), vj = wave_readlane(v, jj[t]);
+            v = wave_writelane(vj, ii - t, v);
+            v = wave_writelane(vi, jj[t], v);
+        }
+    }
+    for (; ii >= 1; --ii) {
+        const int jj = wave_readlane(j, ii);
+        const int vi = wave_readlane(v, ii), vj = wave_readlane(v, jj);
+        v = wave_writelane(vj, ii, v);
+        v = wave_writelane(vi, jj, v);
+    }
+    return v;
+}
+#endif
+
 /* Fisher-Yates of a[0..m), i = m-1 down to 1, swapping a[i] with a[j(i)],
  * `draw(i)` giving j in [0, i].  The partner draws of a chunk of nl indices
  * are computed by the lanes at once and kept in registers; lane 0 applies
@@ -732,17 +815,34 @@ struct ShufDraw {
 template <class T>
 ZHD void zone_shuffle(T* a, int m, int lane, int nl, ShufDraw draw) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    if (m <= 64) {
-        /* element q in lane q's register; each swap reads the two values
-         * and writes them back by lane select */
-        int v = lane < m ? (int)a[lane] : 0;
-        const int j = (lane >= 1 && lane < m) ? (int)draw((uint32_t)lane) : 0;
-        for (int ii = m - 1; ii >= 1; --ii) {
-            const int jj = wave_readlane(j, ii);
-            const int vi = wave_readlane(v, ii), vj = wave_readlane(v, jj);
-            v = lane == ii ? vj : (lane == jj ? vi : v);
+    if (m <= 128) {
+        /* elements q and 64 + q in lane q's registers: a swap is two reads
+         * and two writes of single lanes.  (A list in LDS instead makes each
+         * swap two dependent accesses of one lane, about 250 cycles against
+         * 40; a zone of 25 x 25 cells has 50 to 80 dense cells.) */
+        int v0 = lane < m ? (int)a[lane] : 0, v1 = 0, j1 = 0;
+        const int j0 = (lane >= 1 && lane < m) ? (int)draw((uint32_t)lane) : 0;
+        if (m > 64) {
+            if (64 + lane < m) {
+                v1 = (int)a[64 + lane];
+                j1 = (int)draw((uint32_t)(64 + lane));
+            }
+            for (int ii = m - 65; ii >= 0; --ii) {
+                const int jj = wave_readlane(j1, ii), vi = wave_readlane(v1, ii);
+                if (jj >= 64) {
+                    const int vj = wave_readlane(v1, jj - 64);
+                    v1 = wave_writelane(vj, ii, v1);
+                    v1 = wave_writelane(vi, jj - 64, v1);
+                } else {
+                    const int vj = wave_readlane(v0, jj);
+                    v1 = wave_writelane(vj, ii, v1);
+                    v0 = wave_writelane(vi, jj, v0);
+                }
+            }
+            if (64 + lane < m) a[64 + lane] = (T)v1;
         }
-        if (lane < m) a[lane] = (T)v;
+        v0 = shuffle64(v0, j0, imin(m, 64));
+        if (lane < m) a[lane] = (T)v0;
         ZBAR();
         return;
     }
@@ -769,7 +869,7 @@ ZHD void zone_shuffle(T* a, int m, int lane, int nl, ShufDraw draw) {
  * zone, ranked into the round-robin order of rank_dense_targets_unified
  * (zone_pass.cpp:413-490): 8 angular bins from a random start bin, each bin
  * sorted by the candidate key, then one per bin per round.  All lanes; the
- * order lands in z.ord[0..nOrd) with each target's threshold in z.ordThr.
+ * order lands in z.scr->ord[0..nOrd) with each target's threshold in z.scr->ordThr.
  * Every draw is taken in one round: the tie breaks (t = 0..23, one per
  * neighbour offset) and the start bin (t = 24). */
 template <class Z>
@@ -783,10 +883,10 @@ ZHD void dense_targets(Z& z, int src, int high, int pass, int phase, int lane, i
             int jx, jy, gc = -1;
             if (shift_idx(z, sgx, sgy, dx, dy, jx, jy)) {
                 const int lc = zone_lc(z, jx, jy);
-                if (lc >= 0 && !fget(z, lc, ZF_OUT) && (double)z.cnt[lc] < thr(z, lc, high)) gc = jy + z.g.Ny * jx;
+                if (lc >= 0 && !fget(z, lc, ZF_OUT) && (double)z.cell[lc].cnt < thr(z, lc, high)) gc = jy + z.g.Ny * jx;
             }
-            z.nbGc[t] = gc;
-            if (gc >= 0) z.nbTie[t] = mpcd_draw_tie(z.seed, pass, phase, (uint32_t)sgc, (uint32_t)gc);
+            z.scr->nbGc[t] = gc;
+            if (gc >= 0) z.scr->nbTie[t] = mpcd_draw_tie(z.seed, pass, phase, (uint32_t)sgc, (uint32_t)gc);
         } else {
             z.sh->startBin = mpcd_draw_start_bin(z.seed, pass, phase, (uint32_t)sgc);
         }
@@ -799,11 +899,11 @@ ZHD void dense_targets(Z& z, int src, int high, int pass, int phase, int lane, i
         bool keep = false;
         int gc = -1;
         if (lane < 24) {
-            gc = z.nbGc[lane];
+            gc = z.scr->nbGc[lane];
             keep = gc >= 0;
             if (z.zp.dedupe)
                 for (int q = 0; q < lane && keep; ++q)
-                    if (z.nbGc[q] == gc) keep = false;
+                    if (z.scr->nbGc[q] == gc) keep = false;
         }
         const unsigned long long msk = wave_ballot(keep);
         const int m = wave_popc(msk);
@@ -816,11 +916,11 @@ ZHD void dense_targets(Z& z, int src, int high, int pass, int phase, int lane, i
             min_step(z, sgx, sgy, jx, jy, ddx, ddy);
             bin = zone_bin(z.zp, (ddy + 2) * 5 + (ddx + 2));
             th = thr(z, lc, high);
-            cnt = z.cnt[lc];
+            cnt = z.cell[lc].cnt;
             defn = -dmax(0.0, th - (double)cnt);
             cheb = imax(ddx < 0 ? -ddx : ddx, ddy < 0 ? -ddy : ddy);
             dist2 = ddx * ddx + ddy * ddy;
-            tie = z.nbTie[lane];
+            tie = z.scr->nbTie[lane];
         }
         if (lane == 0) z.sh->nOrd = m;
         if (m == 0) {
@@ -857,8 +957,8 @@ ZHD void dense_targets(Z& z, int src, int high, int pass, int phase, int lane, i
             if (rj < r || (rj == r && sj < si)) ++pos;
         }
         if (keep) {
-            z.ord[pos] = lc;
-            z.ordThr[pos] = th;
+            z.scr->ord[pos] = lc;
+            z.scr->ordThr[pos] = th;
         }
         ZBAR();
     }
@@ -869,15 +969,15 @@ ZHD void dense_targets(Z& z, int src, int high, int pass, int phase, int lane, i
         bool keep = false;
         int gc = -1;
         if (o < 24) {
-            gc = z.nbGc[o];
+            gc = z.scr->nbGc[o];
             keep = gc >= 0;
             if (z.zp.dedupe)
                 for (int q = 0; q < o && keep; ++q)
-                    if (z.nbGc[q] == gc) keep = false;
+                    if (z.scr->nbGc[q] == gc) keep = false;
         }
         const unsigned long long msk = wave_ballot(keep);
         if (keep) {
-            Cand& c = z.cand[base + wave_popc(msk & lanes_below(lane))];
+            Cand& c = z.scr->cand[base + wave_popc(msk & lanes_below(lane))];
             const int jx = gc / z.g.Ny, jy = gc - jx * z.g.Ny;
             const int lc = zone_lc(z, jx, jy);
             int ddx, ddy;
@@ -885,11 +985,11 @@ ZHD void dense_targets(Z& z, int src, int high, int pass, int phase, int lane, i
             c.lc = lc;
             c.gc = gc;
             c.bin = zone_bin(z.zp, (ddy + 2) * 5 + (ddx + 2));
-            c.deficitNeg = -dmax(0.0, thr(z, lc, high) - (double)z.cnt[lc]);
-            c.cnt = z.cnt[lc];
+            c.deficitNeg = -dmax(0.0, thr(z, lc, high) - (double)z.cell[lc].cnt);
+            c.cnt = z.cell[lc].cnt;
             c.cheb = imax(ddx < 0 ? -ddx : ddx, ddy < 0 ? -ddy : ddy);
             c.dist2 = ddx * ddx + ddy * ddy;
-            c.tie = z.nbTie[o];
+            c.tie = z.scr->nbTie[o];
         }
         base += wave_popc(msk);
     }
@@ -899,28 +999,28 @@ ZHD void dense_targets(Z& z, int src, int high, int pass, int phase, int lane, i
     if (m == 0) return;
     /* rank inside the bin: stable order of the candidate key */
     for (int i = lane; i < m; i += nl) {
-        const Cand ci = z.cand[i];
+        const Cand ci = z.scr->cand[i];
         int r = 0;
         for (int j = 0; j < m; ++j) {
-            if (j == i || z.cand[j].bin != ci.bin) continue;
-            if (cand_less(z.cand[j], ci) || (j < i && !cand_less(ci, z.cand[j]))) ++r;
+            if (j == i || z.scr->cand[j].bin != ci.bin) continue;
+            if (cand_less(z.scr->cand[j], ci) || (j < i && !cand_less(ci, z.scr->cand[j]))) ++r;
         }
-        z.rnk[i] = r;
+        z.scr->rnk[i] = r;
     }
     ZBAR();
     /* round robin position: earlier rounds, then earlier bins from startBin */
     const int sb = z.sh->startBin;
     for (int i = lane; i < m; i += nl) {
-        const int ri = z.rnk[i];
-        const int si = (z.cand[i].bin - sb + 8) & 7;
+        const int ri = z.scr->rnk[i];
+        const int si = (z.scr->cand[i].bin - sb + 8) & 7;
         int pos = 0;
         for (int j = 0; j < m; ++j) {
-            const int rj = z.rnk[j];
-            if (rj < ri || (rj == ri && ((z.cand[j].bin - sb + 8) & 7) < si)) ++pos;
+            const int rj = z.scr->rnk[j];
+            if (rj < ri || (rj == ri && ((z.scr->cand[j].bin - sb + 8) & 7) < si)) ++pos;
         }
-        const int lc = z.cand[i].lc;
-        z.ord[pos] = lc;
-        z.ordThr[pos] = thr(z, lc, high);
+        const int lc = z.scr->cand[i].lc;
+        z.scr->ord[pos] = lc;
+        z.scr->ordThr[pos] = thr(z, lc, high);
     }
     ZBAR();
 #endif
@@ -941,17 +1041,15 @@ ZHD int spread(Z& z, int src, int needOut, int pass, int* rv, int& nr) {
         bool progressed = false;
         int R = 0;
         for (int jj = 0; jj < nOrd; ++jj)
-            if (imax(0, (int)MPCD_FLOOR(z.ordThr[jj] - (double)cnt_of(z, z.ord[jj]))) > 0) ++R;
+            if (imax(0, (int)MPCD_FLOOR(z.scr->ordThr[jj] - (double)cnt_of(z, z.scr->ord[jj]))) > 0) ++R;
         for (int kk = 0; kk < nOrd; ++kk) {
-            const int nb = z.ord[kk];
-            const int deficit = imax(0, (int)MPCD_FLOOR(z.ordThr[kk] - (double)cnt_of(z, nb)));
+            const int nb = z.scr->ord[kk];
+            const int deficit = imax(0, (int)MPCD_FLOOR(z.scr->ordThr[kk] - (double)cnt_of(z, nb)));
             if (deficit <= 0) continue;
             const int remaining = R;
             --R;
             const int quota = imax(1, (int)MPCD_CEIL((double)needOut / (double)imax(1, remaining)));
             const int nt = imax(1, imin(imin(quota, deficit), imin(needOut, avail)));
-            /* pops from the head leave an implicit run implicit */
-            ensure_mat(z, nb);
             fset(z, src, ZF_CHG);
             for (int q = 0; q < nt; ++q) {
                 const int k = head_of(z, src);
@@ -1005,101 +1103,86 @@ ZHD double lane_put_d(double v, int dst) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-/* The ranking of dense_targets (zone_pass.cpp:413-490).  Candidate o (lane
- * o < 24) is neighbour offset o; its key (deficit, count, Chebyshev and
- * squared distance, tie draw) is compared only with the other members of its
- * angular bin, fetched by lane permutes; the round-robin position follows
- * from the rank in the bin and the bins' sizes.  On return lane p < nOrd
- * (the return value, same on all lanes) holds the p-th target: zone cell,
- * threshold and count. */
+/* values of the lanes of one's quad, rotated: rotation s hands lane m of a
+ * quad the value of lane (m + s) & 3 */
+template <int S>
+ZHD int quad_rot(int v) {
+    constexpr int ctrl = ((0 + S) & 3) | (((1 + S) & 3) << 2) | (((2 + S) & 3) << 4) | (((3 + S) & 3) << 6);
+    return __builtin_amdgcn_mov_dpp(v, ctrl, 0xf, 0xf, true);
+}
+template <int S>
+ZHD unsigned long long quad_rot64(unsigned long long v) {
+    const unsigned lo = (unsigned)quad_rot<S>((int)(unsigned)v), hi = (unsigned)quad_rot<S>((int)(unsigned)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+ZHD int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+/* A dense cell's ranking lives in lanes by angular bin: lanes 4 b + m and
+ * 32 + 4 b + m (m < 3) hold the m-th neighbour offset of bin b, the first for
+ * the low thresholds (phase 0), the second for the high ones (phase 1).  A
+ * candidate is compared with its bin's other members by quad rotations.  The
+ * offsets of a bin differ in distance, which the key compares before the tie
+ * draw, so no tie draw is ever looked at. */
+struct DenseLane {
+    int dx, dy, bin, code; /* code: Chebyshev << 4 | squared distance, -1 without an offset */
+    double thB, thE;       /* threshold of an occupied and of an empty cell in this lane's phase */
+};
 template <class Z>
-ZHD int dense_rank_wave(const Z& z, int sgx, int sgy, int sgc, int high, int pass, int phase, int lane, int& lcP,
-                        double& thP, int& cP) {
-    int gc = -1, lc = -1, cnt = 0, ddx = 0, ddy = 0;
-    double th = 0.0;
-    if (lane < 24) {
-        const int f = lane < 12 ? lane : lane + 1;
-        const int dy = f / 5 - 2, dx = f % 5 - 2;
-        int jx, jy;
-        if (shift_idx(z, sgx, sgy, dx, dy, jx, jy)) {
-            const int l = zone_lc(z, jx, jy);
-            if (l >= 0 && !fget(z, l, ZF_OUT)) {
-                const int c = (int)z.cnt[l];
-                const double t = thr(z, l, high);
-                if ((double)c < t) {
-                    gc = jy + z.g.Ny * jx;
-                    lc = l;
-                    cnt = c;
-                    th = t;
-                    min_step(z, sgx, sgy, jx, jy, ddx, ddy);
-                }
-            }
+ZHD DenseLane dense_lane(const Z& z, int lane) {
+    DenseLane d{0, 0, (lane >> 2) & 7, -1, 0.0, 0.0};
+    int seen = 0;
+    for (int idx = 0; idx < 25; ++idx) {
+        if (idx == 12 || zone_bin(z.zp, idx) != d.bin) continue;
+        if (seen == (lane & 3)) {
+            d.dx = idx % 5 - 2;
+            d.dy = idx / 5 - 2;
+            const int ax = d.dx < 0 ? -d.dx : d.dx, ay = d.dy < 0 ? -d.dy : d.dy;
+            d.code = (imax(ax, ay) << 4) | (ax * ax + ay * ay);
         }
+        ++seen;
     }
-    bool keep = gc >= 0;
-    if (z.zp.dedupe)
-        for (int q = 0; q < 23; ++q) {
-            const int gq = wave_readlane(gc, q);
-            if (q < lane && gq == gc) keep = false;
-        }
-    const unsigned long long msk = wave_ballot(keep);
-    const int m = wave_popc(msk);
-    lcP = -1;
-    cP = 0;
-    thP = 0.0;
-    if (m == 0) return 0;
-    /* one Philox block per lane: tie break (lanes < 24), start bin (lane 24),
-     * the counters of mpcd_draw_tie and mpcd_draw_start_bin */
-    const mpcd_u32x4 rb = mpcd_philox(z.seed,
-                                      mpcd_ctr0(lane < 24 ? MPCD_TAG_RTIE : MPCD_TAG_RBIN, (uint32_t)((pass << 1) | phase)),
-                                      (uint32_t)sgc, lane < 24 ? (uint32_t)gc : 0u, 0u);
-    const double tie = mpcd_u01(rb.w[0], rb.w[1]);
-    const int sb = wave_readlane((int)mpcd_uint_below(rb.w[0], 8u), 24);
-    const int bin = keep ? zone_bin(z.zp, (ddy + 2) * 5 + (ddx + 2)) : 8;
-    const double defn = -dmax(0.0, th - (double)cnt);
-    const int cheb = imax(ddx < 0 ? -ddx : ddx, ddy < 0 ? -ddy : ddy);
-    /* (count, Chebyshev, squared distance) in one ordered word: cheb <= 2, dist2 <= 8 */
-    const unsigned long long sm =
-        ((unsigned long long)(unsigned)cnt << 8) | (unsigned long long)((cheb << 4) | (ddx * ddx + ddy * ddy));
-    unsigned long long bm[8];
-    unsigned long long mine = 0ull;
-    int smax = 0;
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-        bm[b] = wave_ballot(bin == b);
-        smax = imax(smax, wave_popc(bm[b]));
-        if (bin == b) mine = bm[b];
-    }
-    /* rank inside the bin: the stable order of the candidate key */
-    unsigned long long mm = mine & ~(1ull << lane);
-    int r = 0;
-    for (int s = 1; s < smax; ++s) {
-        const bool have = mm != 0ull;
-        const int j = have ? (int)__builtin_ctzll(mm) : lane;
-        if (have) mm &= mm - 1ull;
-        const double od = lane_get_d(defn, j);
-        const unsigned long long osm = lane_get_u64(sm, j);
-        const double ot = lane_get_d(tie, j);
-        if (have) {
-            const bool oLess = od < defn || (od == defn && (osm < sm || (osm == sm && ot < tie)));
-            const bool meLess = defn < od || (defn == od && (sm < osm || (sm == osm && tie < ot)));
-            if (oLess || (j < lane && !meLess)) ++r;
-        }
-    }
-    /* round-robin position: every bin's members of earlier rounds, then this
-     * round's members of the bins before this one from the start bin */
-    const int si = (bin - sb + 8) & 7;
-    int pos = 0;
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-        const int nb = wave_popc(bm[b]);
-        pos += imin(nb, r) + ((((b - sb + 8) & 7) < si && nb > r) ? 1 : 0);
-    }
-    const int dst = keep ? pos : m + wave_popc(~msk & lanes_below(lane));
-    lcP = lane_put(lc, dst);
-    cP = lane_put(cnt, dst);
-    thP = lane_put_d(th, dst);
-    return m;
+    d.thB = lane < 32 ? z.zp.lowThrBulk : z.zp.highThr;
+    d.thE = lane < 32 ? z.zp.lowLoc1 : z.zp.highLoc1;
+    return d;
+}
+
+/* a periodic axis whose wrapped range-2 neighbours can lie in the zone */
+template <class Z>
+ZHD bool zone_wrap_x(const Z& z) {
+    return z.g.perx && z.zw >= z.g.Nx - 1;
+}
+template <class Z>
+ZHD bool zone_wrap_y(const Z& z) {
+    return z.g.pery && z.zh >= z.g.Ny - 1;
+}
+/* zone-relative coordinate t taken once around an axis of n cells */
+ZHD int wrap_near(int t, int n) { return t < 0 ? t + n : (t >= n ? t - n : t); }
+
+/* A dense cell's surplus over its high threshold (an occupied cell's is the
+ * bulk one), and its start bins of both phases. */
+template <class Z>
+ZHD int dense_need(const Z& z, int nc) {
+    return imax(0, (int)MPCD_CEIL((double)nc - z.zp.highThr));
+}
+template <class Z>
+ZHD unsigned dense_bins(const Z& z, int c, int pass) {
+    const uint32_t gc = (uint32_t)lc_gc(z, c);
+    return (unsigned)mpcd_draw_start_bin(z.seed, pass, 0, gc) | ((unsigned)mpcd_draw_start_bin(z.seed, pass, 1, gc) << 3);
+}
+/* both in the cell's lix entry (the surplus of a cell whose movers fit the
+ * wavefront is below 64) */
+template <class Z>
+ZHD void dense_word(Z& z, int c, int pass) {
+    z.lix[c] = (typename Z::idx_t)((unsigned)dense_need(z, cnt_of(z, c)) | (dense_bins(z, c, pass) << 7));
+}
+
+/* lanes of `half` set in a ballot, as 32 bits */
+ZHD unsigned half_bits(unsigned long long m, int half) { return (unsigned)(m >> (32 * half)); }
+/* lanes of m (in half's 32) that the round-robin order puts before this lane
+ * within one round: the bins from the start bin sb up to this lane's */
+ZHD int round_before(unsigned m, int sb, int bin) {
+    const unsigned rot = sb ? (m >> (4 * sb)) | (m << (32 - 4 * sb)) : m;
+    return wave_popc((unsigned long long)(rot & ((1u << (4 * ((bin - sb) & 7))) - 1u)));
 }
 
 /* One sweep series of spread (zone_pass.cpp:527-589) over the ranking in the
@@ -1123,7 +1206,9 @@ ZHD int spread_plan_wave(int nOrd, double thP, int& cP, int need, int& avail, in
             const int kk = (int)__builtin_ctzll(mk);
             const int d = wave_readlane(defP, kk);
             const int remaining = R--;
-            const int quota = imax(1, (int)MPCD_CEIL((double)need / (double)imax(1, remaining)));
+            /* ceil(need / remaining), both positive and at most 64: need - 1/2
+             * over remaining is at least 1/128 from an integer */
+            const int quota = 1 + (int)(((float)need - 0.5f) / (float)remaining);
             /* cap (the staged movers) never binds: the callers stage
              * enough for both phases; it only keeps lanes in bounds */
             const int nt = imin(imax(1, imin(imin(quota, d), imin(need, avail))), cap - used);
@@ -1156,43 +1241,31 @@ ZHD int spread_plan_wave(int nOrd, double thP, int& cP, int need, int& avail, in
     return moved;
 }
 
-/* Applies a plan: pops the movers from src's head, records their moves,
- * appends them to their targets in mover order. */
+/* Applies a plan: records the movers' moves and appends them to their targets
+ * in mover order; returns src's next head (src itself is left to the caller,
+ * avail: its particles left). */
 template <class Z>
-ZHD void spread_apply_wave(Z& z, int src, bool srcMat, int lane, int q0, int moved, int avail, int pass, int myK,
-                           int myT, int nextQ, int lcP, int cP, int firstQ, int lastQ) {
-    if (moved <= 0) return;
-    /* src first: a materialised list's next head is read before the movers'
-     * links are rewritten */
-    const int kLast = wave_readlane(myK, q0 + moved - 1);
-    const int nh = srcMat ? nx_get(z, kLast) : (kLast < tail_of(z, src) ? kLast + 1 : -1);
+ZHD int spread_apply_wave(Z& z, int src, int h, int lane, int moved, int avail, int pass, int myK, int myT, int nextQ,
+                          int lcP, int cP, int firstQ, int lastQ) {
+    if (moved <= 0) return h;
+    /* src first: its next head is read before the movers' links are rewritten */
+    const int nh = avail > 0 ? uniform(next_k(z, src, wave_readlane(myK, moved - 1))) : -1;
     const int nk = lane_get(myK, nextQ >= 0 ? nextQ : 0);
     const int fk = lane_get(myK, firstQ >= 0 ? firstQ : 0);
     const int lk = lane_get(myK, lastQ >= 0 ? lastQ : 0);
-    ZWSYNC();
-    if (lane == 0) {
-        head_set(z, src, nh);
-        if (nh < 0) tail_set(z, src, -1);
-        fset(z, src, ZF_CHG);
-        cnt_set(z, src, avail);
+    /* a target that takes back particles of its own input run (lane q: mover q) */
+    const int tl = lane_get(lcP, myT >= 0 ? myT : 0);
+    for (unsigned long long bk = wave_ballot(myT >= 0 && in_run(z, tl, myK)); bk; bk &= bk - 1ull) {
+        const int lt = wave_readlane(tl, (int)__builtin_ctzll(bk));
+        if (lane == 0) ensure_mat(z, lt);
+        ZWSYNC();
     }
+    ZWSYNC();
     if (myT >= 0) {
         mark_moved(z, myK, pass);
         nx_set(z, myK, nextQ >= 0 ? nk : -1);
     }
-    /* targets whose lists are still implicit runs: their links written by
-     * all lanes at once, one target at a time */
-    for (unsigned long long nm = wave_ballot(firstQ >= 0 && !fget(z, lcP, ZF_MAT)); nm; nm &= nm - 1ull) {
-        const int lt = wave_readlane(lcP, (int)__builtin_ctzll(nm));
-        const int h = head_of(z, lt), t = tail_of(z, lt);
-        if (h >= 0)
-            for (int k = h + lane; k <= t; k += 64) nx_set(z, k, k < t ? k + 1 : -1);
-        ZWSYNC();
-        if (lane == 0) fset(z, lt, ZF_MAT);
-        ZWSYNC();
-    }
     if (firstQ >= 0) {
-        ensure_mat(z, lcP);
         const int t = tail_of(z, lcP);
         if (t < 0) head_set(z, lcP, fk);
         else nx_set(z, t, fk);
@@ -1201,66 +1274,189 @@ ZHD void spread_apply_wave(Z& z, int src, bool srcMat, int lane, int q0, int mov
         cnt_set(z, lcP, cP);
     }
     ZWSYNC();
+    return nh;
+}
+
+/* The first n (<= 64) entries of a list, entry q in lane q: what is left of
+ * the run by its indices, the rest along the links (the list holds at least
+ * n entries). */
+template <class Z>
+ZHD int list_entry_wave(const Z& z, int h, int left, int n, int lane) {
+    int v = lane < left ? h + lane : -1;
+    if (n > left) {
+        int k = left > 0 ? nx_get(z, h + left - 1) : h;
+        for (int q = left; q < n; ++q) {
+            if (lane == q) v = k;
+            if (q + 1 < n) k = nx_get(z, k);
+        }
+    }
+    return lane < n ? v : -1;
 }
 
 /* One dense cell (zone_pass.cpp:738-779: both target phases, the spreads and
  * the transfer masks) when its movers fit the wavefront:
- * min(needOut + 1, count) <= 64 (phase 1 moves at most what phase 0 left of
- * needOut, up to one more by the rounding of its ceil).  Returns the number
- * of particles moved. */
+ * min(need + 1, count) <= 64 (phase 1 moves at most what phase 0 left of
+ * need, up to one more by the rounding of its ceil).  bins: dense_bins.
+ * Returns the number of particles moved.
+ *
+ * The ranking (zone_pass.cpp:413-490): rank within the bin by (deficit,
+ * count, distances); the round-robin order is by rank, then by bin from the
+ * start bin.  When the need is at most the number R of targets with a
+ * deficit of one or more, every quota of the spread is ceil(need /
+ * remaining) = 1; when no such target has a deficit of two or more, each
+ * takes what it can, one.  In both cases the first min(need, R) targets in
+ * order take one particle each: no sweep, each receiving lane appends its
+ * own particle.  Nine cells of ten of a uniform state go that way.
+ *
+ * The chain of conflicting cells bounds the passes, so what matters is the
+ * instructions between two of its cells: one LDS read per candidate (the
+ * cell's state in 8 bytes), three rotations, three ballots, one batch of
+ * writes. */
 template <class Z>
-ZHD int dense_cell_wave(Z& z, int src, int nc, double hl, int needOut, int pass, int lane) {
-    const int sgx = lc_gx(z, src), sgy = lc_gy(z, src), sgc = lc_gc(z, src);
-    const int nStage = imin(needOut + 1, nc);
-    const bool srcMat = fget(z, src, ZF_MAT);
-    /* movers: lane q is the q-th particle of src's list */
-    int myK = -1;
-    if (srcMat) {
-        if (lane == 0) {
-            int k = head_of(z, src);
-            for (int q = 0; q < nStage && k >= 0; ++q) {
-                z.mvk[q] = k;
-                k = nx_get(z, k);
-            }
+ZHD int dense_cell_wave(Z& z, const DenseLane& dl, int c, int cx, int cy, int need, unsigned bins, int pass, int lane) {
+    typedef typename Z::idx_t IT;
+    int tx = cx + dl.dx, ty = cy + dl.dy;
+    if (zone_wrap_x(z)) tx = wrap_near(tx, z.g.Nx);
+    if (zone_wrap_y(z)) ty = wrap_near(ty, z.g.Ny);
+    const bool in = (dl.code >= 0) & ((unsigned)tx < (unsigned)z.zw) & ((unsigned)ty < (unsigned)z.zh);
+    const int l = in ? tx * z.zh + ty : c;
+    const ZCell<IT> S = z.cell[c];
+    const unsigned fS = (unsigned)S.fl;
+    int h = uniform(iget(S.head)), avail = uniform((int)S.cnt), moved = 0;
+    const int kb = (int)z.k0[c], ke = run_end(z, c);
+    int left = uniform((fS & ZF_MAT) || h < kb || h > ke ? 0 : ke - h + 1);
+    bool rcvF = false;
+    int rg0 = -1, rg1 = -1;
+    bool masked = false, allBulk = false;
+#pragma nounroll
+    for (int half = 0; half < 2; ++half) {
+        const ZCell<IT> T = z.cell[l];
+        const int cT = (int)T.cnt, tT = iget(T.tail);
+        const unsigned fT = (unsigned)T.fl;
+        const double th = z.zp.useLocal ? (lane < 32 ? z.lowA[l] : z.highA[l]) : ((fT & ZF_BULK0) ? dl.thB : dl.thE);
+        const double def = th - (double)cT;
+        const bool keep = in & !(fT & ZF_OUT) & ((lane >> 5) == half) & (def > 0.0);
+        /* the key: deficits are positive, so their bits are ordered as their
+         * values; a lane without a candidate is never ahead of one */
+        const unsigned long long dk = keep ? (unsigned long long)__double_as_longlong(def) : 0ull;
+        const unsigned sm = ((unsigned)cT << 8) | (unsigned)(dl.code & 255);
+        int r = 0;
+        {
+            const unsigned long long o1 = quad_rot64<1>(dk), o2 = quad_rot64<2>(dk), o3 = quad_rot64<3>(dk);
+            const unsigned s1 = (unsigned)quad_rot<1>((int)sm), s2 = (unsigned)quad_rot<2>((int)sm),
+                           s3 = (unsigned)quad_rot<3>((int)sm);
+            r += (int)((o1 > dk) | ((o1 == dk) & (s1 < sm)));
+            r += (int)((o2 > dk) | ((o2 == dk) & (s2 < sm)));
+            r += (int)((o3 > dk) | ((o3 == dk) & (s3 < sm)));
         }
-        ZWSYNC();
-        if (lane < nStage) myK = z.mvk[lane];
-    } else if (lane < nStage) {
-        myK = head_of(z, src) + lane;
-    }
-    int used = 0, avail = nc, moved = 0;
-    int lcP, cP, myT, nextQ = -1, firstQ, lastQ;
-    double thP;
-    /* phase 0: low thresholds */
-    const int n0 = dense_rank_wave(z, sgx, sgy, sgc, 0, pass, 0, lane, lcP, thP, cP);
-    int q0 = used;
-    int m0 = spread_plan_wave(n0, thP, cP, needOut, avail, used, nStage, lane, myT, nextQ, firstQ, lastQ);
-    spread_apply_wave(z, src, srcMat, lane, q0, m0, avail, pass, myK, myT, nextQ, lcP, cP, firstQ, lastQ);
-    moved += m0;
-    const int rcv0 = firstQ >= 0 ? lcP : -1;
-    /* phase 1: high thresholds, for what is left above the high threshold */
-    int rcv1 = -1;
-    const int remaining = imax(0, (int)MPCD_CEIL((double)avail - hl));
-    if (remaining > 0) {
-        const int n1 = dense_rank_wave(z, sgx, sgy, sgc, 1, pass, 1, lane, lcP, thP, cP);
-        q0 = used;
-        nextQ = -1;
-        const int m1 = spread_plan_wave(n1, thP, cP, remaining, avail, used, nStage, lane, myT, nextQ, firstQ, lastQ);
-        spread_apply_wave(z, src, srcMat, lane, q0, m1, avail, pass, myK, myT, nextQ, lcP, cP, firstQ, lastQ);
-        moved += m1;
-        rcv1 = firstQ >= 0 ? lcP : -1;
+        const int sb = (int)((bins >> (3 * half)) & 7u);
+        const bool pd = keep & (def >= 1.0); /* floor(deficit) > 0 */
+        const unsigned q0 = half_bits(wave_ballot(pd & (r == 0)), half), q1 = half_bits(wave_ballot(pd & (r == 1)), half),
+                       q2 = half_bits(wave_ballot(pd & (r == 2)), half);
+        const int n0 = wave_popc(q0), n1 = wave_popc(q1), R = n0 + n1 + wave_popc(q2);
+        const bool deep = wave_ballot(pd & (def >= 2.0)) != 0ull;
+        if ((need <= R || !deep) && need <= avail) {
+            const int mv = imin(need, R);
+            if (mv > 0) {
+                const int e = (r > 0 ? n0 : 0) + (r > 1 ? n1 : 0) +
+                              round_before(r == 0 ? q0 : (r == 1 ? q1 : q2), sb, dl.bin);
+                const bool rcv = pd & (e < mv);
+                avail -= mv;
+                /* the e-th particle of the cell's list, and the list's next head */
+                int k, nh = -1;
+                bool mat = false;
+                if (mv <= left) {
+                    k = h + e;
+                    if (mv < left) nh = h + mv;
+                    else if (avail > 0) nh = uniform(nx_get(z, h + left - 1));
+                } else {
+                    const int v = list_entry_wave(z, h, left, mv, lane);
+                    k = lane_get(v, rcv ? e : 0);
+                    if (avail > 0) nh = uniform(next_k(z, c, wave_readlane(v, mv - 1)));
+                    /* a particle an earlier pass moved may come home: the target's run gets its links first */
+                    for (unsigned long long bk = wave_ballot(rcv & !(fT & ZF_MAT) & (k >= (int)z.k0[l]) & (k <= run_end(z, l)));
+                         bk; bk &= bk - 1ull) {
+                        if (lane == (int)__builtin_ctzll(bk)) {
+                            ensure_mat(z, l);
+                            mat = true;
+                        }
+                        ZWSYNC();
+                    }
+                }
+                /* the cell is done when phase 1 finds nothing above the
+                 * threshold; then its masks are known here */
+                const int rem = half ? 0 : uniform(dense_need(z, avail));
+                unsigned f = fT | ZF_CHG | (mat ? (unsigned)ZF_MAT : 0u);
+                if (rem <= 0 && moved == 0) {
+                    allBulk = (uniform((int)fS) & ZF_BULK0) && wave_ballot(rcv & !(fT & ZF_BULK0)) == 0ull;
+                    f |= ZF_RECV | (allBulk ? ZF_BB : ZF_SKIP);
+                    if (!allBulk) f &= ~(unsigned)ZF_BB;
+                    masked = true;
+                } else {
+                    rcvF = rcvF | rcv;
+                }
+                if (rcv) {
+                    nx_set(z, k, -1);
+                    if (tT < 0) head_set(z, l, k);
+                    else nx_set(z, tT, k);
+                    z.cell[l].cnt = (IT)(cT + 1);
+                    z.cell[l].tail = (IT)k;
+                    z.cell[l].fl = (IT)f;
+                    mark_moved(z, k, pass);
+                }
+                ZWSYNC();
+                h = nh;
+                left = imax(0, left - mv);
+                moved += mv;
+            }
+        } else {
+            /* more need than such targets and a deficit of two or more: the
+             * ranking in order into lanes 0..m-1, then the sweeps */
+            const unsigned k0 = half_bits(wave_ballot(keep & (r == 0)), half), k1 = half_bits(wave_ballot(keep & (r == 1)), half),
+                           k2 = half_bits(wave_ballot(keep & (r == 2)), half);
+            const int m0 = wave_popc(k0), m1 = wave_popc(k1), m = m0 + m1 + wave_popc(k2);
+            const int pos = (r > 0 ? m0 : 0) + (r > 1 ? m1 : 0) + round_before(r == 0 ? k0 : (r == 1 ? k1 : k2), sb, dl.bin);
+            const unsigned long long rest = ~wave_ballot(keep); /* taken by all lanes, outside the choice */
+            const int dst = keep ? pos : m + wave_popc(rest & lanes_below(lane));
+            const int lcP = lane_put(l, dst);
+            int cP = lane_put(cT, dst);
+            const double thP = lane_put_d(th, dst);
+            const int nStage = imin(need, avail);
+            const int myK = list_entry_wave(z, h, left, nStage, lane);
+            int used = 0, myT = -1, nextQ = -1, firstQ = -1, lastQ = -1;
+            const int mv = spread_plan_wave(m, thP, cP, need, avail, used, nStage, lane, myT, nextQ, firstQ, lastQ);
+            h = spread_apply_wave(z, c, h, lane, mv, avail, pass, myK, myT, nextQ, lcP, cP, firstQ, lastQ);
+            left = imax(0, left - mv);
+            moved += mv;
+            const int rc = firstQ >= 0 ? lcP : -1;
+            if (half) rg1 = rc;
+            else rg0 = rc;
+        }
+        /* phase 1: high thresholds, for what is left above the high threshold */
+        need = uniform(dense_need(z, avail));
+        if (need <= 0) break;
     }
     /* transfer masks (zone_pass.cpp:492-525) over both phases' receivers */
-    const bool nonBulk = (rcv0 >= 0 && !fget(z, rcv0, ZF_BULK0)) || (rcv1 >= 0 && !fget(z, rcv1, ZF_BULK0));
-    const bool allBulk = fget(z, src, ZF_BULK0) && wave_ballot(nonBulk) == 0ull;
-    const unsigned short setb = (unsigned short)(ZF_RECV | (allBulk ? ZF_BB : ZF_SKIP));
-    const unsigned short keepb = (unsigned short)(allBulk ? 0xffff : ~ZF_BB);
-    if (rcv0 >= 0) z.fl[rcv0] = (unsigned short)((z.fl[rcv0] | setb) & keepb);
-    ZWSYNC();
-    if (rcv1 >= 0) z.fl[rcv1] = (unsigned short)((z.fl[rcv1] | setb) & keepb);
+    if (!masked) {
+        const bool nonBulk = (rcvF && !fget(z, l, ZF_BULK0)) || (rg0 >= 0 && !fget(z, rg0, ZF_BULK0)) ||
+                             (rg1 >= 0 && !fget(z, rg1, ZF_BULK0));
+        allBulk = (uniform((int)fS) & ZF_BULK0) && wave_ballot(nonBulk) == 0ull;
+        const unsigned setb = ZF_RECV | (allBulk ? ZF_BB : ZF_SKIP), keepb = allBulk ? ~0u : ~(unsigned)ZF_BB;
+        if (rcvF) z.cell[l].fl = (IT)(((unsigned)z.cell[l].fl | setb) & keepb);
+        ZWSYNC();
+        if (rg0 >= 0) z.cell[rg0].fl = (IT)(((unsigned)z.cell[rg0].fl | setb) & keepb);
+        ZWSYNC();
+        if (rg1 >= 0) z.cell[rg1].fl = (IT)(((unsigned)z.cell[rg1].fl | setb) & keepb);
+    }
     if (lane == 0) {
-        if (allBulk) fset(z, src, ZF_BB);
-        else z.fl[src] = (unsigned short)((z.fl[src] | ZF_SKIP) & ~ZF_BB);
+        unsigned f = fS | (moved > 0 ? (unsigned)ZF_CHG : 0u) | (allBulk ? ZF_BB : ZF_SKIP);
+        if (!allBulk) f &= ~(unsigned)ZF_BB;
+        ZCell<IT> w;
+        w.cnt = (IT)avail;
+        w.head = (IT)h;
+        w.tail = avail > 0 ? S.tail : (IT)-1;
+        w.fl = (IT)f;
+        z.cell[c] = w;
     }
     ZWSYNC();
     return moved;
@@ -1272,6 +1468,7 @@ template <class Z>
 ZHD void zone_dense_passes(Z& z, int lane, int nl) {
 #if defined(__HIP_DEVICE_COMPILE__)
     int nHighW = 0, movedW = 0;
+    const DenseLane dlane = dense_lane(z, lane);
 #endif
     for (int pass = 1; pass <= z.zp.maxPasses; ++pass) {
         for (int lc = lane; lc < z.C; lc += nl) zone_maps(z, lc, 0);
@@ -1287,9 +1484,10 @@ ZHD void zone_dense_passes(Z& z, int lane, int nl) {
             if ((double)nc <= hl) continue;
             const int needOut = imax(0, (int)MPCD_CEIL((double)nc - hl));
 #if defined(__HIP_DEVICE_COMPILE__)
-            if (needOut > 0 && imin(needOut + 1, nc) <= ZONE_MAX_MOVE) {
+            if (z.zp.quadBins && needOut > 0 && imin(needOut + 1, nc) <= ZONE_MAX_MOVE) {
                 ++nHighW;
-                movedW += dense_cell_wave(z, c, nc, hl, needOut, pass, lane);
+                const int cx = lc_col(z, c);
+                movedW += dense_cell_wave(z, dlane, c, cx, c - cx * z.zh, needOut, dense_bins(z, c, pass), pass, lane);
                 continue;
             }
 #endif
@@ -1302,7 +1500,7 @@ ZHD void zone_dense_passes(Z& z, int lane, int nl) {
                 dense_targets(z, c, 0, pass, 0, lane, nl);
                 if (lane == 0) {
                     int nr = 0;
-                    moved += spread(z, c, needOut, pass, z.recvT, nr);
+                    moved += spread(z, c, needOut, pass, z.scr->recvT, nr);
                     z.sh->nr = nr;
                 }
                 ZBAR();
@@ -1311,15 +1509,15 @@ ZHD void zone_dense_passes(Z& z, int lane, int nl) {
                     dense_targets(z, c, 1, pass, 1, lane, nl);
                     if (lane == 0) {
                         int nr = z.sh->nr;
-                        moved += spread(z, c, remaining, pass, z.recvT, nr);
+                        moved += spread(z, c, remaining, pass, z.scr->recvT, nr);
                         z.sh->nr = nr;
                     }
                 }
             }
             if (lane == 0) {
                 const int nr = z.sh->nr;
-                for (int r = 0; r < nr; ++r) fset(z, z.recvT[r], ZF_RECV);
-                transfer_masks(z, c, z.recvT, nr);
+                for (int r = 0; r < nr; ++r) fset(z, z.scr->recvT[r], ZF_RECV);
+                transfer_masks(z, c, z.scr->recvT, nr);
                 z.sh->movedDense += moved;
             }
             ZBAR();
@@ -1335,6 +1533,26 @@ ZHD void zone_dense_passes(Z& z, int lane, int nl) {
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)
+/* Order-preserving compaction into z.dl by the four wavefronts from the
+ * ballots of each 64-cell chunk (at most 64 chunks); its first ZONE_TMP_L
+ * entries also go to scr->tmpL.  Returns the count. */
+template <class Z>
+__device__ __forceinline__ int zone_compact_mw(Z& z, const unsigned long long* chunkMask, int wave, int lane) {
+    const int nch = (z.C + 63) >> 6;
+    const int pc = lane < nch ? wave_popc(chunkMask[lane]) : 0;
+    const int incl = wave_shfl_up_add(pc, lane);
+    for (int ch = wave; ch < nch; ch += 4) {
+        const unsigned long long msk = chunkMask[ch];
+        const int base = wave_readlane(incl - pc, ch);
+        if ((msk >> lane) & 1ull) {
+            const int j = base + wave_popc(msk & lanes_below(lane));
+            z.dl[j] = (typename Z::idx_t)(ch * 64 + lane);
+            if (j < ZONE_TMP_L) z.scr->tmpL[j] = (typename Z::idx_t)(ch * 64 + lane);
+        }
+    }
+    return wave_readlane(incl, 63);
+}
+
 /* The dense passes on the four wavefronts of a 256-thread workgroup
  * (device only).  A dense cell's spread reads counts within Chebyshev range 2
  * of it and writes the lists, counts and flags of itself and of targets
@@ -1342,27 +1560,39 @@ ZHD void zone_dense_passes(Z& z, int lane, int nl) {
  * its high threshold, a target below it).  Cells of the shuffled list more
  * than 4 cells apart therefore touch disjoint cells and commute.  A cell
  * whose movers exceed a wavefront takes the one-lane form, which uses the
- * zone's shared scratch.  Waves 1-3 stage their movers in the one-lane form's
- * candidate scratch, free while they run. */
+ * zone's shared scratch.
+ *
+ * The wavefronts take the cells in list order from a counter in LDS; a cell
+ * starts once every earlier cell within Chebyshev range 4 is done.  Those are
+ * found through pos (the list position of each zone cell), and a finished
+ * cell sets its word in done (both in ext, idle in the dense passes).
+ * Conflicting cells thus keep the list order and the result is the serial
+ * loop's bit for bit, while a wavefront waits only for the cells its own
+ * depends on, after everything that does not depend on them (dense_prep).
+ * Cells are taken in increasing order and wait only on smaller positions,
+ * which are taken already, so the smallest unfinished cell can always run;
+ * each wait is bounded all the same (past DS_WAIT_MAX polls it records
+ * schedWait, which the kernel reports as an error, and goes on).  A list with
+ * a cell that needs the one-lane form (its movers exceed a wavefront, or the
+ * grid has no quadBins), thresholds that let a dense cell receive (low above
+ * high) or list an empty one, or a list that leaves ext no room for pos and
+ * done runs on wavefront 0 alone, in list order.
+ *
+ * What a cell writes lies in LDS, whose accesses the release and acquire
+ * order; a zone whose links spill to its global region orders those too. */
 constexpr int ZONE_WAVES = 4;
-static_assert(24 * sizeof(Cand) >= (ZONE_WAVES - 1) * ZONE_MAX_MOVE * sizeof(int),
-              "the candidate scratch holds the other wavefronts' movers");
-
-/* The dense list on the four wavefronts in list order.  Each wavefront takes
- * the next cell from a counter in LDS; a cell starts once every earlier live
- * cell within Chebyshev range 4 is done.  Those are found through pos (the
- * list position of each zone cell, after the m working words in ext), and a
- * finished cell sets DL_DONE in its word.  Conflicting cells thus keep the
- * list order and the result is the serial loop's bit for bit, while a
- * wavefront waits only for the cells its own depends on.  Cells are taken in
- * increasing order and wait only on smaller positions, which are taken
- * already, so the smallest unfinished cell can always run; each wait is
- * bounded all the same (past DS_WAIT_MAX polls it records schedWait, which
- * the kernel reports as an error, and goes on).  A list with a cell that
- * needs the one-lane form (its movers exceed a wavefront), or one that leaves
- * ext no room for pos, runs on wavefront 0 alone, in list order. */
-constexpr unsigned DL_LIVE = 0x8000u, DL_ONE = 0x4000u, DL_DONE = 0x2000u;
 constexpr int DS_WAIT_MAX = 1 << 22;
+
+template <class Z>
+__device__ __forceinline__ void sched_release(const Z& z) {
+    if (z.P > z.nL) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+}
+template <class Z>
+__device__ __forceinline__ void sched_acquire(const Z& z) {
+    if (z.P > z.nL) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 template <class Z>
 __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
@@ -1371,109 +1601,113 @@ __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
     constexpr unsigned NONE = (unsigned)(IT)~(IT)0;
     const int tid = wave * 64 + lane;
     int nHighW = 0, movedW = 0;
-    if (wave > 0) z.mvk = reinterpret_cast<int*>(z.cand) + (wave - 1) * ZONE_MAX_MOVE;
+    const DenseLane dlane = dense_lane(z, lane);
     if (tid == 0) z.sh->schedWait = 0;
     const int nExt = (z.zw + 4) * (z.zh + 4);
-    const bool wrapX = z.g.perx && z.zw == z.g.Nx, wrapY = z.g.pery && z.zh == z.g.Ny;
-    volatile IT* vext = z.ext;
+    const bool wrapX = zone_wrap_x(z), wrapY = zone_wrap_y(z);
+    /* the 9 x 9 window of a cell: lane t checks offsets t and t + 64 of the 81 */
+    const int wx0 = lane / 9 - 4, wy0 = lane % 9 - 4, wx1 = (lane + 64) / 9 - 4, wy1 = (lane + 64) % 9 - 4;
+    IT* const pos = z.ext;
+    volatile IT* const done = z.ext + z.C;
+    unsigned long long* const chunkMask = reinterpret_cast<unsigned long long*>(z.scr->cand); /* idle here */
     for (int pass = 1; pass <= z.zp.maxPasses; ++pass) {
-        for (int lc = tid; lc < z.C; lc += NT) zone_maps(z, lc, 0);
-        __syncthreads();
-        if (wave == 0) {
-            const int m = zone_compact(z, lane, 64, ZC_DENSE);
-            ZBAR();
-            zone_shuffle(z.dl, m, lane, 64, ShufDraw{z.seed, ZS_DENSE, (uint32_t)pass, 0u});
-            if (lane == 0) {
-                z.sh->mwCount = m;
-                z.sh->mwNext = 0;
-            }
-        }
-        __syncthreads();
-        const int m = z.sh->mwCount;
+        /* thresholds and the list: chunk ch of 64 cells on wavefront ch % 4 */
         bool one = false;
-        for (int k = tid; k < m; k += NT) {
-            const int c = (int)z.dl[k];
-            const int nc = cnt_of(z, c);
-            const double hl = high_thr(z, c);
-            unsigned w = 0u;
-            if (nc > 0 && (double)nc > hl) {
-                const int needOut = imax(0, (int)MPCD_CEIL((double)nc - hl));
-                const bool o = !(needOut > 0 && imin(needOut + 1, nc) <= ZONE_MAX_MOVE);
-                one = one || o;
-                w = DL_LIVE | (o ? DL_ONE : 0u);
+        for (int ch = wave; ch * 64 < z.C; ch += ZONE_WAVES) {
+            const int lc = ch * 64 + lane;
+            bool f = false;
+            if (lc < z.C) {
+                zone_maps(z, lc, 0);
+                pos[lc] = (IT)NONE;
+                const int nc = cnt_of(z, lc);
+                f = (double)nc > high_thr(z, lc) && !fget(z, lc, ZF_OUT);
+                one = one || (f && (nc <= 0 || imin(dense_need(z, nc) + 1, nc) > ZONE_MAX_MOVE));
             }
-            z.ext[k] = (IT)w;
+            const unsigned long long msk = wave_ballot(f);
+            if (lane == 0) chunkMask[ch] = msk;
         }
-        const bool serial = __syncthreads_or(one) || m + z.C > nExt;
-        IT* pos = z.ext + m;
-        if (!serial) {
-            for (int lc = tid; lc < z.C; lc += NT) pos[lc] = (IT)NONE;
-            __syncthreads();
-            for (int k = tid; k < m; k += NT)
-                if ((unsigned)z.ext[k] & DL_LIVE) pos[(int)z.dl[k]] = (IT)k;
+        for (int k = z.C + tid; k < nExt; k += NT) z.ext[k] = (IT)0;
+        bool serial = __syncthreads_or(one) || !z.zp.quadBins || z.zp.lowThrBulk > z.zp.highThr;
+        const int m = zone_compact_mw(z, chunkMask, wave, lane);
+        serial = serial || m + z.C > nExt;
+        __syncthreads();
+        /* wavefront 0 shuffles; the others meanwhile take each listed cell's
+         * surplus and start bins, from the copy of a list that fits it */
+        const bool early = m <= ZONE_TMP_L;
+        if (wave > 0) {
+            if (!serial && early)
+                for (int k = tid - 64; k < m; k += NT - 64) dense_word(z, (int)z.scr->tmpL[k], pass);
+        } else {
+            zone_shuffle(z.dl, m, lane, 64, ShufDraw{z.seed, ZS_DENSE, (uint32_t)pass, 0u});
+            if (!serial)
+                for (int k = lane; k < m; k += 64) pos[(int)z.dl[k]] = (IT)k;
+            if (lane == 0) z.sh->mwNext = 0;
+        }
+        __syncthreads();
+        if (!serial && !early) {
+            for (int k = tid; k < m; k += NT) dense_word(z, (int)z.dl[k], pass);
             __syncthreads();
         }
-        if (!serial || wave == 0)
+        if (!serial || wave == 0) {
+            /* the next position is taken one cell ahead */
+            int kv = 0;
+            if (lane == 0) kv = atomicAdd(&z.sh->mwNext, 1);
             for (;;) {
-                int k = 0;
-                if (lane == 0) k = atomicAdd(&z.sh->mwNext, 1);
-                k = __shfl(k, 0, 64);
+                const int k = uniform(kv);
                 if (k >= m) break;
-                const unsigned wk = (unsigned)vext[k];
-                if (!(wk & DL_LIVE)) continue;
-                const int c = (int)z.dl[k];
+                if (lane == 0) kv = atomicAdd(&z.sh->mwNext, 1);
+                const int c = uniform((int)z.dl[k]);
+                const int cx = lc_col(z, c), cy = c - cx * z.zh;
                 if (!serial) {
-                    /* the window's earlier live cells: lane t checks offsets t and t + 64 of the 81 */
-                    const int cx = c / z.zh, cy = c - cx * z.zh;
-                    int q0 = -1, q1 = -1;
-                    for (int h = 0; h < 2; ++h) {
-                        const int t = lane + 64 * h;
-                        int qq = -1;
-                        if (t < 81) {
-                            int x = cx + t / 9 - 4, y = cy + t % 9 - 4;
-                            bool in = true;
-                            if (wrapX) x = x < 0 ? x + z.zw : (x >= z.zw ? x - z.zw : x);
-                            else in = in && x >= 0 && x < z.zw;
-                            if (wrapY) y = y < 0 ? y + z.zh : (y >= z.zh ? y - z.zh : y);
-                            else in = in && y >= 0 && y < z.zh;
-                            if (in) {
-                                const unsigned pq = (unsigned)pos[x * z.zh + y];
-                                if (pq < (unsigned)k) qq = (int)pq;
-                            }
-                        }
-                        if (h == 0) q0 = qq;
-                        else q1 = qq;
+                    ++nHighW;
+                    int x0 = cx + wx0, y0 = cy + wy0, x1 = cx + wx1, y1 = cy + wy1;
+                    if (wrapX) {
+                        x0 = wrap_near(x0, z.g.Nx);
+                        x1 = wrap_near(x1, z.g.Nx);
                     }
+                    if (wrapY) {
+                        y0 = wrap_near(y0, z.g.Ny);
+                        y1 = wrap_near(y1, z.g.Ny);
+                    }
+                    /* outside the zone: the cell itself, which is not earlier */
+                    const bool i0 = ((unsigned)x0 < (unsigned)z.zw) & ((unsigned)y0 < (unsigned)z.zh);
+                    const bool i1 = (lane < 17) & ((unsigned)x1 < (unsigned)z.zw) & ((unsigned)y1 < (unsigned)z.zh);
+                    const int q0 = (int)pos[i0 ? x0 * z.zh + y0 : c], q1 = (int)pos[i1 ? x1 * z.zh + y1 : c];
+                    const unsigned nb = (unsigned)uniform((int)z.lix[c]);
+                    const bool w0 = q0 < k, w1 = q1 < k;
+                    const int d0 = w0 ? q0 : 0, d1 = w1 ? q1 : 0;
                     for (int polls = 0;; ++polls) {
-                        const bool wait0 = q0 >= 0 && !((unsigned)vext[q0] & DL_DONE);
-                        const bool wait1 = q1 >= 0 && !((unsigned)vext[q1] & DL_DONE);
-                        if (wave_ballot(wait0 || wait1) == 0ull) break;
+                        const int v0 = (int)done[d0], v1 = (int)done[d1];
+                        if (wave_ballot((w0 & (v0 == 0)) | (w1 & (v1 == 0))) == 0ull) break;
                         if (polls >= DS_WAIT_MAX) {
                             if (lane == 0) z.sh->schedWait = 1;
                             break;
                         }
                         __builtin_amdgcn_s_sleep(1);
                     }
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                    sched_acquire(z);
+                    movedW += dense_cell_wave(z, dlane, c, cx, cy, (int)(nb & 127u), nb >> 7, pass, lane);
+                    sched_release(z);
+                    if (lane == 0) done[k] = (IT)1;
+                    ZWSYNC();
+                    continue;
                 }
                 const int nc = cnt_of(z, c);
                 const double hl = high_thr(z, c);
-                const int needOut = imax(0, (int)MPCD_CEIL((double)nc - hl));
-                if (!(wk & DL_ONE)) {
-                    ++nHighW;
-                    movedW += dense_cell_wave(z, c, nc, hl, needOut, pass, lane);
+                if (nc <= 0 || (double)nc <= hl) continue;
+                ++nHighW;
+                const int needOut = dense_need(z, nc);
+                if (z.zp.quadBins && imin(needOut + 1, nc) <= ZONE_MAX_MOVE) {
+                    movedW += dense_cell_wave(z, dlane, c, cx, cy, needOut, dense_bins(z, c, pass), pass, lane);
                 } else {
                     /* the one-lane form (serial lists only: wavefront 0, the
                      * zone's shared scratch) */
                     int moved = 0;
-                    if (lane == 0) {
-                        ++z.sh->nHigh;
-                        z.sh->nr = 0;
-                    }
+                    if (lane == 0) z.sh->nr = 0;
                     dense_targets(z, c, 0, pass, 0, lane, 64);
                     if (lane == 0) {
                         int nr = 0;
-                        moved += spread(z, c, needOut, pass, z.recvT, nr);
+                        moved += spread(z, c, needOut, pass, z.scr->recvT, nr);
                         z.sh->nr = nr;
                     }
                     ZBAR();
@@ -1482,24 +1716,20 @@ __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
                         dense_targets(z, c, 1, pass, 1, lane, 64);
                         if (lane == 0) {
                             int nr = z.sh->nr;
-                            moved += spread(z, c, remaining, pass, z.recvT, nr);
+                            moved += spread(z, c, remaining, pass, z.scr->recvT, nr);
                             z.sh->nr = nr;
                         }
                     }
                     if (lane == 0) {
                         const int nr = z.sh->nr;
-                        for (int r = 0; r < nr; ++r) fset(z, z.recvT[r], ZF_RECV);
-                        transfer_masks(z, c, z.recvT, nr);
+                        for (int r = 0; r < nr; ++r) fset(z, z.scr->recvT[r], ZF_RECV);
+                        transfer_masks(z, c, z.scr->recvT, nr);
                         z.sh->movedDense += moved;
                     }
                     ZBAR();
                 }
-                if (!serial) {
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                    if (lane == 0) vext[k] = (IT)(wk | DL_DONE);
-                    ZWSYNC();
-                }
             }
+        }
         __syncthreads();
     }
     if (lane == 0) {
@@ -1535,11 +1765,11 @@ ZHD void inward_dir(Z& z, int gx, int gy, int lane, int nl, double& dxo, double&
     for (int t = lane; t < 4; t += nl) {
         const int qx = (t == 0) ? xa : (t == 1) ? xb : gx;
         const int qy = (t == 2) ? ya : (t == 3) ? yb : gy;
-        z.nsm4[t] = nsm_ext(z, qx, qy);
+        z.scr->nsm4[t] = nsm_ext(z, qx, qy);
     }
     ZBAR();
-    dxo = (fx == 0.5) ? 0.5 * (z.nsm4[0] - z.nsm4[1]) : (z.nsm4[0] - z.nsm4[1]);
-    dyo = (fy == 0.5) ? 0.5 * (z.nsm4[2] - z.nsm4[3]) : (z.nsm4[2] - z.nsm4[3]);
+    dxo = (fx == 0.5) ? 0.5 * (z.scr->nsm4[0] - z.scr->nsm4[1]) : (z.scr->nsm4[0] - z.scr->nsm4[1]);
+    dyo = (fy == 0.5) ? 0.5 * (z.scr->nsm4[2] - z.scr->nsm4[3]) : (z.scr->nsm4[2] - z.scr->nsm4[3]);
 }
 
 /* One donor transfer of the sparse phase (zone_pass.cpp:818-850): copy
@@ -1549,20 +1779,28 @@ template <class Z, class T>
 ZHD void donor_transfer(Z& z, int c, int d, int md, int nt, int cgc, T* tmp, int lane, int nl) {
     typedef typename Z::idx_t IT;
     /* copy the donor list, Fisher-Yates it, move the first nt */
-    if (!fget(z, d, ZF_MAT)) {
-        const int h = head_of(z, d);
-        for (int q = lane; q < md; q += nl) tmp[q] = (IT)(h + q);
-    } else if (lane == 0) {
-        int kk = head_of(z, d);
-        for (int q = 0; q < md; ++q) {
-            tmp[q] = (IT)kk;
-            kk = nx_get(z, kk);
+    {
+        const int h = head_of(z, d), left = imin(md, run_left(z, d, h));
+        for (int q = lane; q < left; q += nl) tmp[q] = (IT)(h + q);
+        if (lane == 0) {
+            int kk = left > 0 ? (left < md ? nx_get(z, h + left - 1) : -1) : h;
+            for (int q = left; q < md; ++q) {
+                tmp[q] = (IT)kk;
+                kk = nx_get(z, kk);
+            }
         }
     }
     ZBAR();
     const int dgc = lc_gc(z, d);
     zone_shuffle(tmp, md, lane, nl,
                  ShufDraw{z.seed, ZS_PARTICLE, (uint32_t)cgc, (uint32_t)dgc});
+    /* c's own particles among the movers: its run's links come first */
+    bool back = false;
+    for (int q = lane; q < nt; q += nl) back = back || in_run(z, c, (int)tmp[q]);
+    if (wave_ballot(back) != 0ull) {
+        if (lane == 0) ensure_mat(z, c);
+        ZBAR();
+    }
     /* the movers' records, links of the moved run and of the donor's
      * remaining run, all lanes */
     for (int q = lane; q < md; q += nl) {
@@ -1574,7 +1812,7 @@ ZHD void donor_transfer(Z& z, int c, int d, int md, int nt, int cgc, T* tmp, int
             nx_set(z, kq, q + 1 < md ? (int)tmp[q + 1] : -1);
         }
     }
-    ensure_mat_lanes(z, c, lane, nl);
+    ZBAR();
     if (lane == 0) {
         const int tc = tail_of(z, c);
         if (tc < 0) head_set(z, c, (int)tmp[0]);
@@ -1606,7 +1844,7 @@ ZHD int sparse_cell(Z& z, int c, int nc, int lowInt, int lane, int nl) {
         int jx, jy, q = -1;
         if (shift_idx(z, cgx, cgy, dx, dy, jx, jy)) q = zone_lc(z, jx, jy);
         if (q >= 0 && fget(z, q, ZF_OUT)) q = -1;
-        z.nbGc[o] = q;
+        z.scr->nbGc[o] = q;
     }
     ZBAR();
     int nn = 0, nd = 0;
@@ -1614,17 +1852,17 @@ ZHD int sparse_cell(Z& z, int c, int nc, int lowInt, int lane, int nl) {
         const int o = b0 + lane;
         bool keep = false;
         if (o < 8) {
-            const int q = z.nbGc[o];
+            const int q = z.scr->nbGc[o];
             keep = q >= 0;
             if (z.zp.dedupe)
                 for (int t = 0; t < o && keep; ++t)
-                    if (z.nbGc[t] == q) keep = false;
+                    if (z.scr->nbGc[t] == q) keep = false;
         }
         const unsigned long long mk = wave_ballot(keep);
         nn += wave_popc(mk);
-        const bool don = keep && cnt_of(z, z.nbGc[o]) > lowInt;
+        const bool don = keep && cnt_of(z, z.scr->nbGc[o]) > lowInt;
         const unsigned long long mdn = wave_ballot(don);
-        if (don) z.dord[nd + wave_popc(mdn & lanes_below(lane))] = z.nbGc[o];
+        if (don) z.scr->dord[nd + wave_popc(mdn & lanes_below(lane))] = z.scr->nbGc[o];
         nd += wave_popc(mdn);
     }
     ZBAR();
@@ -1634,36 +1872,36 @@ ZHD int sparse_cell(Z& z, int c, int nc, int lowInt, int lane, int nl) {
     double gxd, gyd;
     inward_dir(z, cgx, cgy, lane, nl, gxd, gyd);
     /* rank_admissible_neighbors_inward (zone_pass.cpp:636-667) */
-    zone_shuffle(z.dord, nd, lane, nl, ShufDraw{z.seed, ZS_DONOR, (uint32_t)cgc, 0u});
+    zone_shuffle(z.scr->dord, nd, lane, nl, ShufDraw{z.seed, ZS_DONOR, (uint32_t)cgc, 0u});
     const double ndir = mpcd_hypot(gxd, gyd);
     for (int t = lane; t < nd; t += nl) {
-        const int q = z.dord[t];
+        const int q = z.scr->dord[t];
         int ddx, ddy;
         min_step(z, cgx, cgy, lc_gx(z, q), lc_gy(z, q), ddx, ddy);
         const double nstep = mpcd_hypot((double)ddx, (double)ddy);
         double align = 0.0;
         if (ndir >= 1e-14 && nstep >= 1e-14) align = ((double)ddx * gxd + (double)ddy * gyd) / (ndir * nstep);
         const double noise = 1e-9 * mpcd_draw_donor_noise(z.seed, (uint32_t)cgc, (uint32_t)lc_gc(z, q));
-        z.dsc[t] = 100.0 * align + nsm_ext(z, lc_gx(z, q), lc_gy(z, q)) + noise;
+        z.scr->dsc[t] = 100.0 * align + nsm_ext(z, lc_gx(z, q), lc_gy(z, q)) + noise;
     }
     ZBAR();
     for (int t = lane; t < nd; t += nl) { /* stable, descending score */
         int r = 0;
         for (int u = 0; u < nd; ++u)
-            if (z.dsc[u] > z.dsc[t] || (u < t && !(z.dsc[t] > z.dsc[u]))) ++r;
-        z.dord2[r] = z.dord[t];
+            if (z.scr->dsc[u] > z.scr->dsc[t] || (u < t && !(z.scr->dsc[t] > z.scr->dsc[u]))) ++r;
+        z.scr->dord2[r] = z.scr->dord[t];
     }
     ZBAR();
     int moved = 0;
     for (int t = 0; t < nd; ++t) {
-        const int d = z.dord2[t];
+        const int d = z.scr->dord2[t];
         const int md = cnt_of(z, d);
         if (md <= 0) continue;
         const int avail = md - lowInt;
         if (avail <= 0) continue;
         const int nt = imin(imin(need, avail), md);
         if (nt <= 0) continue;
-        if (md <= z.tmpCap) donor_transfer(z, c, d, md, nt, cgc, z.tmpL, lane, nl);
+        if (md <= ZONE_TMP_L) donor_transfer(z, c, d, md, nt, cgc, z.scr->tmpL, lane, nl);
         else donor_transfer(z, c, d, md, nt, cgc, z.tmpG, lane, nl);
         moved += nt;
         need -= nt;
@@ -1681,10 +1919,10 @@ ZHD void sparse_setup(Z& z, int tid, int nt) {
     for (int e = tid; e < ne; e += nt) {
         const int rx = e / H - 2, ry = e % H - 2;
         const int h = halo_slot(z, rx, ry);
-        z.ext[e] = h >= 0 ? z.halo[h] : z.cnt[rx * z.zh + ry];
+        z.ext[e] = h >= 0 ? z.halo[h] : z.cell[rx * z.zh + ry].cnt;
     }
     if (z.dgCnt)
-        for (int lc = tid; lc < z.C; lc += nt) z.dgCnt[lc] = (int)z.cnt[lc];
+        for (int lc = tid; lc < z.C; lc += nt) z.dgCnt[lc] = (int)z.cell[lc].cnt;
 }
 
 /* Sparse pass (zone_pass.cpp:783-854), all lanes. */
@@ -1716,123 +1954,250 @@ ZHD void zone_sparse_pass(Z& z, int lane, int nl) {
  * cell lies within range 2 of it (lix, each cell's list index, is cleared
  * when the cell is finished); the waits are bounded as in the dense phase.
  * Conflicting cells keep the list order, so the result is the serial loop's
- * bit for bit.  A list with a cell one of whose neighbours starts with more
- * particles than a wavefront's share of the transfer scratch runs on
- * wavefront 0 alone, in list order (it has the full scratch and the global
- * region). */
-constexpr int ZONE_TMP_W = 112; /* transfer scratch of each of wavefronts 1..3 */
+ * bit for bit.
+ *
+ * The scores depend on the starting counts and the draws alone, so they are
+ * taken for all low cells at once before the loop, eight lanes per cell, into
+ * the zone's duG region (free until the correction; longer lists in
+ * segments), off the chain of conflicting cells: a cell cost 21,000 cycles
+ * with its gradient, noise draws and ranking on that chain.  Two donors of
+ * exactly equal score would be ordered by the donor shuffle, and a donor list
+ * of more than 64 entries does not fit the wavefront: a segment with either
+ * runs on wavefront 0 alone, in list order, in the general form. */
+constexpr int SPARSE_REG = 64; /* donor lists up to this length are shuffled in registers */
 
-/* a low cell with a zone neighbour at range 1 that starts the phase with
- * more particles than a wavefront's transfer scratch holds (donor lists only
- * shrink in the phase) */
+/* the four smoothed counts of inward_dir by lanes 0..3 of each group of
+ * eight, handed to the group */
 template <class Z>
-ZHD bool sparse_alone(const Z& z, int c) {
-    const int H = z.zh + 4;
-    bool big = false;
-    int jx, jy;
-    for (int dx = -1; dx <= 1; ++dx)
-        for (int dy = -1; dy <= 1; ++dy)
-            if ((dx || dy) && shift_idx(z, lc_gx(z, c), lc_gy(z, c), dx, dy, jx, jy)) {
-                const int q = zone_lc(z, jx, jy);
-                if (q >= 0 && !fget(z, q, ZF_OUT) && iget(z.ext[(q / z.zh + 2) * H + q % z.zh + 2]) > ZONE_TMP_W)
-                    big = true;
-            }
-    return big;
+__device__ __forceinline__ void inward_dir_group(const Z& z, int gx, int gy, int lane, double& dxo, double& dyo) {
+    const int Nx = z.g.Nx, Ny = z.g.Ny, t = lane & 7, g0 = lane & ~7;
+    int xa, xb, ya, yb;
+    bool hx = true, hy = true;
+    if (z.g.perx) { xa = gx + 1 < Nx ? gx + 1 : 0; xb = gx > 0 ? gx - 1 : Nx - 1; }
+    else if (gx == 0) { xa = gx + 1; xb = gx; hx = false; }
+    else if (gx == Nx - 1) { xa = gx; xb = gx - 1; hx = false; }
+    else { xa = gx + 1; xb = gx - 1; }
+    if (z.g.pery) { ya = gy + 1 < Ny ? gy + 1 : 0; yb = gy > 0 ? gy - 1 : Ny - 1; }
+    else if (gy == 0) { ya = gy + 1; yb = gy; hy = false; }
+    else if (gy == Ny - 1) { ya = gy; yb = gy - 1; hy = false; }
+    else { ya = gy + 1; yb = gy - 1; }
+    const double v = t < 4 ? nsm_ext(z, (t == 0) ? xa : (t == 1) ? xb : gx, (t == 2) ? ya : (t == 3) ? yb : gy) : 0.0;
+    const double n0 = __shfl(v, g0, 64), n1 = __shfl(v, g0 + 1, 64), n2 = __shfl(v, g0 + 2, 64), n3 = __shfl(v, g0 + 3, 64);
+    dxo = hx ? 0.5 * (n0 - n1) : (n0 - n1);
+    dyo = hy ? 0.5 * (n2 - n3) : (n2 - n3);
 }
 
+/* zone neighbour o (0..7, the order of local_neighbors_in_zone) of the cell
+ * at zone-relative (cx, cy), or -1 */
 template <class Z>
-ZHD bool sparse_conflict(const Z& z, int a, int b) {
-    int dx = a / z.zh - b / z.zh, dy = a % z.zh - b % z.zh;
-    dx = dx < 0 ? -dx : dx;
-    dy = dy < 0 ? -dy : dy;
-    if (z.g.perx && z.zw == z.g.Nx) dx = imin(dx, z.zw - dx);
-    if (z.g.pery && z.zh == z.g.Ny) dy = imin(dy, z.zh - dy);
-    return dx <= 2 && dy <= 2;
+__device__ __forceinline__ int sparse_neighbour(const Z& z, int cx, int cy, int o, int& dx, int& dy) {
+    const int f = o < 4 ? o : o + 1;
+    dy = f / 3 - 1;
+    dx = f - 3 * (f / 3) - 1;
+    int tx = cx + dx, ty = cy + dy;
+    if (zone_wrap_x(z)) tx = wrap_near(tx, z.g.Nx);
+    if (zone_wrap_y(z)) ty = wrap_near(ty, z.g.Ny);
+    const bool in = (o < 8) & ((unsigned)tx < (unsigned)z.zw) & ((unsigned)ty < (unsigned)z.zh);
+    return in ? tx * z.zh + ty : -1;
+}
+
+/* One donor transfer with the donor's list (md <= 64) in registers: as
+ * donor_transfer.  d, md, nt, dh, left uniform; fd: d's flags. */
+template <class Z>
+__device__ __forceinline__ void donor_transfer_wave(Z& z, int c, int cgc, int d, int md, int nt, int dh, int left,
+                                                    unsigned fd, int lane) {
+    typedef typename Z::idx_t IT;
+    const int dgc = lc_gc(z, d);
+    int j = 0;
+    if (lane >= 1 && lane < md)
+        j = (int)mpcd_draw_particle_shuffle(z.seed, (uint32_t)cgc, (uint32_t)dgc, (uint32_t)lane);
+    int v = list_entry_wave(z, dh, imin(left, md), md, lane);
+    v = shuffle64(v, j, md);
+    const int vn = __shfl_down(v, 1, 64);
+    ZCell<IT> C = z.cell[c];
+    unsigned fc = (unsigned)C.fl;
+    /* c's own particles among the movers: its run's links come first */
+    if (wave_ballot((lane < nt) & !(fc & ZF_MAT) & (v >= (int)z.k0[c]) & (v <= run_end(z, c))) != 0ull) {
+        if (lane == 0) ensure_mat(z, c);
+        fc |= ZF_MAT;
+        ZWSYNC();
+    }
+    if (lane < md) {
+        nx_set(z, v, (lane + 1 == nt || lane + 1 == md) ? -1 : vn);
+        if (lane < nt) mark_moved(z, v, ZM_SPARSE);
+    }
+    const int v0 = wave_readlane(v, 0), vm = wave_readlane(v, nt - 1), vr = wave_readlane(v, nt < md ? nt : 0),
+              vl = wave_readlane(v, md - 1);
+    ZWSYNC();
+    if (lane == 0) {
+        const int tc = iget(C.tail);
+        if (tc < 0) C.head = (IT)v0;
+        else nx_set(z, tc, v0);
+        const bool allBulk = (fd & ZF_BULK0) && (fc & ZF_BULK0);
+        const unsigned setb = allBulk ? ZF_BB : ZF_SKIP, keepb = allBulk ? ~0u : ~(unsigned)ZF_BB;
+        C.cnt = (IT)((int)C.cnt + nt);
+        C.tail = (IT)vm;
+        C.fl = (IT)((fc | ZF_CHG | ZF_RECV | setb) & keepb);
+        z.cell[c] = C;
+        ZCell<IT> D;
+        D.cnt = (IT)(md - nt);
+        D.head = (IT)(md > nt ? vr : -1);
+        D.tail = (IT)(md > nt ? vl : -1);
+        D.fl = (IT)((fd | ZF_MAT | ZF_CHG | setb) & keepb);
+        z.cell[d] = D;
+    }
+    ZWSYNC();
 }
 
 template <class Z>
 __device__ __forceinline__ void zone_sparse_pass_mw(Z& z, int wave, int lane) {
     typedef typename Z::idx_t IT;
-    static_assert(sizeof(IT) == 2, "the wavefronts' scratch shares are laid out for 16-bit indices");
+    static_assert(sizeof(IT) == 2, "the scheduled phases take 16-bit indices");
+    constexpr int NT = 64 * ZONE_WAVES;
     const int tid = wave * 64 + lane;
-    if (wave > 0) {
-        /* this wavefront's scratch: 448 bytes of the dense phase's one-lane
-         * candidate and threshold arrays (cand, ordThr, nbTie, contiguous and
-         * idle now) */
-        unsigned char* b = reinterpret_cast<unsigned char*>(z.cand) + (wave - 1) * 448;
-        z.dsc = reinterpret_cast<double*>(b);
-        z.nsm4 = reinterpret_cast<double*>(b + 64);
-        z.nbGc = reinterpret_cast<int*>(b + 96);
-        z.dord = reinterpret_cast<int*>(b + 128);
-        z.dord2 = reinterpret_cast<int*>(b + 160);
-        z.tmpL = reinterpret_cast<IT*>(b + 224);
-        z.tmpCap = ZONE_TMP_W;
-    }
     const IT none = (IT)~(IT)0;
-    sparse_setup(z, tid, 64 * ZONE_WAVES);
-    for (int lc = tid; lc < z.C; lc += 64 * ZONE_WAVES) z.lix[lc] = none;
+    unsigned long long* const chunkMask = reinterpret_cast<unsigned long long*>(z.scr->cand);
+    const int lowInt = (int)MPCD_CEIL(z.zp.lowThrBulk);
+    /* maps, the low cells, and the counts the phase starts from (the zone and
+     * its ring) in ext */
+    for (int ch = wave; ch * 64 < z.C; ch += ZONE_WAVES) {
+        const int lc = ch * 64 + lane;
+        bool f = false;
+        if (lc < z.C) {
+            zone_maps(z, lc, 0);
+            z.lix[lc] = none;
+            const int nc = cnt_of(z, lc);
+            f = nc > 0 && (double)nc < low_thr(z, lc) && !fget(z, lc, ZF_OUT);
+            const int ix = lc_col(z, lc);
+            z.ext[(ix + 2) * (z.zh + 4) + (lc - ix * z.zh) + 2] = (IT)nc;
+            if (z.dgCnt) z.dgCnt[lc] = nc;
+        }
+        const unsigned long long msk = wave_ballot(f);
+        if (lane == 0) chunkMask[ch] = msk;
+    }
+    for (int h = tid; h < halo_size(z); h += NT) {
+        int rx, ry;
+        halo_xy(z, h, rx, ry);
+        z.ext[rx * (z.zh + 4) + ry] = z.halo[h];
+    }
+    __syncthreads();
+    const int m = zone_compact_mw(z, chunkMask, wave, lane);
     __syncthreads();
     if (wave == 0) {
-        const int m = zone_compact(z, lane, 64, ZC_LOW);
-        ZBAR();
         zone_shuffle(z.dl, m, lane, 64, ShufDraw{z.seed, ZS_LOW, 0u, 0u});
-        if (lane == 0) z.sh->mwCount = m;
+        for (int k = lane; k < m; k += 64) z.lix[(int)z.dl[k]] = (IT)k;
     }
     __syncthreads();
-    const int m = z.sh->mwCount;
-    bool anyAlone = false;
-    for (int k = tid; k < m; k += 64 * ZONE_WAVES) {
-        const int c = (int)z.dl[k];
-        z.lix[c] = (IT)k;
-        anyAlone = anyAlone || sparse_alone(z, c);
-    }
-    anyAlone = __syncthreads_or(anyAlone);
-    const int lowInt = (int)MPCD_CEIL(z.zp.lowThrBulk);
-    const bool wx = z.g.perx && z.zw == z.g.Nx, wy = z.g.pery && z.zh == z.g.Ny;
     int nLowW = 0, movedW = 0;
-    const bool serial = anyAlone;
-    if (tid == 0) z.sh->mwNext = 0;
-    __syncthreads();
     volatile IT* vlix = z.lix;
-    if (!serial || wave == 0)
-        for (;;) {
-            int k = 0;
-            if (lane == 0) k = atomicAdd(&z.sh->mwNext, 1);
-            k = __shfl(k, 0, 64);
-            if (k >= m) break;
-            const int c = (int)z.dl[k];
-            if (!serial) {
-                int q = -1;
-                if (lane < 25) {
-                    const int rx = c / z.zh, ry = c - rx * z.zh;
-                    int qx = rx + lane / 5 - 2, qy = ry + lane % 5 - 2;
-                    if (wx) qx = wrapi(qx, z.zw);
-                    if (wy) qy = wrapi(qy, z.zh);
-                    if (qx >= 0 && qx < z.zw && qy >= 0 && qy < z.zh) q = qx * z.zh + qy;
+    double* const score = z.duG; /* 8 per low cell of the segment */
+    const int SEG = imax(1, z.C / 4);
+    const bool noSeg = z.C < 4 || z.zp.dedupe != 0;
+    for (int s0 = 0; s0 < m; s0 += SEG) {
+        const int s1 = imin(m, s0 + SEG);
+        /* scores: eight lanes per low cell */
+        bool alone = noSeg;
+        if (!noSeg)
+            for (int g0 = s0; g0 < s1; g0 += NT / 8) {
+                const int k = g0 + (tid >> 3), o = lane & 7;
+                const bool act = k < s1;
+                const int c = (int)z.dl[act ? k : s0];
+                const int cx = lc_col(z, c), cy = c - cx * z.zh;
+                int dx, dy;
+                int q = sparse_neighbour(z, cx, cy, o, dx, dy);
+                const int qs = q >= 0 ? q : c, qx = lc_col(z, qs), qy = qs - qx * z.zh;
+                const int n0 = iget(z.ext[(qx + 2) * (z.zh + 4) + qy + 2]);
+                const bool don = act && q >= 0 && !fget(z, qs, ZF_OUT) && n0 > lowInt;
+                double gxd, gyd;
+                inward_dir_group(z, z.xs + cx, z.ys + cy, lane, gxd, gyd);
+                double sc = 0.0;
+                if (don) {
+                    const double ndir = mpcd_hypot(gxd, gyd), nstep = mpcd_hypot((double)dx, (double)dy);
+                    double align = 0.0;
+                    if (ndir >= 1e-14 && nstep >= 1e-14) align = ((double)dx * gxd + (double)dy * gyd) / (ndir * nstep);
+                    const double noise = 1e-9 * mpcd_draw_donor_noise(z.seed, (uint32_t)lc_gc(z, c), (uint32_t)lc_gc(z, qs));
+                    sc = 100.0 * align + nsm_ext(z, z.xs + qx, z.ys + qy) + noise;
                 }
+                if (act) score[8 * (k - s0) + o] = sc;
+                alone = alone || (don && n0 > SPARSE_REG);
+                const unsigned long long dm = wave_ballot(don) >> (lane & ~7);
+                for (int u = 1; u < 8; ++u) {
+                    const int p = (o + u) & 7;
+                    const double other = __shfl(sc, (lane & ~7) + p, 64);
+                    if (don && ((dm >> p) & 1ull) && !(other < sc) && !(other > sc)) alone = true;
+                }
+            }
+        if (tid == 0) z.sh->mwNext = s0;
+        __threadfence_block(); /* the scores lie in global memory */
+        const bool serial = __syncthreads_or(alone) != 0;
+        if (serial) {
+            if (wave == 0)
+                for (int k = s0; k < s1; ++k) {
+                    const int c = (int)z.dl[k];
+                    const int nc = cnt_of(z, c);
+                    if (nc <= 0) continue;
+                    ++nLowW;
+                    movedW += sparse_cell(z, c, nc, lowInt, lane, 64);
+                }
+        } else {
+            int kv = 0;
+            if (lane == 0) kv = atomicAdd(&z.sh->mwNext, 1);
+            for (;;) {
+                const int k = uniform(kv);
+                if (k >= s1) break;
+                if (lane == 0) kv = atomicAdd(&z.sh->mwNext, 1);
+                const int c = uniform((int)z.dl[k]);
+                const int cx = lc_col(z, c), cy = c - cx * z.zh;
+                int dx, dy;
+                int q = sparse_neighbour(z, cx, cy, lane, dx, dy);
+                const double sc = lane < 8 ? score[8 * (k - s0) + lane] : 0.0;
+                const int nc = uniform(cnt_of(z, c)); /* only this treatment changes it */
+                /* earlier cells within range 2 (lanes 0..24) */
+                int wx = cx + lane / 5 - 2, wy = cy + lane % 5 - 2;
+                if (zone_wrap_x(z)) wx = wrap_near(wx, z.g.Nx);
+                if (zone_wrap_y(z)) wy = wrap_near(wy, z.g.Ny);
+                const bool wi = (lane < 25) & ((unsigned)wx < (unsigned)z.zw) & ((unsigned)wy < (unsigned)z.zh);
+                const int wq = wi ? wx * z.zh + wy : c;
                 for (int polls = 0;; ++polls) {
-                    const bool wait = q >= 0 && (int)vlix[q] < k;
-                    if (wave_ballot(wait) == 0ull) break;
+                    if (wave_ballot((int)vlix[wq] < k) == 0ull) break;
                     if (polls >= DS_WAIT_MAX) {
                         if (lane == 0) z.sh->schedWait = 1;
                         break;
                     }
                     __builtin_amdgcn_s_sleep(1);
                 }
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            }
-            const int nc = cnt_of(z, c);
-            if (nc > 0) {
+                sched_acquire(z);
                 ++nLowW;
-                movedW += sparse_cell(z, c, nc, lowInt, lane, 64);
-            }
-            if (!serial) {
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                int need = imax(0, lowInt - nc);
+                const int qs = q >= 0 ? q : c;
+                const ZCell<IT> Q = z.cell[qs];
+                const int kb = (int)z.k0[qs], ke = run_end(z, qs);
+                const int qc = (int)Q.cnt, qh = iget(Q.head);
+                const unsigned qf = (unsigned)Q.fl;
+                const bool don = (q >= 0) & !(qf & ZF_OUT) & (qc > lowInt);
+                const int ql = (qf & ZF_MAT) || qh < kb || qh > ke ? 0 : ke - qh + 1;
+                const unsigned long long md0 = wave_ballot(don);
+                /* rank by descending score */
+                int r = 0;
+                for (unsigned long long mm = md0; mm; mm &= mm - 1ull) r += wave_readlane_d(sc, (int)__builtin_ctzll(mm)) > sc ? 1 : 0;
+                const int nd = wave_popc(md0);
+                for (int t = 0; t < nd && need > 0; ++t) {
+                    const int o = (int)__builtin_ctzll(wave_ballot(don & (r == t)));
+                    const int md = wave_readlane(qc, o);
+                    const int nt = imin(imin(need, md - lowInt), md);
+                    if (nt <= 0) continue;
+                    donor_transfer_wave(z, c, lc_gc(z, c), wave_readlane(q, o), md, nt, wave_readlane(qh, o),
+                                        wave_readlane(ql, o), (unsigned)wave_readlane((int)qf, o), lane);
+                    movedW += nt;
+                    need -= nt;
+                }
+                sched_release(z);
                 if (lane == 0) vlix[c] = none;
                 ZWSYNC();
             }
         }
-    __syncthreads();
+        __syncthreads();
+    }
     if (lane == 0) {
         atomicAdd(&z.sh->nLow, nLowW);
         atomicAdd(&z.sh->movedSparse, movedW);
@@ -1859,21 +2224,8 @@ ZHD unsigned short setup_flags(const Z& z, const ZoneIn& in, int gc) {
 /* zone_setup's entry h of the ring of pass-input counts around the zone */
 template <class Z>
 ZHD void setup_halo(Z& z, int h) {
-    const int W4 = z.zw + 4;
     int hx, hy;
-    if (h < 2 * W4) {
-        hx = h / 2;
-        hy = h % 2;
-    } else if (h < 4 * W4) {
-        hx = (h - 2 * W4) / 2;
-        hy = z.zh + 2 + (h - 2 * W4) % 2;
-    } else if (h < 4 * W4 + 2 * z.zh) {
-        hx = (h - 4 * W4) / z.zh;
-        hy = 2 + (h - 4 * W4) % z.zh;
-    } else {
-        hx = z.zw + 2 + (h - 4 * W4 - 2 * z.zh) / z.zh;
-        hy = 2 + (h - 4 * W4 - 2 * z.zh) % z.zh;
-    }
+    halo_xy(z, h, hx, hy);
     int gx = z.xs + hx - 2, gy = z.ys + hy - 2;
     if (z.g.perx) gx = wrapi(gx, z.g.Nx);
     if (z.g.pery) gy = wrapi(gy, z.g.Ny);
@@ -1904,7 +2256,7 @@ ZHD void zone_setup(Z& z, const ZoneIn& in, int lane, int nl) {
             tail_set(z, lc, m > 0 ? k0 + m - 1 : -1);
             const unsigned short f = setup_flags(z, in, gc);
             if ((f & (ZF_OWN | ZF_COVER)) != ZF_OWN) mixed = true;
-            z.fl[lc] = f;
+            z.cell[lc].fl = (typename Z::idx_t)f;
             if (lc % z.zh == 0) {
                 z.colL[lc / z.zh] = k0;
                 z.colG[lc / z.zh] = z.gstart[gc];
@@ -1970,7 +2322,7 @@ ZHD void zone_setup_mw(Z& z, const ZoneIn& in, int wave, int lane) {
         const int gc = lc_gc(z, lc);
         const unsigned short f = setup_flags(z, in, gc);
         if ((f & (ZF_OWN | ZF_COVER)) != ZF_OWN) mixed = true;
-        z.fl[lc] = f;
+        z.cell[lc].fl = (typename Z::idx_t)f;
         if (lc % z.zh == 0) z.colG[lc / z.zh] = z.gstart[gc];
     }
     const int nh = halo_size(z);
@@ -2179,17 +2531,13 @@ template <class IT>
 ZHD size_t zone_fixed_bytes(int C, int W, int useLocal) {
     size_t b = 0;
     if (useLocal) b += (size_t)C * 2 * sizeof(double);         /* lowA highA */
-    b += 24 * sizeof(Cand) + 2 * 24 * sizeof(double) + 8 * sizeof(double) + 4 * sizeof(double) +
-         (size_t)ZONE_MAX_MOVE * sizeof(int); /* 8-byte items first */
+    b += sizeof(ZScratch<IT>);                                  /* 8-byte items first */
     b += (size_t)W * 2 * sizeof(int);                           /* colL colG */
-    b += (5 * 24 + 3 * 8) * sizeof(int);                        /* ord nbGc rnk recvT (+pad) dord dord2 (+pad) */
-    b += (size_t)C * 5 * sizeof(IT);                            /* cnt head tail dl k0 */
+    b += (size_t)C * sizeof(ZCell<IT>);                         /* cell */
+    b += (size_t)C * 3 * sizeof(IT);                            /* k0 dl lix */
     b += (size_t)(W + 4) * (size_t)(C / (W > 0 ? W : 1) + 4) * sizeof(IT); /* ext */
     b += (size_t)(4 * (W + 4) + 4 * (C / (W > 0 ? W : 1))) * sizeof(IT); /* halo */
-    b += (size_t)C * sizeof(unsigned short); /* fl */
-    b += (size_t)C * sizeof(IT);             /* lix */
-    b += (size_t)ZONE_TMP_L * sizeof(IT);                       /* tmpL */
-    b += 4 + 16;                                                /* alignment after fl and after colG */
+    b += 32;                                                    /* alignment after k0 and colG */
     return (b + 15) & ~(size_t)15;
 }
 
@@ -2202,11 +2550,8 @@ ZHD void zone_carve(ZoneCtxT<IT>& z, unsigned char* base, size_t bytes) {
     /* first what the correction keeps (cell arrays, column map), at the
      * offsets of the correction's own LDS layout, so the correction that
      * follows the passes in one kernel finds them in place */
-    z.cnt = (IT*)p; p += (size_t)C * sizeof(IT);
-    z.head = (IT*)p; p += (size_t)C * sizeof(IT);
-    z.tail = (IT*)p; p += (size_t)C * sizeof(IT);
+    z.cell = (ZCell<IT>*)p; p += (size_t)C * sizeof(ZCell<IT>);
     z.k0 = (IT*)p; p += (size_t)C * sizeof(IT);
-    z.fl = (unsigned short*)p; p += (size_t)C * sizeof(unsigned short);
     p = base + (((size_t)(p - base) + 3) & ~(size_t)3);
     z.colL = (int*)p; p += (size_t)W * sizeof(int);
     z.colG = (int*)p; p += (size_t)W * sizeof(int);
@@ -2219,23 +2564,10 @@ ZHD void zone_carve(ZoneCtxT<IT>& z, unsigned char* base, size_t bytes) {
         z.lowA = nullptr;
         z.highA = nullptr;
     }
-    z.cand = (Cand*)p; p += 24 * sizeof(Cand);
-    z.ordThr = (double*)p; p += 24 * sizeof(double);
-    z.nbTie = (double*)p; p += 24 * sizeof(double);
-    z.dsc = (double*)p; p += 8 * sizeof(double);
-    z.nsm4 = (double*)p; p += 4 * sizeof(double);
-    z.mvk = (int*)p; p += ZONE_MAX_MOVE * sizeof(int);
-    z.ord = (int*)p; p += 24 * sizeof(int);
-    z.nbGc = (int*)p; p += 24 * sizeof(int);
-    z.rnk = (int*)p; p += 24 * sizeof(int);
-    z.recvT = (int*)p; p += 48 * sizeof(int);
-    z.dord = (int*)p; p += 8 * sizeof(int);
-    z.dord2 = (int*)p; p += 16 * sizeof(int);
+    z.scr = (ZScratch<IT>*)p; p += sizeof(ZScratch<IT>);
     z.dl = (IT*)p; p += (size_t)C * sizeof(IT);
     z.ext = (IT*)p; p += (size_t)(z.zw + 4) * (size_t)(z.zh + 4) * sizeof(IT);
     z.halo = (IT*)p; p += (size_t)halo_size(z) * sizeof(IT);
-    z.tmpL = (IT*)p; p += (size_t)ZONE_TMP_L * sizeof(IT);
-    z.tmpCap = ZONE_TMP_L;
     z.lix = (IT*)p; p += (size_t)C * sizeof(IT);
     const size_t fixed = zone_fixed_bytes<IT>(C, W, z.zp.useLocal);
     p = base + fixed;
@@ -2257,6 +2589,7 @@ ZHD void zone_init(ZoneCtxT<IT>& z, const ZoneIn& in, ZoneRect r, int zid, uint6
     z.zw = r.xe - r.xs;
     z.zh = r.ye - r.ys;
     z.C = z.zw * z.zh;
+    z.zhM = z.zh > 1 ? 0xffffffffu / (unsigned)z.zh + 1u : 0u;
     z.zid = zid;
     z.seed = seed;
     z.gcnt = in.gcnt;
@@ -2305,20 +2638,20 @@ ZHD void zone_run(Z& z, int lane, int nl) {
  * threads per zone: the pass kernel leaves the cell arrays, the column map
  * and the flags in a per-zone state region of global memory, and the links
  * all in the zone's global link region.  Layout (16-byte aligned):
- * |dsq C doubles|hdr 4 ints|colL W ints|colG W ints|cnt|head|tail|k0 C IT each|fl C u16| */
+ * |dsq C doubles|cell C ZCell|hdr 4 ints|colL W ints|colG W ints|k0 C IT| */
 template <class IT>
 struct ZoneState {
     double* dsq; /* |du|^2 of each cell, for the ordered stats */
     int* hdr;    /* P, allOwned */
     int *colL, *colG;
-    IT *cnt, *head, *tail, *k0;
-    unsigned short* fl;
+    ZCell<IT>* cell;
+    IT* k0;
 };
 
 template <class IT>
 ZHD size_t zone_state_bytes(int C, int W) {
-    const size_t b = (size_t)C * sizeof(double) + 4 * sizeof(int) + (size_t)W * 2 * sizeof(int) +
-                     (size_t)C * 4 * sizeof(IT) + (size_t)C * sizeof(unsigned short);
+    const size_t b = (size_t)C * sizeof(double) + (size_t)C * sizeof(ZCell<IT>) + 4 * sizeof(int) +
+                     (size_t)W * 2 * sizeof(int) + (size_t)C * sizeof(IT) + sizeof(ZCell<IT>);
     return (b + 15) & ~(size_t)15;
 }
 
@@ -2327,14 +2660,12 @@ ZHD ZoneState<IT> zone_state_at(unsigned char* base, int C, int W) {
     ZoneState<IT> st;
     unsigned char* p = base;
     st.dsq = (double*)p; p += (size_t)C * sizeof(double);
+    p = base + (((size_t)(p - base) + sizeof(ZCell<IT>) - 1) & ~(sizeof(ZCell<IT>) - 1));
+    st.cell = (ZCell<IT>*)p; p += (size_t)C * sizeof(ZCell<IT>);
     st.hdr = (int*)p; p += 4 * sizeof(int);
     st.colL = (int*)p; p += (size_t)W * sizeof(int);
     st.colG = (int*)p; p += (size_t)W * sizeof(int);
-    st.cnt = (IT*)p; p += (size_t)C * sizeof(IT);
-    st.head = (IT*)p; p += (size_t)C * sizeof(IT);
-    st.tail = (IT*)p; p += (size_t)C * sizeof(IT);
-    st.k0 = (IT*)p; p += (size_t)C * sizeof(IT);
-    st.fl = (unsigned short*)p;
+    st.k0 = (IT*)p;
     return st;
 }
 
@@ -2343,11 +2674,8 @@ ZHD ZoneState<IT> zone_state_at(unsigned char* base, int C, int W) {
 template <class IT>
 ZHD void zone_dump(ZoneCtxT<IT>& z, const ZoneState<IT>& st, int lane, int nl) {
     for (int lc = lane; lc < z.C; lc += nl) {
-        st.cnt[lc] = z.cnt[lc];
-        st.head[lc] = z.head[lc];
-        st.tail[lc] = z.tail[lc];
+        st.cell[lc] = z.cell[lc];
         st.k0[lc] = z.k0[lc];
-        st.fl[lc] = z.fl[lc];
     }
     for (int c = lane; c < z.zw; c += nl) {
         st.colL[c] = z.colL[c];
@@ -2367,11 +2695,8 @@ ZHD void zone_dump(ZoneCtxT<IT>& z, const ZoneState<IT>& st, int lane, int nl) {
  * state region, every link in the global link region */
 template <class IT>
 ZHD void zone_attach_state(ZoneCtxT<IT>& z, const ZoneState<IT>& st) {
-    z.cnt = st.cnt;
-    z.head = st.head;
-    z.tail = st.tail;
+    z.cell = st.cell;
     z.k0 = st.k0;
-    z.fl = st.fl;
     z.colL = st.colL;
     z.colG = st.colG;
     z.P = st.hdr[0];
@@ -2472,24 +2797,34 @@ __device__ __forceinline__ void fin_input_sum_group(const Z& z, int lc, int r, i
     pby = py;
 }
 
+/* A final list as a group walks it: its head, the entries still implicit,
+ * and the walk along the links (entry at and local index kw). */
+struct FinWalk {
+    int h, left, at, kw;
+};
 template <class Z>
-__device__ __forceinline__ void fin_group_entries(const Z& z, bool mat, int h, int t, int m, int c0, int r, int& kw,
-                                                  int* kk) {
-    for (int u = 0; u < FIN_L; ++u) kk[u] = -1;
-    if (!mat) {
-        for (int u = 0; u < FIN_L; ++u) {
-            const int e = c0 + FIN_L * r + u;
-            kk[u] = (e < m && h + e <= t) ? h + e : -1;
-        }
-        return;
+__device__ __forceinline__ FinWalk fin_walk(const Z& z, int lc, int m) {
+    FinWalk w;
+    w.h = head_of(z, lc);
+    w.left = imin(m, run_left(z, lc, w.h));
+    w.at = w.left;
+    w.kw = w.left > 0 ? (w.left < m ? nx_get(z, w.h + w.left - 1) : -1) : w.h;
+    return w;
+}
+/* entries [c0 + FIN_L r, c0 + FIN_L (r + 1)) of the list of m entries (-1
+ * beyond its end): the run's by their indices, the others by the walk, which
+ * the whole group takes in step */
+template <class Z>
+__device__ __forceinline__ void fin_group_entries(const Z& z, FinWalk& w, int m, int c0, int r, int* kk) {
+    constexpr int CH = FIN_G * FIN_L;
+    const int e0 = c0 + FIN_L * r;
+    for (int u = 0; u < FIN_L; ++u) kk[u] = e0 + u < w.left ? w.h + e0 + u : -1;
+    const int end = imin(m, c0 + CH);
+    while (w.at < end) {
+        const int q = w.at - e0;
+        for (int u = 0; u < FIN_L; ++u) kk[u] = q == u ? w.kw : kk[u];
+        if (++w.at < m) w.kw = nx_get(z, w.kw);
     }
-    int k = kw;
-    for (int a = 0; a < FIN_G; ++a)
-        for (int u = 0; u < FIN_L; ++u) {
-            if (a == r) kk[u] = k;
-            if (k >= 0) k = nx_get(z, k);
-        }
-    kw = k;
 }
 
 template <class Z>
@@ -2497,17 +2832,15 @@ __device__ __forceinline__ double fin_cell_group(Z& z, int lc, int r, int lane, 
     constexpr int CH = FIN_G * FIN_L;
     const int m = cnt_of(z, lc);
     const int kb = (int)z.k0[lc], ke = kb + in_cnt(z, lc);
-    const bool mat = fget(z, lc, ZF_MAT);
-    const int t = tail_of(z, lc), h = head_of(z, lc);
-    const unsigned short ownLc = (unsigned short)(z.fl[lc] & (ZF_OWN | ZF_COVER));
+    FinWalk w = fin_walk(z, lc, m);
+    const unsigned short ownLc = (unsigned short)((unsigned)z.cell[lc].fl & (ZF_OWN | ZF_COVER));
     const int g0 = lane - r;
     int kk[FIN_L], sl[FIN_L];
     unsigned short ow[FIN_L];
     double ax[FIN_L], ay[FIN_L];
     double px = 0.0, py = 0.0;
-    int kw = h;
     for (int c0 = 0; c0 < m; c0 += CH) {
-        fin_group_entries(z, mat, h, t, m, c0, r, kw, kk);
+        fin_group_entries(z, w, m, c0, r, kk);
         for (int u = 0; u < FIN_L; ++u) {
             sl[u] = -1;
             ow[u] = 0;
@@ -2540,9 +2873,9 @@ __device__ __forceinline__ double fin_cell_group(Z& z, int lc, int r, int lane, 
     if (corr && !(dux != 0.0 || duy != 0.0)) corr = false;
     if (m > CH) {
         /* a longer list: walk it again for the writes */
-        kw = h;
+        w = fin_walk(z, lc, m);
         for (int c0 = 0; c0 < m; c0 += CH) {
-            fin_group_entries(z, mat, h, t, m, c0, r, kw, kk);
+            fin_group_entries(z, w, m, c0, r, kk);
             for (int u = 0; u < FIN_L; ++u) {
                 sl[u] = -1;
                 ow[u] = 0;
