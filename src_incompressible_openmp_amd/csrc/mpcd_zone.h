@@ -2139,6 +2139,8 @@ __device__ __forceinline__ void zone_sparse_pass_mw(Z& z, int wave, int lane) {
                     ++nLowW;
                     movedW += sparse_cell(z, c, nc, lowInt, lane, 64);
                 }
+            /* later segments wait for none of these */
+            for (int k = s0 + tid; k < s1; k += NT) z.lix[(int)z.dl[k]] = none;
         } else {
             int kv = 0;
             if (lane == 0) kv = atomicAdd(&z.sh->mwNext, 1);

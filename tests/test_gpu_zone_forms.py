@@ -1,0 +1,83 @@
+"""The zone kernel's forms against the oracle (bitwise states, exact moved
+counts) where their choice changes: periodic axes one cell wider than a zone
+(wrapped neighbours inside it) and as wide as it, axes narrower than five
+cells, zones one cell wide or high, dense lists past one and two registers of
+shuffle and past the list copy, cells with more movers than a wavefront,
+donor lists past the registers, thresholds that let a dense cell receive,
+several passes (lists that take back their own particles), local thresholds.
+Inputs are what a pass meets (streamed and collided states) or crowded ones."""
+import numpy as np
+import pytest
+
+from src_incompressible_openmp_amd.fileio import uniform_state
+from src_incompressible_openmp_amd.params import LAYOUT_BASE, LAYOUT_SHIFTED, poiseuille_params, to_struct
+from tests.oracle_lib import CTR
+
+pytestmark = pytest.mark.gpu
+
+FORMS = {
+    "wrap_gap_of_one": dict(Nx=26, Ny=26, gamma=12.0, boundary_bottom="periodic", boundary_top="periodic"),
+    "wrap_full_axis": dict(Nx=25, Ny=25, gamma=12.0, boundary_bottom="periodic", boundary_top="periodic"),
+    "narrow_periodic": dict(Nx=4, Ny=30, gamma=15.0),
+    "one_wide": dict(Nx=31, Ny=23, gamma=10.0, zoneTileNx=1, zoneTileNy=9),
+    "one_high": dict(Nx=31, Ny=23, gamma=10.0, zoneTileNx=10, zoneTileNy=1),
+    "list_past_128": dict(Nx=60, Ny=45, gamma=12.0, coef=0.02, zoneTileNx=30, zoneTileNy=30),
+    "list_past_copy": dict(Nx=80, Ny=40, gamma=12.0, coef=0.02, zoneTileNx=40, zoneTileNy=40),
+    "low_above_high": dict(Nx=40, Ny=30, gamma=12.0, lowThrBulkOverride=16.0),
+    "many_passes": dict(Nx=50, Ny=30, gamma=9.0, coef=0.01, maxRedistribPasses=6),
+    "local_thresholds": dict(Nx=50, Ny=30, gamma=6.0, useLocalFluidFractionThresholds=True, highMode="1+coef",
+                             lowMode="1+coef", coef=0.2, lowThrFloor=3.0, highThrFloor=8.0),
+    "dense_population": dict(Nx=30, Ny=26, gamma=90.0),
+}
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    from src_incompressible_openmp_amd import gpu as g
+
+    g.load()
+    assert g.device_count() >= 1, "no GPU visible"
+    return g
+
+
+def state(p, crowded):
+    x, v, _, _ = uniform_state(p.n, p.Lx, p.Ly, seed=17)
+    if crowded:  # a third of the particles in six spots: surpluses past a wavefront, empty cells
+        rng = np.random.default_rng(5)
+        m = p.n // 3
+        spot = rng.integers(0, 6, size=m)
+        cx, cy = rng.random(6) * p.Lx, rng.random(6) * p.Ly
+        x[0:2 * m:2] = np.clip(cx[spot] + 0.3 * rng.standard_normal(m), 0.0, p.Lx * (1.0 - 1e-9))
+        x[1:2 * m:2] = np.clip(cy[spot] + 0.3 * rng.standard_normal(m), 0.0, p.Ly * (1.0 - 1e-9))
+    return x, v
+
+
+@pytest.mark.parametrize("crowded", [False, True], ids=["uniform", "crowded"])
+@pytest.mark.parametrize("form", sorted(FORMS))
+def test_zone_pass_forms(gpu, oracle, form, crowded):
+    p = to_struct(poiseuille_params(**FORMS[form]))
+    for layout in (LAYOUT_BASE, LAYOUT_SHIFTED):
+        x, v = state(p, crowded)
+        xo, vo = x.copy(), v.copy()
+        m, _ = oracle.zone_pass(CTR, p, xo, vo, layout, 88172645463325252)
+        g, _ = gpu.zone_pass(p, x, v, layout, 88172645463325252)
+        assert g["nParticlesMovedDense"] == m["nParticlesMovedDense"], layout
+        assert g["nParticlesMovedSparse"] == m["nParticlesMovedSparse"], layout
+        assert x.tobytes() == xo.tobytes(), layout
+        assert v.tobytes() == vo.tobytes(), layout
+
+
+def test_steps_after_a_wrapped_zone(gpu, oracle):
+    """Whole steps on the grid one cell wider than a zone: the binning update
+    after the pass sees the moved particles."""
+    p = to_struct(poiseuille_params(**FORMS["wrap_gap_of_one"]))
+    x, v = state(p, False)
+    sim = gpu.Sim(p)
+    sim.set_state(x, v)
+    sim.step(1, 2)
+    xg, vg = sim.get_state()
+    sim.close()
+    for s in (1, 2):
+        oracle.step(CTR, p, x, v, s)
+    assert xg.tobytes() == x.tobytes()
+    assert float(np.max(np.abs(vg - v))) <= 1e-12 * max(1.0, float(np.max(np.abs(v))))
