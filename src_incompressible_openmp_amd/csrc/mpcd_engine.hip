@@ -990,6 +990,7 @@ struct ZoneArgs {
     unsigned char* gscratch; /* working sets in global memory when they do not fit LDS */
     size_t gstride;
     ZoneOut* out;
+    int wantStats; /* the correction's stats4, stats5 are read */
     int* err;
     /* an ensemble's pass (the kEns kernels): zone -> replica, the replicas'
      * own inputs (binning views, owner and cover maps, geometry, thresholds),
@@ -1114,22 +1115,13 @@ __global__ void __launch_bounds__(ZONE_TPB) k_zone(ZoneArgs a) {
  * order), then one wavefront for the ordered stats. */
 constexpr int FINISH_TPB = 256;
 constexpr int FINISH_LDS = 40 * 1024; /* cell arrays, column map and as many links as fit */
-/* The passes' zone, still in the workgroup's LDS (zone_carve's layout), for
- * the correction in the same kernel: its particle count, ownership flag and
- * the number of links the passes held in LDS. */
-struct ZoneHandoff {
-    int P, allOwned, nL;
-};
-
 /* The correction of zone zi by TPB threads (zones of more than CPT x TPB
- * cells take the two-sweep form); lds/ldsBytes: the staging space (kLds).
- * hand (kLds only): the passes left the zone in lds, so the cell arrays and
- * column map are already in place and the links move down from behind the
- * passes' scratch; otherwise the zone state comes from global memory. */
+ * cells take the two-sweep form); lds/ldsBytes: the staging space (kLds) of
+ * the zone state k_zone left in global memory. */
 template <class IT, bool kLds, int TPB, int CPT>
 __device__ __forceinline__ void zone_finish_body(const ZoneArgs& a, const ZoneIn& in, int zid, uint64_t seed, int zi,
                                                  long long off, int tid, unsigned char* lds, long long ldsBytes,
-                                                 int* queue, const ZoneHandoff* hand = nullptr) {
+                                                 int* queue) {
     ZoneCtxT<IT> z;
     zone_init(z, in, a.rects[zi], zid, seed, nullptr);
     z.nxG = (IT*)a.nextG + off;
@@ -1137,12 +1129,7 @@ __device__ __forceinline__ void zone_finish_body(const ZoneArgs& a, const ZoneIn
     z.duG = a.duG + (size_t)zi * (size_t)a.duStride;
     z.rec = a.rec + off;
     const ZoneState<IT> st = zone_state_at<IT>(a.zstate + (size_t)zi * a.zsStride, z.C, z.zw);
-    if (kLds && hand) {
-        z.P = hand->P;
-        z.allOwned = hand->allOwned;
-    } else {
-        zone_attach_state(z, st);
-    }
+    zone_attach_state(z, st);
     if (kLds) {
         unsigned char* p = lds;
         ZCell<IT>* cell = (ZCell<IT>*)p; p += (size_t)z.C * sizeof(ZCell<IT>);
@@ -1153,32 +1140,16 @@ __device__ __forceinline__ void zone_finish_body(const ZoneArgs& a, const ZoneIn
         IT* links = (IT*)p;
         const long long room = (ldsBytes - (long long)(p - lds)) / (long long)sizeof(IT);
         const int nL = (int)(room < (long long)z.P ? (room > 0 ? room : 0) : z.P);
-        if (hand) {
-            /* the passes' links k < hand->nL, behind their scratch, move down in
-             * chunks no longer than the distance they move, so a chunk overwrites
-             * only links earlier chunks have copied; the rest come from the
-             * zone's global link region */
-            const IT* src = (const IT*)(lds + zone_fixed_bytes<IT>(z.C, z.zw, z.zp.useLocal));
-            const int gap = (int)(src - links);
-            const int nP = hand->nL < nL ? hand->nL : nL;
-            for (int c0 = 0; c0 < nP; c0 += gap) {
-                const int c1 = c0 + gap < nP ? c0 + gap : nP;
-                for (int k = c0 + tid; k < c1; k += TPB) links[k] = src[k];
-                __syncthreads();
-            }
-            for (int k = nP + tid; k < nL; k += TPB) links[k] = z.nxG[k];
-        } else {
-            /* the state and the first links to LDS */
-            for (int lc = tid; lc < z.C; lc += TPB) {
-                cell[lc] = st.cell[lc];
-                k0[lc] = st.k0[lc];
-            }
-            for (int c = tid; c < z.zw; c += TPB) {
-                colL[c] = st.colL[c];
-                colG[c] = st.colG[c];
-            }
-            for (int k = tid; k < nL; k += TPB) links[k] = z.nxG[k];
+        /* the state and the first links to LDS */
+        for (int lc = tid; lc < z.C; lc += TPB) {
+            cell[lc] = st.cell[lc];
+            k0[lc] = st.k0[lc];
         }
+        for (int c = tid; c < z.zw; c += TPB) {
+            colL[c] = st.colL[c];
+            colG[c] = st.colG[c];
+        }
+        for (int k = tid; k < nL; k += TPB) links[k] = z.nxG[k];
         z.cell = cell;
         z.k0 = k0;
         z.colL = colL;
@@ -1209,6 +1180,7 @@ __device__ __forceinline__ void zone_finish_body(const ZoneArgs& a, const ZoneIn
         for (int lc0 = 0; lc0 < z.C; lc0 += TPB / FIN_G) {
             const int lc = lc0 + gi;
             if (lc >= z.C) continue;
+            if (r == 0) mark_changed(z, lc, true);
             if (!fget(z, lc, ZF_CHG) || cnt_of(z, lc) == 0) {
                 if (r == 0) {
                     /* nothing to correct: the diagnostics' record, the side-buffer copy of a covered cell */
@@ -1284,7 +1256,7 @@ template <class IT, bool kEns = false>
 __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 waves per SIMD: four zones per CU */
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ ZoneShared sh;
-    __shared__ int queue[FUSED_TPB];
+    __shared__ unsigned queue[FUSED_TPB];
     const int zi = blockIdx.x;
     if (zi >= a.nZones) return;
     const int P = a.zsize[zi];
@@ -1333,32 +1305,33 @@ __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 
     if (threadIdx.x == 0 && sh.schedWait) atomicOr(a.err, 16);
     zone_sparse_pass_mw(z, wave, lane);
     if (threadIdx.x == 0 && sh.schedWait) atomicOr(a.err, 16);
+    __builtin_amdgcn_s_setprio(0);
+    /* the correction takes the zone over where the passes left it in LDS */
+    double* const dsq = a.wantStats ? zone_state_at<IT>(a.zstate + (size_t)zi * a.zsStride, z.C, z.zw).dsq : nullptr;
+    zone_finish_fused(z, wave, lane, dsq, queue);
     if (threadIdx.x == 0) {
         ZoneOut o;
         o.nHigh = sh.nHigh;
         o.nLow = sh.nLow;
         o.movedDense = sh.movedDense;
         o.movedSparse = sh.movedSparse;
-        o.stats4 = 0.0;
-        o.stats5 = 0.0;
+        o.stats4 = sh.stats4;
+        o.stats5 = sh.stats5;
         a.out[zi] = o;
     }
-    __builtin_amdgcn_s_setprio(0);
-    /* the correction takes the zone over where the passes left it in LDS */
-    const ZoneHandoff hand{z.P, z.allOwned, z.nL};
-    __syncthreads();
-    zone_finish_body<IT, true, FUSED_TPB, 3>(a, in, zid, seed, zi, off, (int)threadIdx.x, lds, a.ldsBytes, queue,
-                                            &hand);
 }
 
 /* velocities of the particles of cells several zones cover, from the side
- * buffer (their input runs in the pass-input binning) */
-__global__ void k_overlap_copyback(const int* __restrict__ cells, int ncells, const int* __restrict__ start,
-                                   const int* __restrict__ list, const double* __restrict__ vsx,
-                                   const double* __restrict__ vsy, double* __restrict__ vx, double* __restrict__ vy) {
+ * buffer (their input runs in the pass-input binning), for the cells their
+ * owner changed: the others' velocities are what they were */
+__global__ void k_overlap_copyback(const int* __restrict__ cells, int ncells, const unsigned char* __restrict__ chg,
+                                   const int* __restrict__ start, const int* __restrict__ list,
+                                   const double* __restrict__ vsx, const double* __restrict__ vsy,
+                                   double* __restrict__ vx, double* __restrict__ vy) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ncells) return;
     const int c = cells[t];
+    if (!chg[c]) return;
     for (int j = start[c]; j < start[c + 1]; ++j) {
         const int slot = list[j];
         vx[slot] = vsx[slot];
@@ -2002,6 +1975,7 @@ struct mpcd_gpu_sim {
     double* duG = nullptr;
     unsigned char* recG = nullptr; /* move records, 1 byte per particle slot of the zone regions */
     unsigned char* zstate = nullptr; /* per-zone pass state for the correction kernel */
+    unsigned char* chg = nullptr;    /* covered cells their owner changed in a pass */
     size_t zstateCap = 0;
     size_t duCap = 0;
     unsigned char* zscratch = nullptr;
@@ -2127,6 +2101,7 @@ struct mpcd_gpu_sim {
                             &duRX, &duRY, &duEX, &duEY, &pdrive, &cellTmp};
         for (double** c : cells) *c = dalloc<double>(Nc);
         mask = dalloc<int>(Nc);
+        chg = dalloc<unsigned char>(Nc);
         redN = dalloc<int>(Nc);
         redT = dalloc<double>(Nc);
         refN = dalloc<int>(Nc);
@@ -2213,7 +2188,7 @@ struct mpcd_gpu_sim {
         void* ptrs[] = {x, y, vx, vy, vx2, vy2, x2, y2, pid, pid2, cid, cidS, bin.cnt, bin.start, bin.cursor, bin.list, bin.key, bin.startB, bin.listB, bin.inc, bin.rnk, bin.keyB, bin.cntS, bin.dout, tileSum, next,
                         tmpg, zsize, zoff, owner[0], owner[1], cover[0], cover[1], overCells[0], overCells[1], stage,
                         refPx, refPy, refUx, refUy, pdriveRaw, redPx, redPy, redUx, redUy, duRX, duRY, duEX, duEY,
-                        pdrive, cellTmp, mask, part, scal, err, wallPart, rects[0], rects[1], zout, zscratch, duG, recG, zstate,
+                        pdrive, cellTmp, mask, part, scal, err, wallPart, rects[0], rects[1], zout, zscratch, duG, recG, zstate, chg,
                         redN, redT, featBuf, tgtBuf, surFlag, diagDev, outN, outF, surDev, rowAcc, refN, refT, snapN, snapF};
         for (void* q : ptrs)
             if (q) (void)hipFree(q);
@@ -2452,7 +2427,7 @@ struct mpcd_gpu_sim {
     void zone_pass(uint64_t seedBase, const ZoneRect* rectsDev, int nZ, int maxC, int maxW, const int* ownerDev,
                    const unsigned char* coverDev, const int* overDev, int nOverCells, int single,
                    const double* inPx = nullptr, const double* inPy = nullptr, bool record = false,
-                   const unsigned char* zmask = nullptr) {
+                   const unsigned char* zmask = nullptr, bool stats = true) {
         hipLaunchKernelGGL(k_zone_sizes, dim3(nZ + 1), dim3(64), 0, stream, rectsDev, nZ, bin.start, p.Ny, zsize);
         const int nt = (nZ + 1 + SCAN_TILE - 1) / SCAN_TILE;
         hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(TPB), 0, stream, zsize, nZ + 1, zoff, tileSum,
@@ -2478,6 +2453,7 @@ struct mpcd_gpu_sim {
         a.in.vy = vy;
         a.in.vsx = vx2; /* the side buffer: free during a pass */
         a.in.vsy = vy2;
+        a.in.gchg = single || !coverDev ? nullptr : chg;
         a.in.inPx = inPx;
         a.in.inPy = inPy;
         a.in.dgCell = zdCell;
@@ -2515,6 +2491,7 @@ struct mpcd_gpu_sim {
         a.zstate = zstate;
         a.duStride = 2 * maxC;
         a.out = zout;
+        a.wantStats = stats;
         a.err = err;
         pbeg(MPCD_PROF_ZONE_KERNEL);
         const size_t fix16 = zone_fixed_bytes<uint16_t>(maxC, maxW, zp.useLocal);
@@ -2576,15 +2553,15 @@ struct mpcd_gpu_sim {
         check_launch();
         if (!single && coverDev && nOverCells > 0) {
             hipLaunchKernelGGL(k_overlap_copyback, dim3(nblk(nOverCells)), dim3(TPB), 0, stream, overDev, nOverCells,
-                               bin.start, bin.list, vx2, vy2, vx, vy);
+                               chg, bin.start, bin.list, vx2, vy2, vx, vy);
             check_launch();
         }
     }
 
     void layout_pass(int L, uint64_t seedBase, const double* inPx = nullptr, const double* inPy = nullptr,
-                     bool record = false) {
+                     bool record = false, bool stats = true) {
         zone_pass(seedBase, rects[L], nz[L], maxCells[L], maxCols[L], owner[L], cover[L], overCells[L], nOver[L], 0,
-                  inPx, inPy, record);
+                  inPx, inPy, record, nullptr, stats);
     }
 
     void pass_metrics(int nZ, mpcd_zone_pass_metrics* m) {
@@ -2917,7 +2894,7 @@ struct mpcd_gpu_sim {
         /* the base pass's input is the state the reference fields were
          * summed over (same runs, same order): the correction takes its
          * input sums from them */
-        layout_pass(0, zs, refPx, refPy, true);
+        layout_pass(0, zs, refPx, refPy, true, sm != nullptr);
         pend(MPCD_PROF_ZONE_PASS);
         if (sm) pass_metrics(nz[0], &sm->base);
         /* the passes move a few particles: the binning is updated */
@@ -2928,7 +2905,7 @@ struct mpcd_gpu_sim {
         if (wantDiag) occupancy(bin.cnt, DIAG_OCC_BASE); /* the counts after the base pass */
         if (stages && stages[2]) get_state(stages[2], stages[3]);
         pbeg(MPCD_PROF_ZONE_PASS);
-        layout_pass(1, zs + 4099ULL, nullptr, nullptr, true);
+        layout_pass(1, zs + 4099ULL, nullptr, nullptr, true, sm != nullptr);
         pend(MPCD_PROF_ZONE_PASS);
         if (sm) pass_metrics(nz[1], &sm->shifted);
         pbeg(MPCD_PROF_BIN);

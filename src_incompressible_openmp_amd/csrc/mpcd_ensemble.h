@@ -493,6 +493,7 @@ struct mpcd_gpu_ensemble {
     int* zoneOff[2] = {nullptr, nullptr};
     int* owner[2] = {nullptr, nullptr};
     unsigned char* cover[2] = {nullptr, nullptr};
+    unsigned char* chg = nullptr; /* covered cells their owner changed in a pass */
     int* overCells[2] = {nullptr, nullptr};
     int nOver[2] = {0, 0};
     ZoneIn* ensIn[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}}; /* [parity][layout] */
@@ -662,6 +663,7 @@ struct mpcd_gpu_ensemble {
             HIP_OK(hipMemcpy(mask, hm.data(), hm.size() * sizeof(int), hipMemcpyHostToDevice));
             HIP_OK(hipMemcpy(reps, hreps.data(), (size_t)R * sizeof(EnsRep), hipMemcpyHostToDevice));
         }
+        chg = dalloc<unsigned char>((size_t)C);
         /* zones of both layouts: rects, replica of each zone, owner and cover
          * maps at each replica's cells, and each replica's zone inputs */
         for (int L = 0; L < 2; ++L) {
@@ -729,6 +731,7 @@ struct mpcd_gpu_ensemble {
                     q.vy = par ? vy2 : vy;
                     q.vsx = par ? vx : vx2; /* the side buffer: the other set, free during a pass */
                     q.vsy = par ? vy : vy2;
+                    q.gchg = q.gcover ? chg + e.coff : nullptr;
                 }
                 ensIn[par][L] = dalloc<ZoneIn>((size_t)R);
                 HIP_OK(hipMemcpy(ensIn[par][L], zi.data(), zi.size() * sizeof(ZoneIn), hipMemcpyHostToDevice));
@@ -756,7 +759,7 @@ struct mpcd_gpu_ensemble {
         void* ptrs[] = {reps, poff, coff, boff, x, y, vx, vy, x2, y2, vx2, vy2, pid, pid2, cidS, cidU, cnt, start,
                         cursor, list, tileSum, key, startB, listB, keyB, dout, inc, rnk, refPx, refPy, refUx, refUy, pdriveRaw, redPx, redPy, redUx, redUy,
                         duRX, duRY, duEX, duEY, pdrive, mask, part, scal, rects[0], rects[1], zrep[0], zrep[1],
-                        zoneOff[0], zoneOff[1], owner[0], owner[1], cover[0], cover[1], overCells[0], overCells[1],
+                        zoneOff[0], zoneOff[1], owner[0], owner[1], cover[0], cover[1], chg, overCells[0], overCells[1],
                         ensIn[0][0], ensIn[0][1], ensIn[1][0], ensIn[1][1], zsize, zoff, next, tmpg, recG, zstate,
                         duG, zout, stepDev, shift, zseed, seeds, err, flowPart, flowAcc, stage, cntS};
         for (void* q : ptrs)
@@ -851,7 +854,7 @@ struct mpcd_gpu_ensemble {
         check_launch();
         if (nOver[L] > 0) {
             hipLaunchKernelGGL(k_overlap_copyback, dim3(nblk(nOver[L])), dim3(TPB), 0, stream, overCells[L], nOver[L],
-                               start, list, vx2, vy2, vx, vy);
+                               chg, start, list, vx2, vy2, vx, vy);
             check_launch();
         }
     }

@@ -199,6 +199,9 @@ struct ZoneIn {
     const unsigned char* gcover; /* per cell: several zones cover it, or nullptr */
     double *x, *y, *vx, *vy;
     double *vsx, *vsy;  /* side buffer for covered cells */
+    /* per cell several zones cover: its owner changed it, so the side buffer
+     * holds its particles' velocities (nullptr with gcover) */
+    unsigned char* gchg = nullptr;
     /* per-cell velocity sums of the pass input (each cell's run summed in
      * order from zero), or nullptr: the correction sums the runs itself */
     const double *inPx = nullptr, *inPy = nullptr;
@@ -229,7 +232,7 @@ struct ZoneShared {
     int mwNext;            /* and the next list position a wavefront takes */
     int schedWait;         /* nonzero: a wait of the dependency-driven dense phase hit its bound */
     int nHigh, nLow, movedDense, movedSparse;
-    int mixedW[3];         /* zone_setup_mw: wavefront 1..3 saw a cell not plainly owned */
+    int mixed;             /* zone_setup_mw: a cell is not plainly owned */
     double stats4, stats5;
 };
 
@@ -262,6 +265,7 @@ struct ZoneCtxT {
     const int *gcnt, *gstart, *glist;
     const unsigned long long* gkey;
     double *x, *y, *vx, *vy, *vsx, *vsy;
+    unsigned char* gchg; /* changed covered cells, or nullptr */
     const double *inPx, *inPy; /* input run sums per global cell, or nullptr */
     int *dcid, *dout, *dinc, *drnk; /* cell-change record, or nullptr */
     int cellOff;    /* added to the recorded new cells */
@@ -2283,27 +2287,27 @@ ZHD void zone_setup(Z& z, const ZoneIn& in, int lane, int nl) {
     }
 }
 
-/* zone_setup on the four wavefronts of a 256-thread workgroup: wavefront 0
- * takes the counts, runs and column starts (its prefix sum over the cells),
- * wavefronts 1..3 the flags, the column map's global starts and the halo
- * ring; each of them records in sh->mixedW whether it saw a cell that is not
- * plainly owned.  After a workgroup barrier, zone_setup_all_owned gives the
- * zone's allOwned. */
+/* zone_setup on the four wavefronts of a 256-thread workgroup, with two
+ * rounds of global loads: a column's cells are one run of the binning, so
+ * wavefront 0 takes the columns' starts and lengths (their prefix sum gives
+ * the local indices) while the others take the ring; then every cell's run
+ * follows from its start and its column's.  The barrier in between and the
+ * one the caller takes after it are workgroup barriers; zone_setup_all_owned
+ * gives the zone's allOwned after the second. */
 template <class Z>
 ZHD void zone_setup_mw(Z& z, const ZoneIn& in, int wave, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef typename Z::idx_t IT;
     if (wave == 0) {
         int base = 0;
-        for (int b0 = 0; b0 < z.C; b0 += 64) {
-            const int lc = b0 + lane;
-            const int m = lc < z.C ? z.gcnt[lc_gc(z, lc)] : 0;
-            const int incl = wave_shfl_up_add(m, lane);
-            if (lc < z.C) {
-                const int k0 = base + incl - m;
-                cnt_set(z, lc, m);
-                z.k0[lc] = (typename Z::idx_t)k0;
-                head_set(z, lc, m > 0 ? k0 : -1);
-                tail_set(z, lc, m > 0 ? k0 + m - 1 : -1);
-                if (lc % z.zh == 0) z.colL[lc / z.zh] = k0;
+        for (int b0 = 0; b0 < z.zw; b0 += 64) {
+            const int col = b0 + lane;
+            const int g0 = z.ys + z.g.Ny * (z.xs + (col < z.zw ? col : 0));
+            const int s0 = z.gstart[g0], len = col < z.zw ? z.gstart[g0 + z.zh] - s0 : 0;
+            const int incl = wave_shfl_up_add(len, lane);
+            if (col < z.zw) {
+                z.colL[col] = base + incl - len;
+                z.colG[col] = s0;
             }
             base += wave_bcast(incl, 63);
         }
@@ -2315,26 +2319,33 @@ ZHD void zone_setup_mw(Z& z, const ZoneIn& in, int wave, int lane) {
             z.sh->movedSparse = 0;
             z.sh->stats4 = 0.0;
             z.sh->stats5 = 0.0;
+            z.sh->mixed = 0;
         }
-        return;
+    } else {
+        const int nh = halo_size(z);
+        for (int h = (wave - 1) * 64 + lane; h < nh; h += 192) setup_halo(z, h);
     }
-    const int t = (wave - 1) * 64 + lane;
+    __syncthreads();
     bool mixed = false;
-    for (int lc = t; lc < z.C; lc += 192) {
-        const int gc = lc_gc(z, lc);
+    for (int lc = wave * 64 + lane; lc < z.C; lc += 256) {
+        const int col = lc_col(z, lc), gc = lc_gc(z, lc);
+        const int m = z.gcnt[gc], k0 = z.colL[col] + (z.gstart[gc] - z.colG[col]);
         const unsigned short f = setup_flags(z, in, gc);
-        if ((f & (ZF_OWN | ZF_COVER)) != ZF_OWN) mixed = true;
-        z.cell[lc].fl = (typename Z::idx_t)f;
-        if (lc % z.zh == 0) z.colG[lc / z.zh] = z.gstart[gc];
+        mixed = mixed || (f & (ZF_OWN | ZF_COVER)) != ZF_OWN;
+        ZCell<IT> c;
+        c.cnt = (IT)m;
+        c.head = (IT)(m > 0 ? k0 : -1);
+        c.tail = (IT)(m > 0 ? k0 + m - 1 : -1);
+        c.fl = (IT)f;
+        z.cell[lc] = c;
+        z.k0[lc] = (IT)k0;
     }
-    const int nh = halo_size(z);
-    for (int h = t; h < nh; h += 192) setup_halo(z, h);
-    const bool anyMixed = wave_ballot(mixed) != 0ull;
-    if (lane == 0) z.sh->mixedW[wave - 1] = anyMixed ? 1 : 0;
+    if (wave_ballot(mixed) != 0ull && lane == 0) z.sh->mixed = 1;
+#endif
 }
 template <class Z>
 ZHD int zone_setup_all_owned(const Z& z) {
-    return (z.sh->mixedW[0] | z.sh->mixedW[1] | z.sh->mixedW[2]) ? 0 : 1;
+    return z.sh->mixed ? 0 : 1;
 }
 
 /* sum over the slots glist[s0 .. s0+n) in order, loads issued 8 at a time */
@@ -2426,12 +2437,20 @@ ZHD void zone_correct_sums(Z& z, int lc) {
     if (corr) fset(z, lc, ZF_CORR);
 }
 
+/* records whether the side buffer holds the velocities of cell lc's input
+ * particles (a cell this zone owns and others cover) */
+template <class Z>
+ZHD void mark_changed(Z& z, int lc, bool chg) {
+    if (z.gchg && fget(z, lc, ZF_OWN) && fget(z, lc, ZF_COVER)) z.gchg[lc_gc(z, lc)] = chg ? 1 : 0;
+}
+
 /* Second half, one lane per cell: write the velocities of the owned
  * particles of a changed cell; for an unchanged cell that several zones
  * cover, pass its owned particles' input velocities through to the side
  * buffer.  Returns the cell's |du|^2 (0 for an unchanged cell). */
 template <class Z>
 ZHD double zone_correct_write(Z& z, int lc) {
+    mark_changed(z, lc, true);
     if (fget(z, lc, ZF_CHG)) {
         if (cnt_of(z, lc) == 0) return 0.0;
         const bool corr = fget(z, lc, ZF_CORR);
@@ -2613,6 +2632,7 @@ ZHD void zone_init(ZoneCtxT<IT>& z, const ZoneIn& in, ZoneRect r, int zid, uint6
     z.vy = in.vy;
     z.vsx = in.vsx;
     z.vsy = in.vsy;
+    z.gchg = in.gchg;
     z.sh = sh;
 }
 
@@ -2906,12 +2926,267 @@ __device__ __forceinline__ double fin_cell_group(Z& z, int lc, int r, int lane, 
     }
     return dux * dux + duy * duy;
 }
+/* the value of lane A of one's quad */
+template <int A>
+__device__ __forceinline__ double quad_bcast_d(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, A * 0x55, 0xf, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), A * 0x55, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+/* lane A of each quad adds its entries to the running sums, which the quad
+ * then holds (absent entries are +0: a running sum from +0 is never -0) */
+template <int A>
+__device__ __forceinline__ void fin_add(double& px, double& py, const double* ax, const double* ay, int r) {
+    if (r == A)
+        for (int u = 0; u < FIN_L; ++u) {
+            px += ax[u];
+            py += ay[u];
+        }
+    px = quad_bcast_d<A>(px);
+    py = quad_bcast_d<A>(py);
+}
+
+/* The moved particles a wavefront has met, local index << 16 | final cell,
+ * placed 64 at a time. */
+struct FinQueue {
+    unsigned* q;
+    int n;
+};
+template <class Z>
+__device__ __forceinline__ void fin_flush(Z& z, FinQueue& fq, int lane) {
+    ZWSYNC();
+    if (lane < fq.n) {
+        const unsigned e = fq.q[lane];
+        const int k = (int)(e >> 16);
+        uint32_t pid;
+        const int slot = slot_pid_in(z, k, col_of(z, k), pid);
+        place_moved(z, (int)(e & 0xffffu), slot, pid, z.rec[k]);
+    }
+    ZWSYNC();
+    fq.n = 0;
+}
+/* entries u of kk with bit u of mv set, of every lane */
+template <class Z>
+__device__ __forceinline__ void fin_push(Z& z, FinQueue& fq, unsigned mv, const int* kk, int lc, int lane) {
+    int next = 0;
+    while (wave_ballot(mv != 0u) != 0ull && next < FIN_L) {
+        bool full = false;
+#pragma unroll
+        for (int u = 0; u < FIN_L; ++u) {
+            const bool mine = (mv >> u) & 1u;
+            const unsigned long long msk = wave_ballot(mine);
+            const int add = wave_popc(msk);
+            if (u < next || full || add == 0) continue;
+            if (fq.n + add > 64) {
+                full = true;
+                next = u;
+                continue;
+            }
+            if (mine) fq.q[fq.n + wave_popc(msk & lanes_below(lane))] = ((unsigned)kk[u] << 16) | (unsigned)lc;
+            fq.n += add;
+        }
+        if (!full) break;
+        fin_flush(z, fq, lane);
+    }
+}
+
+/* slots of a group's entries kk: the cell's own run's entries lie in its
+ * column, the others' columns by a search all entries take in step.  Returns
+ * entry u's ZF_OWN in bit u, its ZF_COVER in bit 8 + u. */
+template <class Z>
+__device__ __forceinline__ unsigned fin_slots(const Z& z, int lc, int kb, int ke, unsigned ownLc, const int* kk, int* sl) {
+    const int own = lc_col(z, lc);
+    int lo[FIN_L];
+    bool far = false;
+    for (int u = 0; u < FIN_L; ++u) {
+        lo[u] = own;
+        far = far || (kk[u] >= 0 && (kk[u] < kb || kk[u] >= ke));
+    }
+    if (wave_ballot(far) != 0ull) {
+        int hi[FIN_L];
+        for (int u = 0; u < FIN_L; ++u) {
+            const bool f = kk[u] >= 0 && (kk[u] < kb || kk[u] >= ke);
+            lo[u] = f ? 0 : own;
+            hi[u] = f ? z.zw - 1 : own;
+        }
+        for (int s = z.zw - 1; s > 0; s >>= 1)
+            for (int u = 0; u < FIN_L; ++u) {
+                const int mid = (lo[u] + hi[u] + 1) >> 1;
+                const bool up = z.colL[mid] <= kk[u];
+                const bool open = lo[u] < hi[u];
+                lo[u] = (open & up) ? mid : lo[u];
+                hi[u] = (open & !up) ? mid - 1 : hi[u];
+            }
+    }
+    for (int u = 0; u < FIN_L; ++u) sl[u] = kk[u] >= 0 ? z.glist[z.colG[lo[u]] + (kk[u] - z.colL[lo[u]])] : -1;
+    unsigned ow = 0u;
+    for (int u = 0; u < FIN_L; ++u) {
+        unsigned b = ownLc;
+        if (!z.allOwned && kk[u] >= 0 && (kk[u] < kb || kk[u] >= ke)) b = own_bits(z, kk[u], lo[u]);
+        ow |= ((b & ZF_OWN) ? 1u << u : 0u) | ((b & ZF_COVER) ? 256u << u : 0u);
+    }
+    return ow;
+}
+
+/* a chunk of a group's list: its moved particles to the queue (what the links
+ * hold has moved, but for lists whose links were all written), its slots and
+ * velocities loaded; returns the ownership bits */
+template <class Z>
+__device__ __forceinline__ unsigned fin_load(Z& z, FinWalk& w, int lc, int m, int kb, int ke, unsigned f, int left, int c0,
+                                             int r, int lane, FinQueue* fq, int* sl, double* ax, double* ay) {
+    int kk[FIN_L];
+    fin_group_entries(z, w, m, c0, r, kk);
+    const unsigned ow = fin_slots(z, lc, kb, ke, f, kk, sl);
+    if (fq) {
+        unsigned mv = 0u;
+        for (int u = 0; u < FIN_L; ++u) {
+            bool v = kk[u] >= 0 && c0 + FIN_L * r + u >= left && ((ow >> u) & 1u);
+            if (v && (f & ZF_MAT)) v = z.rec[kk[u]] != ZM_NONE;
+            mv |= v ? 1u << u : 0u;
+        }
+        fin_push(z, *fq, mv, kk, lc, lane);
+    }
+    for (int u = 0; u < FIN_L; ++u) {
+        ax[u] = sl[u] >= 0 ? z.vx[sl[u]] : 0.0;
+        ay[u] = sl[u] >= 0 ? z.vy[sl[u]] : 0.0;
+    }
+    return ow;
+}
+template <class Z>
+__device__ __forceinline__ void fin_store(Z& z, const int* sl, unsigned ow, bool corr, const double* ax, const double* ay,
+                                          double dux, double duy) {
+    for (int u = 0; u < FIN_L; ++u)
+        if (sl[u] >= 0 && ((ow >> u) & 1u)) {
+            const bool cov = (ow >> (8 + u)) & 1u;
+            double* const X = cov ? z.vsx : z.vx;
+            double* const Y = cov ? z.vsy : z.vy;
+            X[sl[u]] = corr ? ax[u] + dux : ax[u];
+            Y[sl[u]] = corr ? ay[u] + duy : ay[u];
+        }
+}
+
+/* Phase 2 for cell lc of the fused kernel (fin_cell_group's sums and writes);
+ * act: the group has a cell (the whole wavefront calls it).  Its moved
+ * particles go to the queue. */
+template <class Z>
+__device__ __forceinline__ double fin_cell_fused(Z& z, int lc, bool act, int r, int lane, double pbx, double pby,
+                                                 FinQueue& fq) {
+    constexpr int CH = FIN_G * FIN_L;
+    const ZCell<typename Z::idx_t> S = z.cell[lc];
+    const unsigned f = (unsigned)S.fl;
+    const int m = act ? (int)S.cnt : 0;
+    const int kb = (int)z.k0[lc], ke = run_end(z, lc) + 1;
+    FinWalk w;
+    w.h = iget(S.head);
+    w.left = (f & ZF_MAT) || w.h < kb || w.h >= ke ? 0 : imin(m, ke - w.h);
+    w.at = w.left;
+    w.kw = w.left > 0 ? (w.left < m ? nx_get(z, w.h + w.left - 1) : -1) : w.h;
+    const FinWalk w0 = w;
+    int sl[FIN_L];
+    unsigned ow = 0u;
+    double ax[FIN_L], ay[FIN_L];
+    double px = 0.0, py = 0.0;
+    const bool again = wave_ballot(m > CH) != 0ull;
+    for (int c0 = 0; wave_ballot(c0 < m) != 0ull; c0 += CH) {
+        ow = fin_load(z, w, lc, m, kb, ke, f, w0.left, c0, r, lane, &fq, sl, ax, ay);
+        fin_add<0>(px, py, ax, ay, r);
+        fin_add<1>(px, py, ax, ay, r);
+        fin_add<2>(px, py, ax, ay, r);
+        fin_add<3>(px, py, ax, ay, r);
+    }
+    if (z.dgCell && r == 0 && act) diag_cell(z, lc, pbx - px, pby - py, px, py);
+    const double dux = act ? (pbx - px) / (double)m : 0.0, duy = act ? (pby - py) / (double)m : 0.0;
+    const bool corr = z.zp.corrEnabled != 0 && !(f & ZF_SKIP) && !((f & ZF_RECV) && !(f & ZF_BB)) && (dux != 0.0 || duy != 0.0);
+    if (!again) {
+        fin_store(z, sl, ow, corr, ax, ay, dux, duy);
+    } else {
+        /* a list past one chunk in this wavefront: loaded again for the writes */
+        w = w0;
+        for (int c0 = 0; wave_ballot(c0 < m) != 0ull; c0 += CH) {
+            ow = fin_load(z, w, lc, m, kb, ke, f, w0.left, c0, r, lane, nullptr, sl, ax, ay);
+            fin_store(z, sl, ow, corr, ax, ay, dux, duy);
+        }
+    }
+    return dux * dux + duy * duy;
+}
+
+/* The correction of a zone on the 256 threads that ran its passes, its state
+ * still in LDS: the changed, occupied cells are listed first, so a group of
+ * four lanes always has one (a few hundred of 625 in the base pass, a handful
+ * in the shifted one); lists are mostly what is left of an input run, whose
+ * entries need no walk; the sums pass between the lanes of a quad in
+ * registers; a moved particle is met in its final cell's links and placed
+ * from there, with no pass over all particles' records.  dsq: |du|^2 per cell
+ * for the ordered stats, or nullptr (no metrics asked). */
+template <class Z>
+__device__ __forceinline__ void zone_finish_fused(Z& z, int wave, int lane, double* dsq, unsigned* queue) {
+    constexpr int NT = 64 * ZONE_WAVES;
+    const int tid = wave * 64 + lane;
+    unsigned long long* const chunkMask = reinterpret_cast<unsigned long long*>(z.scr->cand);
+    for (int ch = wave; ch * 64 < z.C; ch += ZONE_WAVES) {
+        const int lc = ch * 64 + lane;
+        bool f = false;
+        if (lc < z.C) {
+            const bool chg = fget(z, lc, ZF_CHG);
+            f = chg && cnt_of(z, lc) > 0;
+            mark_changed(z, lc, chg);
+            if (dsq) dsq[lc] = 0.0;
+            if (z.dgCell && !chg && cnt_of(z, lc) > 0 && !fget(z, lc, ZF_OUT)) diag_cell_unchanged(z, lc);
+        }
+        const unsigned long long msk = wave_ballot(f);
+        if (lane == 0) chunkMask[ch] = msk;
+    }
+    __syncthreads();
+    const int m = zone_compact_mw(z, chunkMask, wave, lane);
+    __syncthreads();
+    const int r = tid % FIN_G, gi = tid / FIN_G;
+    /* input-run sums of the changed cells, before any velocity is written
+     * (the base pass has them from the reference fields) */
+    if (!z.inPx) {
+        for (int j = gi; j < m; j += NT / FIN_G) {
+            const int lc = (int)z.dl[j];
+            double bx, by;
+            fin_input_sum_group(z, lc, r, lane, bx, by);
+            if (r == 0) {
+                z.duG[2 * lc] = bx;
+                z.duG[2 * lc + 1] = by;
+            }
+        }
+        __threadfence_block();
+        __syncthreads();
+    }
+    FinQueue fq{queue + 64 * wave, 0};
+    for (int j0 = 0; j0 < m; j0 += NT / FIN_G) {
+        const bool act = j0 + gi < m;
+        const int lc = (int)z.dl[act ? j0 + gi : j0];
+        const int gc = lc_gc(z, lc);
+        const double bx = z.inPx ? z.inPx[gc] : z.duG[2 * lc], by = z.inPx ? z.inPy[gc] : z.duG[2 * lc + 1];
+        const double d = fin_cell_fused(z, lc, act, r, lane, bx, by, fq);
+        if (dsq && act && r == 0) dsq[lc] = d;
+    }
+    fin_flush(z, fq, lane);
+    if (dsq) {
+        __threadfence_block();
+        __syncthreads();
+        if (wave == 0) {
+            double rms, mx;
+            zone_correct_stats(z, dsq, lane, 64, rms, mx);
+            if (lane == 0) {
+                z.sh->stats4 = rms;
+                z.sh->stats5 = mx;
+            }
+        }
+    }
+}
 #else
 /* (the host passes of the compilers see a declaration only) */
 template <class Z>
 ZHD void fin_input_sum_group(const Z&, int, int, int, double&, double&) {}
 template <class Z>
 ZHD double fin_cell_group(Z&, int, int, int, double, double) { return 0.0; }
+template <class Z>
+ZHD void zone_finish_fused(Z&, int, int, double*, unsigned*) {}
 #endif
 
 /* phase 3, all threads of the zone: the new positions of the moved
