@@ -3068,8 +3068,11 @@ __device__ __forceinline__ void fin_store(Z& z, const int* sl, unsigned ow, bool
 
 /* Phase 2 for cell lc of the fused kernel (fin_cell_group's sums and writes);
  * act: the group has a cell (the whole wavefront calls it).  Its moved
- * particles go to the queue. */
-template <class Z>
+ * particles go to the queue.  kLong: lists of more than one chunk, walked
+ * twice; the others stay in registers (a form of its own: with both in one,
+ * the registers do not hold it, and the spills cost a quarter of the kernel's
+ * time at 2048 x 1024 x 20). */
+template <bool kLong, class Z>
 __device__ __forceinline__ double fin_cell_fused(Z& z, int lc, bool act, int r, int lane, double pbx, double pby,
                                                  FinQueue& fq) {
     constexpr int CH = FIN_G * FIN_L;
@@ -3087,8 +3090,7 @@ __device__ __forceinline__ double fin_cell_fused(Z& z, int lc, bool act, int r, 
     unsigned ow = 0u;
     double ax[FIN_L], ay[FIN_L];
     double px = 0.0, py = 0.0;
-    const bool again = wave_ballot(m > CH) != 0ull;
-    for (int c0 = 0; wave_ballot(c0 < m) != 0ull; c0 += CH) {
+    for (int c0 = 0; c0 == 0 || (kLong && wave_ballot(c0 < m) != 0ull); c0 += CH) {
         ow = fin_load(z, w, lc, m, kb, ke, f, w0.left, c0, r, lane, &fq, sl, ax, ay);
         fin_add<0>(px, py, ax, ay, r);
         fin_add<1>(px, py, ax, ay, r);
@@ -3098,10 +3100,10 @@ __device__ __forceinline__ double fin_cell_fused(Z& z, int lc, bool act, int r, 
     if (z.dgCell && r == 0 && act) diag_cell(z, lc, pbx - px, pby - py, px, py);
     const double dux = act ? (pbx - px) / (double)m : 0.0, duy = act ? (pby - py) / (double)m : 0.0;
     const bool corr = z.zp.corrEnabled != 0 && !(f & ZF_SKIP) && !((f & ZF_RECV) && !(f & ZF_BB)) && (dux != 0.0 || duy != 0.0);
-    if (!again) {
+    if (!kLong) {
         fin_store(z, sl, ow, corr, ax, ay, dux, duy);
     } else {
-        /* a list past one chunk in this wavefront: loaded again for the writes */
+        /* loaded again for the writes */
         w = w0;
         for (int c0 = 0; wave_ballot(c0 < m) != 0ull; c0 += CH) {
             ow = fin_load(z, w, lc, m, kb, ke, f, w0.left, c0, r, lane, nullptr, sl, ax, ay);
@@ -3157,14 +3159,26 @@ __device__ __forceinline__ void zone_finish_fused(Z& z, int wave, int lane, doub
         __syncthreads();
     }
     FinQueue fq{queue + 64 * wave, 0};
+    bool anyLong = false;
     for (int j0 = 0; j0 < m; j0 += NT / FIN_G) {
-        const bool act = j0 + gi < m;
-        const int lc = (int)z.dl[act ? j0 + gi : j0];
+        const int lc = (int)z.dl[j0 + gi < m ? j0 + gi : j0];
+        const bool act = j0 + gi < m && cnt_of(z, lc) <= FIN_G * FIN_L;
+        anyLong = anyLong || cnt_of(z, lc) > FIN_G * FIN_L;
         const int gc = lc_gc(z, lc);
         const double bx = z.inPx ? z.inPx[gc] : z.duG[2 * lc], by = z.inPx ? z.inPy[gc] : z.duG[2 * lc + 1];
-        const double d = fin_cell_fused(z, lc, act, r, lane, bx, by, fq);
+        const double d = fin_cell_fused<false>(z, lc, act, r, lane, bx, by, fq);
         if (dsq && act && r == 0) dsq[lc] = d;
     }
+    if (wave_ballot(anyLong) != 0ull)
+        for (int j0 = 0; j0 < m; j0 += NT / FIN_G) {
+            const int lc = (int)z.dl[j0 + gi < m ? j0 + gi : j0];
+            const bool act = j0 + gi < m && cnt_of(z, lc) > FIN_G * FIN_L;
+            if (wave_ballot(act) == 0ull) continue;
+            const int gc = lc_gc(z, lc);
+            const double bx = z.inPx ? z.inPx[gc] : z.duG[2 * lc], by = z.inPx ? z.inPy[gc] : z.duG[2 * lc + 1];
+            const double d = fin_cell_fused<true>(z, lc, act, r, lane, bx, by, fq);
+            if (dsq && act && r == 0) dsq[lc] = d;
+        }
     fin_flush(z, fq, lane);
     if (dsq) {
         __threadfence_block();
