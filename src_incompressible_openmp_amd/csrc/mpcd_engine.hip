@@ -1251,6 +1251,35 @@ __global__ void __launch_bounds__(FINISH_TPB) k_zone_finish(ZoneArgs a) {
  * phases, then the correction, which takes the zone over in LDS where the
  * passes left it.  A zone's correction starts as soon as its own passes
  * end, beside the passes of slower zones. */
+/* a value every lane holds alike, in scalar registers */
+template <class T>
+__device__ __forceinline__ T uniform_value(T v) {
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "one or two words");
+    unsigned w[sizeof(T) / 4];
+    __builtin_memcpy(w, &v, sizeof(T));
+    for (unsigned k = 0; k < sizeof(T) / 4; ++k) w[k] = (unsigned)__builtin_amdgcn_readfirstlane((int)w[k]);
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+template <class... T>
+__device__ __forceinline__ void make_uniform(T&... v) {
+    ((v = uniform_value(v)), ...);
+}
+/* An ensemble zone's inputs come from its replica's table: the compiler sees
+ * memory, not kernel arguments, and would hold every pointer and threshold in
+ * vector registers (416 bytes of spills per lane). */
+template <class Z>
+__device__ __forceinline__ void zone_uniform(Z& z) {
+    make_uniform(z.g.Nx, z.g.Ny, z.g.Nc, z.g.n, z.g.perx, z.g.pery, z.g.Lx, z.g.Ly, z.g.a0, z.g.dxc, z.g.dyc);
+    make_uniform(z.zp.highThr, z.zp.lowThrBulk, z.zp.lowFrac, z.zp.highFrac, z.zp.gamma, z.zp.fluidFracGain,
+                 z.zp.lowThrFloor, z.zp.highThrFloor, z.zp.lowLoc1, z.zp.highLoc1, z.zp.useLocal, z.zp.maxPasses,
+                 z.zp.corrEnabled, z.zp.dedupe, z.zp.quadBins, z.zp.binLo, z.zp.binHi);
+    make_uniform(z.xs, z.xe, z.ys, z.ye, z.zw, z.zh, z.C, z.zhM, z.zid, z.seed, z.gcnt, z.gstart, z.glist, z.gkey, z.x,
+                 z.y, z.vx, z.vy, z.vsx, z.vsy, z.gchg, z.inPx, z.inPy, z.dcid, z.dout, z.dinc, z.drnk, z.cellOff, z.dgCell,
+                 z.dgCnt);
+}
+
 constexpr int FUSED_TPB = 256;
 template <class IT, bool kEns = false>
 __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 waves per SIMD: four zones per CU */
@@ -1288,6 +1317,7 @@ __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 
     }
     const ZoneIn& in = *inp;
     zone_init(z, in, a.rects[zi], zid, seed, &sh);
+    if constexpr (kEns) zone_uniform(z);
     z.nxG = (IT*)a.nextG + off;
     z.tmpG = (IT*)a.tmpG + off;
     z.duG = a.duG + (size_t)zi * (size_t)a.duStride;
