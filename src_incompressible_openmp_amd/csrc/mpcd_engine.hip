@@ -300,6 +300,59 @@ __global__ void __launch_bounds__(TPB) k_scan_add_prefix(int* __restrict__ out, 
     if (i < m) out[i] += s[0];
 }
 
+/* The whole scan by one block, for up to ONE_TILES x 4096 entries: every load
+ * is issued before the first sum, so it takes about what one of the two
+ * kernels above does, whose launches a small grid's step otherwise pays four
+ * times (4.4 us each; 9.0 -> 5 us per scan at 2,501 and 32,769 entries). */
+constexpr int ONE_TPB = 1024, ONE_TILES = 9;
+__global__ void __launch_bounds__(ONE_TPB) k_scan_one(const int* __restrict__ in, int m, int* __restrict__ out,
+                                                      const int* __restrict__ in2, int* __restrict__ zero,
+                                                      const int* __restrict__ sub) {
+    __shared__ int ws[ONE_TILES][ONE_TPB / 64];
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int v[ONE_TILES][4], incl[ONE_TILES];
+#pragma unroll
+    for (int t = 0; t < ONE_TILES; ++t) {
+        const int b = t * 4 * ONE_TPB + 4 * tid;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            v[t][k] = b + k < m ? in[b + k] + (in2 ? in2[b + k] : 0) - (sub ? sub[b + k] : 0) : 0;
+    }
+#pragma unroll
+    for (int t = 0; t < ONE_TILES; ++t) {
+        int x = v[t][0] + v[t][1] + v[t][2] + v[t][3];
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+        incl[t] = x;
+        if (lane == 63) ws[t][wave] = x;
+    }
+    __syncthreads();
+    int base = 0;
+#pragma unroll
+    for (int t = 0; t < ONE_TILES; ++t) {
+        int pre = 0, tot = 0;
+#pragma unroll
+        for (int w = 0; w < ONE_TPB / 64; ++w) {
+            const int x = ws[t][w];
+            pre += w < wave ? x : 0;
+            tot += x;
+        }
+        int run = base + pre + incl[t] - (v[t][0] + v[t][1] + v[t][2] + v[t][3]);
+        base += tot;
+        const int b = t * 4 * ONE_TPB + 4 * tid;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (b + k < m) {
+                out[b + k] = run;
+                if (zero) zero[b + k] = 0;
+            }
+            run += v[t][k];
+        }
+    }
+}
+
 /* Scatter (pid, slot) keys into their cell's run: one returning atomic per
  * key group, all groups in one instruction, the group base passed back from
  * its leader. */
@@ -452,29 +505,45 @@ __global__ void __launch_bounds__(SEG_CELLS) k_segsort(const int* __restrict__ s
 /* ---- incremental unshifted binning ---- */
 
 /* Arrivals go to the tail of their new cell's run (after the stayers), in
- * arrival order; the merge sorts them. */
-constexpr int PLACE_PER = 4; /* slots per thread (one 16-byte load of ranks) */
-__global__ void k_place_arrivals(const int* __restrict__ cid, const int* __restrict__ pid,
-                                 const int* __restrict__ rnk, int n, const int* __restrict__ startB,
-                                 const int* __restrict__ cnt, const int* __restrict__ dout,
-                                 unsigned long long* __restrict__ keyB) {
-    const int i0 = (blockIdx.x * blockDim.x + threadIdx.x) * PLACE_PER;
-    if (i0 >= n) return;
-    int r[PLACE_PER];
-    if (i0 + PLACE_PER <= n) {
-        const int4 q = *reinterpret_cast<const int4*>(rnk + i0);
-        r[0] = q.x;
-        r[1] = q.y;
-        r[2] = q.z;
-        r[3] = q.w;
-    } else {
-        for (int u = 0; u < PLACE_PER; ++u) r[u] = i0 + u < n ? rnk[i0 + u] : -1;
+ * arrival order; the merge sorts them.  The pass listed them (slot and rank
+ * among the new cell's arrivals), about 3% of the particles in the base pass
+ * and far fewer in the shifted one, so a fixed grid strides over the list.
+ * Blocks from nPlace on restore the velocities of the covered cells the pass
+ * changed (k_overlap_copyback's work, independent of the keys). */
+constexpr int PLACE_BLOCKS = 512;
+struct CopybackArgs {
+    const int* cells;
+    int ncells;
+    const unsigned char* chg;
+    const int *start, *list;
+    const double *vsx, *vsy;
+    double *vx, *vy;
+};
+__device__ __forceinline__ void copyback_cell(const CopybackArgs& a, int t) {
+    if (t >= a.ncells) return;
+    const int c = a.cells[t];
+    if (!a.chg[c]) return;
+    for (int j = a.start[c]; j < a.start[c + 1]; ++j) {
+        const int slot = a.list[j];
+        a.vx[slot] = a.vsx[slot];
+        a.vy[slot] = a.vsy[slot];
     }
-    for (int u = 0; u < PLACE_PER; ++u) {
-        if (r[u] < 0) continue;
-        const int i = i0 + u;
-        const int c = cid[i];
-        keyB[startB[c] + cnt[c] - dout[c] + r[u]] = ((unsigned long long)(unsigned)pid[i] << 32) | (unsigned)i;
+}
+__global__ void __launch_bounds__(TPB) k_place_arrivals(const int* __restrict__ cid, const int* __restrict__ pid,
+                                                        const int2* __restrict__ arr, const int* __restrict__ arrN,
+                                                        const int* __restrict__ startB, const int* __restrict__ cnt,
+                                                        const int* __restrict__ dout,
+                                                        unsigned long long* __restrict__ keyB, int nPlace,
+                                                        CopybackArgs cb) {
+    if ((int)blockIdx.x >= nPlace) {
+        copyback_cell(cb, ((int)blockIdx.x - nPlace) * TPB + (int)threadIdx.x);
+        return;
+    }
+    const int m = *arrN;
+    for (int j = blockIdx.x * TPB + (int)threadIdx.x; j < m; j += nPlace * TPB) {
+        const int2 e = arr[j];
+        const int c = cid[e.x];
+        keyB[startB[c] + cnt[c] - dout[c] + e.y] = ((unsigned long long)(unsigned)pid[e.x] << 32) | (unsigned)e.x;
     }
 }
 
@@ -571,9 +640,10 @@ __global__ void __launch_bounds__(REB_CELLS) k_rebin_merge(const int* __restrict
                                                            const int* __restrict__ cid, int Nc, int cpb,
                                                            const int* __restrict__ startB, int* __restrict__ cnt,
                                                            int* __restrict__ inc, int* __restrict__ dout,
-                                                           int* __restrict__ rnk, unsigned long long* keyB,
+                                                           int* __restrict__ arrN, unsigned long long* keyB,
                                                            int* __restrict__ listB, int* __restrict__ err) {
     __shared__ unsigned long long so[REB_CAP];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *arrN = 0; /* the list is used up */
     const int c0 = blockIdx.x * cpb;
     const int c1 = min(c0 + cpb, Nc);
     const int q0 = startB[c0], q1 = startB[c1];
@@ -587,7 +657,6 @@ __global__ void __launch_bounds__(REB_CELLS) k_rebin_merge(const int* __restrict
         const int ms = cnt[c] - dout[c], ki = inc[c];
         inc[c] = 0; /* clear for the next update */
         dout[c] = 0;
-        for (int j = 0; j < ki; ++j) rnk[(int)(unsigned)(keyB[nb + ms + j] & 0xffffffffull)] = -1;
         m = ms + ki;
         if (lds)
             rebin_cell(c, b, mo, nb, ms, ki, key, cid, keyB, so, nb - q0, err);
@@ -975,8 +1044,12 @@ struct ZoneArgs {
     int nZones;
     uint64_t seedBase;
     int singleSeed; /* 1: seedBase is the zone's own seed (single-zone call) */
-    const int* zsize; /* particles of each zone */
-    const int* zoff;  /* per-zone offsets into the particle regions (exclusive scan of zsize) */
+    int* zsize; /* particles of each zone */
+    int* zoff;  /* per-zone offsets into the particle regions (an exclusive scan of zsize, or k_zone_fused's) */
+    /* k_zone_fused: its zones take their regions from a counter (which zone
+     * gets which region does not matter); [1] counts the zones done, and the
+     * last one clears both */
+    unsigned long long* zcur;
     long long scratchCap;
     void* nextG;    /* links beyond LDS, IT per particle */
     void* tmpG;     /* long donor lists, IT per particle */
@@ -1276,8 +1349,46 @@ __device__ __forceinline__ void zone_uniform(Z& z) {
                  z.zp.lowThrFloor, z.zp.highThrFloor, z.zp.lowLoc1, z.zp.highLoc1, z.zp.useLocal, z.zp.maxPasses,
                  z.zp.corrEnabled, z.zp.dedupe, z.zp.quadBins, z.zp.binLo, z.zp.binHi);
     make_uniform(z.xs, z.xe, z.ys, z.ye, z.zw, z.zh, z.C, z.zhM, z.zid, z.seed, z.gcnt, z.gstart, z.glist, z.gkey, z.x,
-                 z.y, z.vx, z.vy, z.vsx, z.vsy, z.gchg, z.inPx, z.inPy, z.dcid, z.dout, z.dinc, z.drnk, z.cellOff, z.dgCell,
+                 z.y, z.vx, z.vy, z.vsx, z.vsy, z.gchg, z.inPx, z.inPy, z.dcid, z.dout, z.dinc, z.darr, z.darrN, z.cellOff, z.dgCell,
                  z.dgCnt);
+}
+
+/* The zones of more particles than 16-bit indices take: the passes on the
+ * first wavefront, then the correction on all four (one launch: as a rule it
+ * finds no such zone, and only its launch costs). */
+template <bool kLds>
+__global__ void __launch_bounds__(FINISH_TPB) k_zone_wide(ZoneArgs a) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ ZoneShared sh;
+    __shared__ int queue[FINISH_TPB];
+    int k0 = 0, zi = 0;
+    unsigned long long todo = 0ull; /* the same in every wavefront of the block */
+    while (next_zone(a, k0, todo, zi)) {
+        const int P = a.zsize[zi];
+        const long long off = a.zoff[zi];
+        if (off + (long long)P > a.scratchCap) {
+            if (threadIdx.x == 0) atomicOr(a.err, 2);
+            continue;
+        }
+        if (threadIdx.x < 64) zone_pass_body<int, kLds>(a, zi, off, (int)threadIdx.x, lds, &sh);
+        __threadfence_block();
+        __syncthreads();
+        int zid;
+        uint64_t seed;
+        const ZoneIn& in = zone_in_of<false>(a, zi, zid, seed);
+        zone_finish_body<int, kLds, FINISH_TPB, 4>(a, in, zid, seed, zi, off, (int)threadIdx.x, lds, (long long)a.ldsBytes,
+                                                  queue);
+        __syncthreads(); /* the next zone reuses the working set */
+    }
+}
+
+/* one zone of the launch is done with the region counter; the last one clears
+ * it for the next launch */
+__device__ __forceinline__ void zone_region_done(const ZoneArgs& a) {
+    if (threadIdx.x == 0 && atomicAdd(&a.zcur[1], 1ull) + 1ull == (unsigned long long)a.nZones) {
+        a.zcur[0] = 0ull;
+        a.zcur[1] = 0ull;
+    }
 }
 
 constexpr int FUSED_TPB = 256;
@@ -1288,13 +1399,6 @@ __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 
     __shared__ unsigned queue[FUSED_TPB];
     const int zi = blockIdx.x;
     if (zi >= a.nZones) return;
-    const int P = a.zsize[zi];
-    if (P < a.pMin || P > a.pMax) return;
-    const long long off = a.zoff[zi];
-    if (off + (long long)P > a.scratchCap) {
-        if (threadIdx.x == 0) atomicOr(a.err, 2);
-        return;
-    }
     /* the passes are the critical path: their wavefronts issue ahead of the
      * corrections of zones that are done */
     __builtin_amdgcn_s_setprio(3);
@@ -1318,15 +1422,32 @@ __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 
     const ZoneIn& in = *inp;
     zone_init(z, in, a.rects[zi], zid, seed, &sh);
     if constexpr (kEns) zone_uniform(z);
-    z.nxG = (IT*)a.nextG + off;
-    z.tmpG = (IT*)a.tmpG + off;
     z.duG = a.duG + (size_t)zi * (size_t)a.duStride;
-    z.rec = a.rec + off;
     zone_carve(z, lds, a.ldsBytes);
-    static_assert(FUSED_TPB == 256, "zone_setup_mw and the phases take four wavefronts");
-    zone_setup_mw(z, in, wave, lane);
+    static_assert(FUSED_TPB == 256, "the set-up and the phases take four wavefronts");
+    zone_setup_columns(z, wave, lane);
     __syncthreads();
     z.P = sh.P;
+    unsigned long long off = 0ull;
+    if (threadIdx.x == 0) off = atomicAdd(&a.zcur[0], (unsigned long long)z.P);
+    if (z.P <= a.pMax) zone_setup_cells(z, in, wave, lane);
+    if (threadIdx.x == 0) {
+        sh.off = off;
+        /* (a zone of more particles is left to the 32-bit kernels) */
+        a.zsize[zi] = z.P;
+        a.zoff[zi] = (int)off;
+        if (off + (unsigned long long)z.P > (unsigned long long)a.scratchCap) atomicOr(a.err, 2);
+        else if (kEns && z.P > a.pMax) atomicOr(a.err, 8);
+    }
+    __syncthreads();
+    off = sh.off;
+    if (z.P > a.pMax || off + (unsigned long long)z.P > (unsigned long long)a.scratchCap) {
+        zone_region_done(a);
+        return;
+    }
+    z.nxG = (IT*)a.nextG + off;
+    z.tmpG = (IT*)a.tmpG + off;
+    z.rec = a.rec + off;
     z.allOwned = zone_setup_all_owned(z);
     for (int k = (int)threadIdx.x; k < z.P; k += FUSED_TPB) z.rec[k] = (unsigned char)ZM_NONE;
     __syncthreads();
@@ -1349,24 +1470,14 @@ __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 
         o.stats5 = sh.stats5;
         a.out[zi] = o;
     }
+    zone_region_done(a);
 }
 
 /* velocities of the particles of cells several zones cover, from the side
  * buffer (their input runs in the pass-input binning), for the cells their
  * owner changed: the others' velocities are what they were */
-__global__ void k_overlap_copyback(const int* __restrict__ cells, int ncells, const unsigned char* __restrict__ chg,
-                                   const int* __restrict__ start, const int* __restrict__ list,
-                                   const double* __restrict__ vsx, const double* __restrict__ vsy,
-                                   double* __restrict__ vx, double* __restrict__ vy) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ncells) return;
-    const int c = cells[t];
-    if (!chg[c]) return;
-    for (int j = start[c]; j < start[c + 1]; ++j) {
-        const int slot = list[j];
-        vx[slot] = vsx[slot];
-        vy[slot] = vsy[slot];
-    }
+__global__ void __launch_bounds__(TPB) k_overlap_copyback(CopybackArgs a) {
+    copyback_cell(a, (int)(blockIdx.x * TPB + threadIdx.x));
 }
 
 /* a plain closure's grids and applied beta into a snapshot: out = 6 grids of
@@ -1405,19 +1516,78 @@ struct ClosureArgs {
  * check's flag: with the flag clear every block leaves at once */
 __device__ inline bool gated_off(const int* gate) { return gate && *gate == 0; }
 
-__global__ void __launch_bounds__(TPB) k_closure_repair(ClosureArgs a) {
+/* pdrive with the interzone cross smoothing (liquid_closure.cpp:401-419) of
+ * cell c */
+__device__ __forceinline__ double pdrive_at(const Geom& g, const double* __restrict__ raw, const int* __restrict__ mask,
+                                            double blend, int anyMask, int c) {
+    double v = raw[c];
+    if (anyMask && mask[c] != 0) {
+        const int ix = c / g.Ny, iy = c - ix * g.Ny;
+        double acc = raw[c];
+        int n = 1;
+        /* left, right, down, up (liquid_closure.cpp:233-236) */
+        const int ddx[4] = {-1, 1, 0, 0}, ddy[4] = {0, 0, -1, 1};
+        for (int k = 0; k < 4; ++k) {
+            int jx = ix + ddx[k], jy = iy + ddy[k];
+            if (g.perx) jx = wrapi(jx, g.Nx);
+            else if (jx < 0 || jx >= g.Nx) continue;
+            if (g.pery) jy = wrapi(jy, g.Ny);
+            else if (jy < 0 || jy >= g.Ny) continue;
+            acc += raw[jy + g.Ny * jx];
+            ++n;
+        }
+        const double ps = acc / (double)n;
+        v = (1.0 - blend) * raw[c] + blend * ps;
+    }
+    return v;
+}
+
+/* The closure's grids of one cell per thread: the repair and its block
+ * partials of (num, den), pdrive, and duEOS = -(dt/rhoT) * grad(pdrive) *
+ * betaEOS (liquid_closure.cpp:243-295, :424-430), whose neighbours' pdrive is
+ * taken again here rather than in a kernel of its own; clear0, clear1 (Nc + 1
+ * counters each, or nullptr) are cleared on the way, also when gated off. */
+__global__ void __launch_bounds__(TPB) k_closure_grids(ClosureArgs a, Geom g, const double* __restrict__ raw,
+                                                       const int* __restrict__ mask, double blend, int anyMask,
+                                                       double dtOverRho, double betaEOS, double* __restrict__ pd,
+                                                       double* __restrict__ ex, double* __restrict__ ey,
+                                                       int* __restrict__ clear0, int* __restrict__ clear1) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (clear0 && c < a.Nc) {
+        clear0[c] = 0;
+        clear1[c] = 0;
+        if (c == 0) {
+            clear0[a.Nc] = 0;
+            clear1[a.Nc] = 0;
+        }
+    }
     if (gated_off(a.gate)) return;
     __shared__ double s0[TPB], s1[TPB];
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
     double num = 0.0, den = 0.0;
     if (c < a.Nc) {
         const double ax = (a.refPx[c] - a.redPx[c]) / a.gamma;
         const double ay = (a.refPy[c] - a.redPy[c]) / a.gamma;
         a.duRX[c] = ax;
         a.duRY[c] = ay;
-        const double ex = a.redUx[c] - a.refUx[c], ey = a.redUy[c] - a.refUy[c];
-        num = -(ex * ax + ey * ay);
+        const double ux = a.redUx[c] - a.refUx[c], uy = a.redUy[c] - a.refUy[c];
+        num = -(ux * ax + uy * ay);
         den = ax * ax + ay * ay;
+        const int ix = c / g.Ny, iy = c - ix * g.Ny;
+        const double dx = g.dxc, dy = g.dyc;
+        auto p = [&](int jx, int jy) { return pdrive_at(g, raw, mask, blend, anyMask, jy + g.Ny * jx); };
+        const double pc = p(ix, iy);
+        pd[c] = pc;
+        double gx, gy;
+        if (g.perx) gx = (p(wrapi(ix + 1, g.Nx), iy) - p(wrapi(ix - 1, g.Nx), iy)) / (2.0 * dx);
+        else if (ix == 0) gx = (p(ix + 1, iy) - pc) / dx;
+        else if (ix == g.Nx - 1) gx = (pc - p(ix - 1, iy)) / dx;
+        else gx = (p(ix + 1, iy) - p(ix - 1, iy)) / (2.0 * dx);
+        if (g.pery) gy = (p(ix, wrapi(iy + 1, g.Ny)) - p(ix, wrapi(iy - 1, g.Ny))) / (2.0 * dy);
+        else if (iy == 0) gy = (p(ix, iy + 1) - pc) / dy;
+        else if (iy == g.Ny - 1) gy = (pc - p(ix, iy - 1)) / dy;
+        else gy = (p(ix, iy + 1) - p(ix, iy - 1)) / (2.0 * dy);
+        ex[c] = -dtOverRho * gx * betaEOS;
+        ey[c] = -dtOverRho * gy * betaEOS;
     }
     s0[threadIdx.x] = num;
     s1[threadIdx.x] = den;
@@ -1457,53 +1627,6 @@ __global__ void __launch_bounds__(TPB) k_reduce_beta(const double* __restrict__ 
     if (gated_off(gate)) return;
     reduce_parts_block(part, np, 2, scal);
     if (threadIdx.x == 0) beta_from_sums(scal, useOptimal, betaRepair);
-}
-
-/* pdrive with the interzone cross smoothing (liquid_closure.cpp:401-419) */
-__global__ void k_pdrive(Geom g, const double* __restrict__ raw, const int* __restrict__ mask, double blend,
-                         int anyMask, double* __restrict__ pd, const int* gate = nullptr) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= g.Nc || gated_off(gate)) return;
-    double v = raw[c];
-    if (anyMask && mask[c] != 0) {
-        const int ix = c / g.Ny, iy = c - ix * g.Ny;
-        double acc = raw[c];
-        int n = 1;
-        /* left, right, down, up (liquid_closure.cpp:233-236) */
-        const int ddx[4] = {-1, 1, 0, 0}, ddy[4] = {0, 0, -1, 1};
-        for (int k = 0; k < 4; ++k) {
-            int jx = ix + ddx[k], jy = iy + ddy[k];
-            if (g.perx) jx = wrapi(jx, g.Nx);
-            else if (jx < 0 || jx >= g.Nx) continue;
-            if (g.pery) jy = wrapi(jy, g.Ny);
-            else if (jy < 0 || jy >= g.Ny) continue;
-            acc += raw[jy + g.Ny * jx];
-            ++n;
-        }
-        const double ps = acc / (double)n;
-        v = (1.0 - blend) * raw[c] + blend * ps;
-    }
-    pd[c] = v;
-}
-
-/* duEOS = -(dt/rhoT) * grad(pdrive) * betaEOS (liquid_closure.cpp:243-295, :424-430) */
-__global__ void k_eos(Geom g, const double* __restrict__ p, double dtOverRho, double betaEOS, double* __restrict__ ex,
-                      double* __restrict__ ey, const int* gate = nullptr) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= g.Nc || gated_off(gate)) return;
-    const int ix = c / g.Ny, iy = c - ix * g.Ny;
-    const double dx = g.dxc, dy = g.dyc;
-    double gx, gy;
-    if (g.perx) gx = (p[iy + g.Ny * wrapi(ix + 1, g.Nx)] - p[iy + g.Ny * wrapi(ix - 1, g.Nx)]) / (2.0 * dx);
-    else if (ix == 0) gx = (p[iy + g.Ny * (ix + 1)] - p[c]) / dx;
-    else if (ix == g.Nx - 1) gx = (p[c] - p[iy + g.Ny * (ix - 1)]) / dx;
-    else gx = (p[iy + g.Ny * (ix + 1)] - p[iy + g.Ny * (ix - 1)]) / (2.0 * dx);
-    if (g.pery) gy = (p[wrapi(iy + 1, g.Ny) + g.Ny * ix] - p[wrapi(iy - 1, g.Ny) + g.Ny * ix]) / (2.0 * dy);
-    else if (iy == 0) gy = (p[(iy + 1) + g.Ny * ix] - p[c]) / dy;
-    else if (iy == g.Ny - 1) gy = (p[c] - p[(iy - 1) + g.Ny * ix]) / dy;
-    else gy = (p[(iy + 1) + g.Ny * ix] - p[(iy - 1) + g.Ny * ix]) / (2.0 * dy);
-    ex[c] = -dtOverRho * gx * betaEOS;
-    ey[c] = -dtOverRho * gy * betaEOS;
 }
 
 /* The closure's kick: repair (scaled by beta) then EOS correction. */
@@ -1918,8 +2041,10 @@ struct Binning {
     int *cnt = nullptr, *start = nullptr, *cursor = nullptr, *list = nullptr;
     unsigned long long* key = nullptr; /* (pid << 32 | slot) in (cell, pid) order */
     /* the incremental update's second buffers (swapped with the above),
-     * per-cell incoming counts and per-slot rank among a cell's incoming */
-    int *startB = nullptr, *listB = nullptr, *inc = nullptr, *rnk = nullptr;
+     * per-cell incoming counts */
+    int *startB = nullptr, *listB = nullptr, *inc = nullptr;
+    int2* arr = nullptr; /* the arrivals a pass listed */
+    int* arrN = nullptr; /* and their number (zero between updates) */
     unsigned long long* keyB = nullptr;
     int* cntS = nullptr; /* counts of the shifted collision cells */
     int* dout = nullptr; /* departures per cell recorded by a zone pass (zero between updates) */
@@ -1945,6 +2070,7 @@ struct mpcd_gpu_sim {
     int *next = nullptr, *tmpg = nullptr;
     long long scratchCap = 0;
     int *zsize = nullptr, *zoff = nullptr;
+    unsigned long long* zcur = nullptr; /* k_zone_fused's region counter (zero between launches) */
     double* stage = nullptr; /* 2n doubles, host<->device transfers */
     double *refPx = nullptr, *refPy = nullptr, *refUx = nullptr, *refUy = nullptr, *pdriveRaw = nullptr;
     double *redPx = nullptr, *redPy = nullptr, *redUx = nullptr, *redUy = nullptr;
@@ -2015,6 +2141,7 @@ struct mpcd_gpu_sim {
     BCParams bc{};
     double xmax = 0, ymax = 0;
     int fuseNext = -1; /* step whose stream the current kick performs (-1: none) */
+    CopybackArgs pendCopy{};  /* a recording pass's copy-back, taken by its update */
     bool recDirty = false; /* a recording pass was launched and its update has not run */
     int streamed = -1; /* step whose stream has been performed by a kick (-1: none) */
     int cellCap = 0; /* LDS entries of a per-cell block (k_collide, k_cell_fields) */
@@ -2120,7 +2247,10 @@ struct mpcd_gpu_sim {
         bin.startB = dalloc<int>((size_t)Nc + 1);
         bin.listB = dalloc<int>(n);
         bin.inc = dalloc<int>((size_t)Nc + 1);
-        bin.rnk = dalloc<int>(n);
+        bin.arr = dalloc<int2>(n);
+        bin.arrN = dalloc<int>(1);
+        zcur = dalloc<unsigned long long>(2);
+        HIP_OK(hipMemset(zcur, 0, 2 * sizeof(unsigned long long)));
         bin.keyB = dalloc<unsigned long long>(n);
         bin.cntS = dalloc<int>((size_t)Nc + 1);
         bin.dout = dalloc<int>((size_t)Nc + 1);
@@ -2150,7 +2280,7 @@ struct mpcd_gpu_sim {
         hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, stream, err, 1, 0); /* no error flagged yet */
         hipLaunchKernelGGL(k_fill_int, dim3(nblk(Nc + 1)), dim3(TPB), 0, stream, bin.inc, Nc + 1, 0);
         hipLaunchKernelGGL(k_fill_int, dim3(nblk(Nc + 1)), dim3(TPB), 0, stream, bin.dout, Nc + 1, 0);
-        hipLaunchKernelGGL(k_fill_int, dim3(nblk(n)), dim3(TPB), 0, stream, bin.rnk, n, -1);
+        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, stream, bin.arrN, 1, 0);
         check_launch();
         /* constants */
         bc = make_bc_params(p);
@@ -2215,7 +2345,7 @@ struct mpcd_gpu_sim {
     }
 
     ~mpcd_gpu_sim() {
-        void* ptrs[] = {x, y, vx, vy, vx2, vy2, x2, y2, pid, pid2, cid, cidS, bin.cnt, bin.start, bin.cursor, bin.list, bin.key, bin.startB, bin.listB, bin.inc, bin.rnk, bin.keyB, bin.cntS, bin.dout, tileSum, next,
+        void* ptrs[] = {x, y, vx, vy, vx2, vy2, x2, y2, pid, pid2, cid, cidS, bin.cnt, bin.start, bin.cursor, bin.list, bin.key, bin.startB, bin.listB, bin.inc, bin.arr, bin.arrN, zcur, bin.keyB, bin.cntS, bin.dout, tileSum, next,
                         tmpg, zsize, zoff, owner[0], owner[1], cover[0], cover[1], overCells[0], overCells[1], stage,
                         refPx, refPy, refUx, refUy, pdriveRaw, redPx, redPy, redUx, redUy, duRX, duRY, duEX, duEY,
                         pdrive, cellTmp, mask, part, scal, err, wallPart, rects[0], rects[1], zout, zscratch, duG, recG, zstate, chg,
@@ -2297,6 +2427,17 @@ struct mpcd_gpu_sim {
         if (hv) download_xy(vx, vy, hv);
     }
 
+    /* exclusive scan of in + in2 - sub over m entries; zero cleared beside it */
+    void scan(const int* in, int m, int* out, const int* in2, int* zero, const int* sub) {
+        if (m <= ONE_TILES * 4 * ONE_TPB) {
+            hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(ONE_TPB), 0, stream, in, m, out, in2, zero, sub);
+            return;
+        }
+        hipLaunchKernelGGL(k_scan_tiles, dim3((m + SCAN_TILE - 1) / SCAN_TILE), dim3(TPB), 0, stream, in, m, out, tileSum,
+                           in2, zero, sub);
+        hipLaunchKernelGGL(k_scan_add_prefix, dim3(nblk(m)), dim3(TPB), 0, stream, out, m, tileSum);
+    }
+
     /* ---- binning: cnt/start/list of the cell ids in `key` ---- */
     void bin_cells(const int* key) { bin_cells(key, bin.cnt, false, true); }
     /* cnt: the counts (the unshifted binning keeps them in bin.cnt);
@@ -2309,9 +2450,7 @@ struct mpcd_gpu_sim {
             hipLaunchKernelGGL(k_hist, dim3(bin_blocks(n)), dim3(TPB), 0, stream, key, n, cnt);
         }
         /* the scan clears the scatter's cursors */
-        hipLaunchKernelGGL(k_scan_tiles, dim3(nTiles), dim3(TPB), 0, stream, cnt, Nc + 1, bin.start, tileSum,
-                           (const int*)nullptr, bin.cursor);
-        hipLaunchKernelGGL(k_scan_add_prefix, dim3(nblk(Nc + 1)), dim3(TPB), 0, stream, bin.start, Nc + 1, tileSum);
+        scan(cnt, Nc + 1, bin.start, nullptr, bin.cursor, nullptr);
         hipLaunchKernelGGL(k_scatter, dim3(bin_blocks(n)), dim3(TPB), 0, stream, key, pid, n, bin.start, bin.cursor,
                            bin.key);
         hipLaunchKernelGGL(k_segsort, dim3(nblk(Nc, SEG_CELLS)), dim3(SEG_CELLS), 0, stream, bin.start, Nc, bin.key,
@@ -2324,21 +2463,22 @@ struct mpcd_gpu_sim {
         bin_cells(cid);
     }
     /* The unshifted binning after a zone pass that recorded its cell changes
-     * (bin.rnk -1 for every slot before it, then each moved particle's new cell in
-     * cid, its departure in dout, its rank among its new cell's arrivals):
-     * the runs are the old runs' stayers merged with the arrivals, in pid
-     * order, the same binning a counting sort of the new cells gives. */
+     * (each moved particle's new cell in cid, its departure in dout, itself in
+     * the list of arrivals): the runs are the old runs' stayers merged with
+     * the arrivals, in pid order, the same binning a counting sort of the new
+     * cells gives.  The pass's copy-back runs beside the arrivals' placing. */
     void rebin_recorded() {
-        hipLaunchKernelGGL(k_scan_tiles, dim3(nTiles), dim3(TPB), 0, stream, bin.cnt, Nc + 1, bin.startB, tileSum,
-                           bin.inc, (int*)nullptr, bin.dout);
-        hipLaunchKernelGGL(k_scan_add_prefix, dim3(nblk(Nc + 1)), dim3(TPB), 0, stream, bin.startB, Nc + 1, tileSum);
-        hipLaunchKernelGGL(k_place_arrivals, dim3(nblk((n + PLACE_PER - 1) / PLACE_PER)), dim3(TPB), 0, stream, cid, pid,
-                           bin.rnk, n, bin.startB, bin.cnt, bin.dout, bin.keyB);
+        scan(bin.cnt, Nc + 1, bin.startB, bin.inc, nullptr, bin.dout);
+        const int nPlace = (int)std::min<unsigned>(nblk(n), PLACE_BLOCKS);
+        const int nCopy = pendCopy.ncells > 0 ? (int)nblk(pendCopy.ncells) : 0;
+        hipLaunchKernelGGL(k_place_arrivals, dim3(nPlace + nCopy), dim3(TPB), 0, stream, cid, pid, bin.arr, bin.arrN,
+                           bin.startB, bin.cnt, bin.dout, bin.keyB, nPlace, pendCopy);
+        pendCopy = CopybackArgs{};
         /* cells per block: the block's runs fit the LDS staging at 1.25x the mean density */
         int cpb = REB_CELLS;
         while (cpb > 64 && (double)cpb * (double)n / (double)Nc * 1.25 > (double)REB_CAP) cpb >>= 1;
         hipLaunchKernelGGL(k_rebin_merge, dim3(nblk(Nc, cpb)), dim3(REB_CELLS), 0, stream, bin.start, bin.key, cid,
-                           Nc, cpb, bin.startB, bin.cnt, bin.inc, bin.dout, bin.rnk, bin.keyB, bin.listB, err);
+                           Nc, cpb, bin.startB, bin.cnt, bin.inc, bin.dout, bin.arrN, bin.keyB, bin.listB, err);
         check_launch();
         recDirty = false;
         std::swap(bin.start, bin.startB);
@@ -2458,15 +2598,23 @@ struct mpcd_gpu_sim {
                    const unsigned char* coverDev, const int* overDev, int nOverCells, int single,
                    const double* inPx = nullptr, const double* inPy = nullptr, bool record = false,
                    const unsigned char* zmask = nullptr, bool stats = true) {
-        hipLaunchKernelGGL(k_zone_sizes, dim3(nZ + 1), dim3(64), 0, stream, rectsDev, nZ, bin.start, p.Ny, zsize);
-        const int nt = (nZ + 1 + SCAN_TILE - 1) / SCAN_TILE;
-        hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(TPB), 0, stream, zsize, nZ + 1, zoff, tileSum,
-                           (const int*)nullptr, (int*)nullptr);
-        if (nt > 1) { /* one tile is already the whole scan */
-            hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(TPB), 0, stream, tileSum, nt);
-            hipLaunchKernelGGL(k_scan_add, dim3(nblk(nZ + 1)), dim3(TPB), 0, stream, zoff, nZ + 1, tileSum);
+        const size_t fix16 = zone_fixed_bytes<uint16_t>(maxC, maxW, zp.useLocal);
+        const bool fast = maxC < 65535 && fix16 + 2048 <= (size_t)ZONE_LDS_FAST;
+        /* LDS staging of the correction: the cell arrays and the column map leave room for links */
+        const size_t cellB16 = (size_t)maxC * (sizeof(ZCell<uint16_t>) + sizeof(uint16_t)) + 8 * (size_t)maxW + 16;
+        /* passes and correction in one kernel when the correction fits the passes' LDS */
+        const bool fused = fast && cellB16 + 4096 <= (size_t)ZONE_LDS_FAST;
+        if (!fused) { /* the fused kernel finds its zones' sizes and regions itself */
+            hipLaunchKernelGGL(k_zone_sizes, dim3(nZ + 1), dim3(64), 0, stream, rectsDev, nZ, bin.start, p.Ny, zsize);
+            const int nt = (nZ + 1 + SCAN_TILE - 1) / SCAN_TILE;
+            hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(TPB), 0, stream, zsize, nZ + 1, zoff, tileSum,
+                               (const int*)nullptr, (int*)nullptr);
+            if (nt > 1) { /* one tile is already the whole scan */
+                hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(TPB), 0, stream, tileSum, nt);
+                hipLaunchKernelGGL(k_scan_add, dim3(nblk(nZ + 1)), dim3(TPB), 0, stream, zoff, nZ + 1, tileSum);
+            }
+            check_launch();
         }
-        check_launch();
         ensure_du((size_t)nZ * 2 * (size_t)maxC);
         ZoneArgs a{};
         a.in.g = g;
@@ -2491,19 +2639,20 @@ struct mpcd_gpu_sim {
         a.in.zmask = zmask;
         if (record) {
             /* moved particles record their cell changes for rebin_recorded()
-             * (bin.rnk is -1 for every slot here: set at creation, and each
-             * merge resets the ranks of the arrivals it took; after an
-             * interrupted pass-and-update the record is cleared again) */
+             * (the record is empty here: the merge leaves it so; after an
+             * interrupted pass-and-update it is cleared again) */
             if (recDirty) {
-                hipLaunchKernelGGL(k_fill_int, dim3(nblk(n)), dim3(TPB), 0, stream, bin.rnk, n, -1);
+                hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, stream, bin.arrN, 1, 0);
                 hipLaunchKernelGGL(k_fill_int, dim3(nblk(Nc + 1)), dim3(TPB), 0, stream, bin.inc, Nc + 1, 0);
                 hipLaunchKernelGGL(k_fill_int, dim3(nblk(Nc + 1)), dim3(TPB), 0, stream, bin.dout, Nc + 1, 0);
             }
             recDirty = true;
+            pendCopy = CopybackArgs{};
             a.in.dcid = cid;
             a.in.dout = bin.dout;
             a.in.dinc = bin.inc;
-            a.in.drnk = bin.rnk;
+            a.in.darr = reinterpret_cast<int*>(bin.arr);
+            a.in.darrN = bin.arrN;
         }
         a.rects = rectsDev;
         a.nZones = nZ;
@@ -2511,6 +2660,7 @@ struct mpcd_gpu_sim {
         a.singleSeed = single;
         a.zsize = zsize;
         a.zoff = zoff;
+        a.zcur = zcur;
         a.scratchCap = scratchCap;
         a.nextG = next;
         a.tmpG = tmpg;
@@ -2524,13 +2674,6 @@ struct mpcd_gpu_sim {
         a.wantStats = stats;
         a.err = err;
         pbeg(MPCD_PROF_ZONE_KERNEL);
-        const size_t fix16 = zone_fixed_bytes<uint16_t>(maxC, maxW, zp.useLocal);
-        const bool fast = maxC < 65535 && fix16 + 2048 <= (size_t)ZONE_LDS_FAST;
-        /* LDS staging of the correction: the cell arrays and the column map leave room for links */
-        const size_t cellB16 = (size_t)maxC * (sizeof(ZCell<uint16_t>) + sizeof(uint16_t)) + 8 * (size_t)maxW + 16;
-        const size_t cellB32 = (size_t)maxC * (sizeof(ZCell<int>) + sizeof(int)) + 8 * (size_t)maxW + 16;
-        /* passes and correction in one kernel when the correction fits the passes' LDS */
-        const bool fused = fast && cellB16 + 4096 <= (size_t)ZONE_LDS_FAST;
         if (fast) {
             a.pMin = 0;
             a.pMax = 65534;
@@ -2541,50 +2684,52 @@ struct mpcd_gpu_sim {
                 hipLaunchKernelGGL((k_zone<uint16_t, true>), dim3(nZ), dim3(ZONE_TPB), ZONE_LDS_FAST, stream, a);
             check_launch();
         }
-        /* zones the uint16_t path does not take (none, as a rule: a small grid
-         * strides over the zones then; all zones when the 16-bit form is out) */
-        const int nBig = fast ? std::min(nZ, 64) : nZ;
-        a.pMin = fast ? 65535 : 0;
-        a.pMax = 0x7fffffff;
-        const size_t fix32 = zone_fixed_bytes<int>(maxC, maxW, zp.useLocal);
-        if (fix32 <= (size_t)ZONE_LDS_CAP) {
-            a.ldsBytes = ZONE_LDS_CAP;
-            hipLaunchKernelGGL((k_zone<int, true>), dim3(nBig), dim3(ZONE_TPB), ZONE_LDS_CAP, stream, a);
-        } else {
-            const size_t need = fix32 * (size_t)nZ;
-            if (need > zscratchCap) {
-                if (zscratch) HIP_OK(hipFree(zscratch));
-                zscratch = dalloc<unsigned char>(need);
-                zscratchCap = need;
-            }
-            a.gscratch = zscratch;
-            a.gstride = fix32;
-            hipLaunchKernelGGL((k_zone<int, false>), dim3(nBig), dim3(ZONE_TPB), 0, stream, a);
-        }
         pend(MPCD_PROF_ZONE_KERNEL);
-        check_launch();
-        /* the correction, with the same split of the zones by index type */
-        pbeg(MPCD_PROF_ZONE_FINISH);
         if (fast && !fused) {
-            a.pMin = 0;
-            a.pMax = 65534;
+            pbeg(MPCD_PROF_ZONE_FINISH);
             if (cellB16 + 4096 <= (size_t)FINISH_LDS)
                 hipLaunchKernelGGL((k_zone_finish<uint16_t, true>), dim3(nZ), dim3(FINISH_TPB), FINISH_LDS, stream, a);
             else
                 hipLaunchKernelGGL((k_zone_finish<uint16_t, false>), dim3(nZ), dim3(FINISH_TPB), 0, stream, a);
-        }
-        a.pMin = fast ? 65535 : 0;
-        a.pMax = 0x7fffffff;
-        if (cellB32 + 4096 <= (size_t)FINISH_LDS)
-            hipLaunchKernelGGL((k_zone_finish<int, true>), dim3(nBig), dim3(FINISH_TPB), FINISH_LDS, stream, a);
-        else
-            hipLaunchKernelGGL((k_zone_finish<int, false>), dim3(nBig), dim3(FINISH_TPB), 0, stream, a);
-        pend(MPCD_PROF_ZONE_FINISH);
-        check_launch();
-        if (!single && coverDev && nOverCells > 0) {
-            hipLaunchKernelGGL(k_overlap_copyback, dim3(nblk(nOverCells)), dim3(TPB), 0, stream, overDev, nOverCells,
-                               chg, bin.start, bin.list, vx2, vy2, vx, vy);
+            pend(MPCD_PROF_ZONE_FINISH);
             check_launch();
+        }
+        /* zones the 16-bit path does not take, passes and correction in one
+         * launch: none, as a rule, and none at all in a state of fewer
+         * particles than such a zone has (a small grid strides over the zones;
+         * all zones when the 16-bit form is out) */
+        if (!fast || n >= 65535) {
+            const int nBig = fast ? std::min(nZ, 64) : nZ;
+            a.pMin = fast ? 65535 : 0;
+            a.pMax = 0x7fffffff;
+            const size_t fix32 = zone_fixed_bytes<int>(maxC, maxW, zp.useLocal);
+            const size_t cellB32 = (size_t)maxC * (sizeof(ZCell<int>) + sizeof(int)) + 8 * (size_t)maxW + 16;
+            pbeg(MPCD_PROF_ZONE_FINISH);
+            if (fix32 <= (size_t)ZONE_LDS_CAP && cellB32 + 4096 <= (size_t)ZONE_LDS_CAP) {
+                a.ldsBytes = ZONE_LDS_CAP;
+                hipLaunchKernelGGL((k_zone_wide<true>), dim3(nBig), dim3(FINISH_TPB), ZONE_LDS_CAP, stream, a);
+            } else {
+                const size_t need = fix32 * (size_t)nZ;
+                if (need > zscratchCap) {
+                    if (zscratch) HIP_OK(hipFree(zscratch));
+                    zscratch = dalloc<unsigned char>(need);
+                    zscratchCap = need;
+                }
+                a.gscratch = zscratch;
+                a.gstride = fix32;
+                hipLaunchKernelGGL((k_zone_wide<false>), dim3(nBig), dim3(FINISH_TPB), 0, stream, a);
+            }
+            pend(MPCD_PROF_ZONE_FINISH);
+            check_launch();
+        }
+        if (!single && coverDev && nOverCells > 0) {
+            const CopybackArgs cb{overDev, nOverCells, chg, bin.start, bin.list, vx2, vy2, vx, vy};
+            if (record) {
+                pendCopy = cb; /* with the binning update that follows a recording pass */
+            } else {
+                hipLaunchKernelGGL(k_overlap_copyback, dim3(nblk(nOverCells)), dim3(TPB), 0, stream, cb);
+                check_launch();
+            }
         }
     }
 
@@ -2631,8 +2776,7 @@ struct mpcd_gpu_sim {
             const uint64_t un = (uint64_t)fuseNext;
             double sh[2];
             mpcd_draw_shift(130363ULL + 10007ULL * un + seedOff, p.a0, &sh[0], &sh[1]);
-            hipLaunchKernelGGL(k_fill_int, dim3(nblk(Nc + 1)), dim3(TPB), 0, stream, bin.cntS, Nc + 1, 0);
-            hipLaunchKernelGGL(k_fill_int, dim3(nblk(Nc + 1)), dim3(TPB), 0, stream, bin.cnt, Nc + 1, 0);
+            /* closure_grids() cleared both histograms */
             hipLaunchKernelGGL(k_kick_reorder_stream, dim3(nblk(n)), dim3(TPB), 0, stream, g, bc,
                                104729ULL + 10007ULL * un + seedOff, bin.list, x, y, vx, vy, pid, x2, y2, vx2, vy2, pid2, duRX,
                                duRY, duEX, duEY, scal, cidS, cid, sh[0], sh[1], xmax, ymax, bin.cntS, bin.cnt, err);
@@ -2687,13 +2831,13 @@ struct mpcd_gpu_sim {
         ClosureArgs ca = closure_args();
         ca.gate = gate;
         const int nbc = (int)nblk(Nc);
-        hipLaunchKernelGGL(k_closure_repair, dim3(nbc), dim3(TPB), 0, stream, ca);
+        /* the counters the fused kick fills are cleared beside */
+        const bool clr = fuseNext >= 0;
+        hipLaunchKernelGGL(k_closure_grids, dim3(nbc), dim3(TPB), 0, stream, ca, g, pdriveRaw, mask,
+                           p.smoothPdriveInterzoneBlend, anyMask, p.dt / rho_target(), p.betaEOS, pdrive, duEX, duEY,
+                           clr ? bin.cntS : (int*)nullptr, clr ? bin.cnt : (int*)nullptr);
         hipLaunchKernelGGL(k_reduce_beta, dim3(1), dim3(TPB), 0, stream, part, nbc, scal, p.useOptimalBetaRepair,
                            p.betaRepair, gate);
-        hipLaunchKernelGGL(k_pdrive, dim3(nbc), dim3(TPB), 0, stream, g, pdriveRaw, mask, p.smoothPdriveInterzoneBlend,
-                           anyMask, pdrive, gate);
-        const double dtr = p.dt / rho_target();
-        hipLaunchKernelGGL(k_eos, dim3(nbc), dim3(TPB), 0, stream, g, pdrive, dtr, p.betaEOS, duEX, duEY, gate);
         check_launch();
     }
 

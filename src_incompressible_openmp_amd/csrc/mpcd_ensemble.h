@@ -197,32 +197,6 @@ __global__ void __launch_bounds__(CELL_BLK) k_ens_cell_fields(const EnsRep* __re
     if (f.P) f.P[c] = s.P;
 }
 
-/* particles of each zone of every replica (k_zone_sizes on the replica's
- * cells); a zone too large for the 16-bit working set is flagged (bit 8) */
-__global__ void __launch_bounds__(64) k_ens_zone_sizes(const ZoneRect* __restrict__ rects,
-                                                       const int* __restrict__ zrep,
-                                                       const EnsRep* __restrict__ reps, int nZ,
-                                                       const int* __restrict__ start, int* __restrict__ sizes,
-                                                       int* __restrict__ err) {
-    const int zi = blockIdx.x, lane = threadIdx.x;
-    if (zi > nZ) return;
-    if (zi == nZ) {
-        if (lane == 0) sizes[zi] = 0;
-        return;
-    }
-    const ZoneRect rc = rects[zi];
-    const EnsRep& e = reps[zrep[zi]];
-    const int* st = start + e.coff;
-    const int Ny = e.g.Ny;
-    int P = 0;
-    for (int gx = rc.xs + lane; gx < rc.xe; gx += 64) P += st[(rc.ye - 1 + Ny * gx) + 1] - st[rc.ys + Ny * gx];
-    for (int o = 32; o > 0; o >>= 1) P += __shfl_xor(P, o, 64);
-    if (lane == 0) {
-        sizes[zi] = P;
-        if (P > 65534) atomicOr(err, 8);
-    }
-}
-
 /* closure repair per replica in blocks aligned to its cells (block b of the
  * launch is block b - boff[r] of replica r): the same per-block partials of
  * (num, den) as k_closure_repair on the replica alone */
@@ -479,7 +453,9 @@ struct mpcd_gpu_ensemble {
     unsigned long long* keyB = nullptr;
     /* the passes' record of moved particles: departures and arrivals per cell,
      * each arrival's rank (-1 for every slot between updates) */
-    int *dout = nullptr, *inc = nullptr, *rnk = nullptr;
+    int *dout = nullptr, *inc = nullptr, *arrN = nullptr;
+    int2* arr = nullptr; /* the arrivals a pass listed, arrN of them */
+    unsigned long long* zcur = nullptr; /* k_zone_fused's region counter */
     int nTiles = 0, narrow = 1, cellCap = 256;
     /* cells */
     double *refPx = nullptr, *refPy = nullptr, *refUx = nullptr, *refUy = nullptr, *pdriveRaw = nullptr;
@@ -494,6 +470,7 @@ struct mpcd_gpu_ensemble {
     int* owner[2] = {nullptr, nullptr};
     unsigned char* cover[2] = {nullptr, nullptr};
     unsigned char* chg = nullptr; /* covered cells their owner changed in a pass */
+    CopybackArgs pendCopy{};      /* a pass's copy-back, taken by its binning update */
     int* overCells[2] = {nullptr, nullptr};
     int nOver[2] = {0, 0};
     ZoneIn* ensIn[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}}; /* [parity][layout] */
@@ -624,7 +601,7 @@ struct mpcd_gpu_ensemble {
         HIP_OK(hipMemcpy(boff, hb.data(), hb.size() * sizeof(int), hipMemcpyHostToDevice));
         /* state and binning */
         for (double** q : {&x, &y, &vx, &vy, &x2, &y2, &vx2, &vy2}) *q = dalloc<double>((size_t)N);
-        for (int** q : {&pid, &pid2, &cidS, &cidU, &list, &listB, &rnk}) *q = dalloc<int>((size_t)N);
+        for (int** q : {&pid, &pid2, &cidS, &cidU, &list, &listB}) *q = dalloc<int>((size_t)N);
         key = dalloc<unsigned long long>((size_t)N);
         keyB = dalloc<unsigned long long>((size_t)N);
         for (int** q : {&cnt, &start, &cursor, &startB, &dout, &inc}) *q = dalloc<int>((size_t)C + 1);
@@ -648,7 +625,11 @@ struct mpcd_gpu_ensemble {
         err = dalloc<int>(1);
         hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, stream, err, 1, 0);
         hipLaunchKernelGGL(k_fill_double, dim3(nblk(2 * (size_t)R)), dim3(TPB), 0, stream, flowAcc, 2 * R, 0.0);
-        hipLaunchKernelGGL(k_fill_int, dim3(nblk(N)), dim3(TPB), 0, stream, rnk, N, -1);
+        arr = dalloc<int2>((size_t)N);
+        arrN = dalloc<int>(1);
+        zcur = dalloc<unsigned long long>(2);
+        HIP_OK(hipMemset(zcur, 0, 2 * sizeof(unsigned long long)));
+        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, stream, arrN, 1, 0);
         hipLaunchKernelGGL(k_fill_int, dim3(nblk(C + 1)), dim3(TPB), 0, stream, dout, C + 1, 0);
         hipLaunchKernelGGL(k_fill_int, dim3(nblk(C + 1)), dim3(TPB), 0, stream, inc, C + 1, 0);
         check_launch();
@@ -721,7 +702,8 @@ struct mpcd_gpu_ensemble {
                     q.dcid = cidU; /* global cells: the recorded ones get cellOff */
                     q.dout = dout;
                     q.dinc = inc;
-                    q.drnk = rnk;
+                    q.darr = reinterpret_cast<int*>(arr);
+                    q.darrN = arrN;
                     q.cellOff = e.coff;
                     q.owner = owner[L] + e.coff;
                     q.gcover = hasCover[(size_t)r] ? cover[L] + e.coff : nullptr;
@@ -757,7 +739,7 @@ struct mpcd_gpu_ensemble {
                 for (hipGraphExec_t& g : b)
                     if (g) (void)hipGraphExecDestroy(g);
         void* ptrs[] = {reps, poff, coff, boff, x, y, vx, vy, x2, y2, vx2, vy2, pid, pid2, cidS, cidU, cnt, start,
-                        cursor, list, tileSum, key, startB, listB, keyB, dout, inc, rnk, refPx, refPy, refUx, refUy, pdriveRaw, redPx, redPy, redUx, redUy,
+                        cursor, list, tileSum, key, startB, listB, keyB, dout, inc, arr, arrN, zcur, refPx, refPy, refUx, refUy, pdriveRaw, redPx, redPy, redUx, redUy,
                         duRX, duRY, duEX, duEY, pdrive, mask, part, scal, rects[0], rects[1], zrep[0], zrep[1],
                         zoneOff[0], zoneOff[1], owner[0], owner[1], cover[0], cover[1], chg, overCells[0], overCells[1],
                         ensIn[0][0], ensIn[0][1], ensIn[1][0], ensIn[1][1], zsize, zoff, next, tmpg, recG, zstate,
@@ -819,20 +801,12 @@ struct mpcd_gpu_ensemble {
     /* one snapshot zone pass of layout L over every replica */
     void zone_pass(int L) {
         const int nz = Z[L];
-        hipLaunchKernelGGL(k_ens_zone_sizes, dim3(nz + 1), dim3(64), 0, stream, rects[L], zrep[L], reps, nz, start,
-                           zsize, err);
-        const int nt = (nz + 1 + SCAN_TILE - 1) / SCAN_TILE;
-        hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(TPB), 0, stream, zsize, nz + 1, zoff, tileSum,
-                           (const int*)nullptr, (int*)nullptr);
-        if (nt > 1) {
-            hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(TPB), 0, stream, tileSum, nt);
-            hipLaunchKernelGGL(k_scan_add, dim3(nblk(nz + 1)), dim3(TPB), 0, stream, zoff, nz + 1, tileSum);
-        }
         ZoneArgs a{};
         a.rects = rects[L];
         a.nZones = nz;
         a.zsize = zsize;
         a.zoff = zoff;
+        a.zcur = zcur;
         a.scratchCap = scratchCap;
         a.nextG = next;
         a.tmpG = tmpg;
@@ -852,11 +826,7 @@ struct mpcd_gpu_ensemble {
         a.ensZoneOff = zoneOff[L];
         hipLaunchKernelGGL((k_zone_fused<uint16_t, true>), dim3(nz), dim3(FUSED_TPB), ZONE_LDS_FAST, stream, a);
         check_launch();
-        if (nOver[L] > 0) {
-            hipLaunchKernelGGL(k_overlap_copyback, dim3(nblk(nOver[L])), dim3(TPB), 0, stream, overCells[L], nOver[L],
-                               chg, start, list, vx2, vy2, vx, vy);
-            check_launch();
-        }
+        pendCopy = nOver[L] > 0 ? CopybackArgs{overCells[L], nOver[L], chg, start, list, vx2, vy2, vx, vy} : CopybackArgs{};
     }
 
     /* the unshifted binning after a zone pass from its recorded moves
@@ -867,12 +837,14 @@ struct mpcd_gpu_ensemble {
         hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(TPB), 0, stream, cnt, C + 1, startB, tileSum, inc,
                            (int*)nullptr, dout);
         hipLaunchKernelGGL(k_scan_add_prefix, dim3(nblk(C + 1)), dim3(TPB), 0, stream, startB, C + 1, tileSum);
-        hipLaunchKernelGGL(k_place_arrivals, dim3(nblk((N + PLACE_PER - 1) / PLACE_PER)), dim3(TPB), 0, stream, cidU,
-                           pid, rnk, N, startB, cnt, dout, keyB);
+        const int nPlace = (int)std::min<unsigned>(nblk(N), PLACE_BLOCKS);
+        const int nCopy = pendCopy.ncells > 0 ? (int)nblk(pendCopy.ncells) : 0;
+        hipLaunchKernelGGL(k_place_arrivals, dim3(nPlace + nCopy), dim3(TPB), 0, stream, cidU, pid, arr, arrN, startB, cnt,
+                           dout, keyB, nPlace, pendCopy);
         int cpb = REB_CELLS;
         while (cpb > 64 && (double)cpb * (double)N / (double)C * 1.25 > (double)REB_CAP) cpb >>= 1;
         hipLaunchKernelGGL(k_rebin_merge, dim3(nblk(C, cpb)), dim3(REB_CELLS), 0, stream, start, key, cidU, C, cpb,
-                           startB, cnt, inc, dout, rnk, keyB, listB, err);
+                           startB, cnt, inc, dout, arrN, keyB, listB, err);
         check_launch();
         std::swap(start, startB);
         std::swap(key, keyB);

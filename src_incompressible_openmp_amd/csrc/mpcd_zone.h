@@ -207,8 +207,9 @@ struct ZoneIn {
     const double *inPx = nullptr, *inPy = nullptr;
     /* non-null: each moved particle's cell change is recorded for the
      * binning update (cell of each slot, departures and arrivals per cell,
-     * rank among the new cell's arrivals) */
-    int *dcid = nullptr, *dout = nullptr, *dinc = nullptr, *drnk = nullptr;
+     * the list of arrivals: slot and rank among the new cell's, and its
+     * length) */
+    int *dcid = nullptr, *dout = nullptr, *dinc = nullptr, *darr = nullptr, *darrN = nullptr;
     /* non-null (a single-zone call that reports ZoneKernelStats.diag): per
      * zone cell, the momentum defect and the final list's momentum before
      * the correction (4 doubles), and the count the sparse phase starts
@@ -232,7 +233,8 @@ struct ZoneShared {
     int mwNext;            /* and the next list position a wavefront takes */
     int schedWait;         /* nonzero: a wait of the dependency-driven dense phase hit its bound */
     int nHigh, nLow, movedDense, movedSparse;
-    int mixed;             /* zone_setup_mw: a cell is not plainly owned */
+    int mixed;             /* zone_setup_cells: a cell is not plainly owned */
+    unsigned long long off; /* the zone's offset into the particle regions */
     double stats4, stats5;
 };
 
@@ -267,7 +269,7 @@ struct ZoneCtxT {
     double *x, *y, *vx, *vy, *vsx, *vsy;
     unsigned char* gchg; /* changed covered cells, or nullptr */
     const double *inPx, *inPy; /* input run sums per global cell, or nullptr */
-    int *dcid, *dout, *dinc, *drnk; /* cell-change record, or nullptr */
+    int *dcid, *dout, *dinc, *darr, *darrN; /* cell-change record, or nullptr */
     int cellOff;    /* added to the recorded new cells */
     double* dgCell; /* diagnostics' per-cell record, or nullptr */
     int* dgCnt;     /* diagnostics' sparse-phase start counts, or nullptr */
@@ -709,10 +711,19 @@ ZHD void place_moved(Z& z, int lc, int slot, uint32_t pid, int tag) {
             z.dcid[slot] = cn;
 #if defined(__HIP_DEVICE_COMPILE__)
             atomicAdd(&z.dout[co], 1);
-            z.drnk[slot] = atomicAdd(&z.dinc[cn], 1);
+            const int r = atomicAdd(&z.dinc[cn], 1);
+            /* one place in the list for all lanes here at once */
+            const unsigned long long act = wave_ballot(true);
+            const int ln = (int)__lane_id();
+            int base = 0;
+            if (ln == (int)__builtin_ctzll(act)) base = atomicAdd(z.darrN, wave_popc(act));
+            base = __builtin_amdgcn_readfirstlane(base) + wave_popc(act & lanes_below(ln));
+            reinterpret_cast<int2*>(z.darr)[base] = make_int2(slot, r);
 #else
             ++z.dout[co];
-            z.drnk[slot] = z.dinc[cn]++;
+            const int j = (*z.darrN)++;
+            z.darr[2 * (size_t)j] = slot;
+            z.darr[2 * (size_t)j + 1] = z.dinc[cn]++;
 #endif
         }
     }
@@ -2291,13 +2302,11 @@ ZHD void zone_setup(Z& z, const ZoneIn& in, int lane, int nl) {
  * rounds of global loads: a column's cells are one run of the binning, so
  * wavefront 0 takes the columns' starts and lengths (their prefix sum gives
  * the local indices) while the others take the ring; then every cell's run
- * follows from its start and its column's.  The barrier in between and the
- * one the caller takes after it are workgroup barriers; zone_setup_all_owned
- * gives the zone's allOwned after the second. */
+ * follows from its start and its column's (zone_setup_cells).  The caller
+ * takes a workgroup barrier after each; sh->P holds the particle count after
+ * the first, zone_setup_all_owned the zone's allOwned after the second. */
 template <class Z>
-ZHD void zone_setup_mw(Z& z, const ZoneIn& in, int wave, int lane) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    typedef typename Z::idx_t IT;
+ZHD void zone_setup_columns(Z& z, int wave, int lane) {
     if (wave == 0) {
         int base = 0;
         for (int b0 = 0; b0 < z.zw; b0 += 64) {
@@ -2325,7 +2334,10 @@ ZHD void zone_setup_mw(Z& z, const ZoneIn& in, int wave, int lane) {
         const int nh = halo_size(z);
         for (int h = (wave - 1) * 64 + lane; h < nh; h += 192) setup_halo(z, h);
     }
-    __syncthreads();
+}
+template <class Z>
+ZHD void zone_setup_cells(Z& z, const ZoneIn& in, int wave, int lane) {
+    typedef typename Z::idx_t IT;
     bool mixed = false;
     for (int lc = wave * 64 + lane; lc < z.C; lc += 256) {
         const int col = lc_col(z, lc), gc = lc_gc(z, lc);
@@ -2341,7 +2353,6 @@ ZHD void zone_setup_mw(Z& z, const ZoneIn& in, int wave, int lane) {
         z.k0[lc] = (IT)k0;
     }
     if (wave_ballot(mixed) != 0ull && lane == 0) z.sh->mixed = 1;
-#endif
 }
 template <class Z>
 ZHD int zone_setup_all_owned(const Z& z) {
@@ -2622,7 +2633,8 @@ ZHD void zone_init(ZoneCtxT<IT>& z, const ZoneIn& in, ZoneRect r, int zid, uint6
     z.dcid = in.dcid;
     z.dout = in.dout;
     z.dinc = in.dinc;
-    z.drnk = in.drnk;
+    z.darr = in.darr;
+    z.darrN = in.darrN;
     z.cellOff = in.cellOff;
     z.dgCell = in.dgCell;
     z.dgCnt = in.dgCnt;
