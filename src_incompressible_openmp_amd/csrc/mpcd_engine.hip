@@ -300,57 +300,38 @@ __global__ void __launch_bounds__(TPB) k_scan_add_prefix(int* __restrict__ out, 
     if (i < m) out[i] += s[0];
 }
 
-/* The whole scan by one block, for up to ONE_TILES x 4096 entries: every load
- * is issued before the first sum, so it takes about what one of the two
- * kernels above does, whose launches a small grid's step otherwise pays four
- * times (4.4 us each; 9.0 -> 5 us per scan at 2,501 and 32,769 entries). */
-constexpr int ONE_TPB = 1024, ONE_TILES = 9;
+/* The whole scan by one block of 1024 threads, four entries each: a grid of
+ * up to 4,095 cells pays one launch instead of two, four times a step (at
+ * 2,501 entries 4.5 us against 8.9; with nine entries' loads per thread a
+ * block of its own took 29 us at 32,769 entries against 9.7, so larger scans
+ * keep the two kernels). */
+constexpr int ONE_TPB = 1024, ONE_MAX = 4 * ONE_TPB;
 __global__ void __launch_bounds__(ONE_TPB) k_scan_one(const int* __restrict__ in, int m, int* __restrict__ out,
                                                       const int* __restrict__ in2, int* __restrict__ zero,
                                                       const int* __restrict__ sub) {
-    __shared__ int ws[ONE_TILES][ONE_TPB / 64];
-    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int v[ONE_TILES][4], incl[ONE_TILES];
-#pragma unroll
-    for (int t = 0; t < ONE_TILES; ++t) {
-        const int b = t * 4 * ONE_TPB + 4 * tid;
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            v[t][k] = b + k < m ? in[b + k] + (in2 ? in2[b + k] : 0) - (sub ? sub[b + k] : 0) : 0;
+    __shared__ int ws[ONE_TPB / 64];
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6, b = 4 * tid;
+    int v[4], x = 0;
+    for (int k = 0; k < 4; ++k) {
+        v[k] = b + k < m ? in[b + k] + (in2 ? in2[b + k] : 0) - (sub ? sub[b + k] : 0) : 0;
+        x += v[k];
     }
-#pragma unroll
-    for (int t = 0; t < ONE_TILES; ++t) {
-        int x = v[t][0] + v[t][1] + v[t][2] + v[t][3];
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        incl[t] = x;
-        if (lane == 63) ws[t][wave] = x;
+    const int own = x;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
     }
     __syncthreads();
-    int base = 0;
-#pragma unroll
-    for (int t = 0; t < ONE_TILES; ++t) {
-        int pre = 0, tot = 0;
-#pragma unroll
-        for (int w = 0; w < ONE_TPB / 64; ++w) {
-            const int x = ws[t][w];
-            pre += w < wave ? x : 0;
-            tot += x;
-        }
-        int run = base + pre + incl[t] - (v[t][0] + v[t][1] + v[t][2] + v[t][3]);
-        base += tot;
-        const int b = t * 4 * ONE_TPB + 4 * tid;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (b + k < m) {
-                out[b + k] = run;
-                if (zero) zero[b + k] = 0;
-            }
-            run += v[t][k];
+    if (lane == 63) ws[wave] = x;
+    int run = x - own;
+    for (int w = 0; w < ONE_TPB / 64; ++w) run += w < wave ? ws[w] : 0;
+    for (int k = 0; k < 4; ++k) {
+        if (b + k < m) {
+            out[b + k] = run;
+            if (zero) zero[b + k] = 0;
         }
     }
+        run += v[k];
 }
 
 /* Scatter (pid, slot) keys into their cell's run: one returning atomic per
@@ -1542,16 +1523,13 @@ __device__ __forceinline__ double pdrive_at(const Geom& g, const double* __restr
     return v;
 }
 
-/* The closure's grids of one cell per thread: the repair and its block
- * partials of (num, den), pdrive, and duEOS = -(dt/rhoT) * grad(pdrive) *
- * betaEOS (liquid_closure.cpp:243-295, :424-430), whose neighbours' pdrive is
- * taken again here rather than in a kernel of its own; clear0, clear1 (Nc + 1
- * counters each, or nullptr) are cleared on the way, also when gated off. */
-__global__ void __launch_bounds__(TPB) k_closure_grids(ClosureArgs a, Geom g, const double* __restrict__ raw,
-                                                       const int* __restrict__ mask, double blend, int anyMask,
-                                                       double dtOverRho, double betaEOS, double* __restrict__ pd,
-                                                       double* __restrict__ ex, double* __restrict__ ey,
-                                                       int* __restrict__ clear0, int* __restrict__ clear1) {
+/* The closure's first grids, one cell per thread: the repair with its block
+ * partials of (num, den), and pdrive; clear0, clear1 (Nc + 1 counters each,
+ * or nullptr) are cleared on the way, also when gated off. */
+__global__ void __launch_bounds__(TPB) k_closure_repair(ClosureArgs a, Geom g, const double* __restrict__ raw,
+                                                        const int* __restrict__ mask, double blend, int anyMask,
+                                                        double* __restrict__ pd, int* __restrict__ clear0,
+                                                        int* __restrict__ clear1) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (clear0 && c < a.Nc) {
         clear0[c] = 0;
@@ -1569,25 +1547,10 @@ __global__ void __launch_bounds__(TPB) k_closure_grids(ClosureArgs a, Geom g, co
         const double ay = (a.refPy[c] - a.redPy[c]) / a.gamma;
         a.duRX[c] = ax;
         a.duRY[c] = ay;
-        const double ux = a.redUx[c] - a.refUx[c], uy = a.redUy[c] - a.refUy[c];
-        num = -(ux * ax + uy * ay);
+        const double ex = a.redUx[c] - a.refUx[c], ey = a.redUy[c] - a.refUy[c];
+        num = -(ex * ax + ey * ay);
         den = ax * ax + ay * ay;
-        const int ix = c / g.Ny, iy = c - ix * g.Ny;
-        const double dx = g.dxc, dy = g.dyc;
-        auto p = [&](int jx, int jy) { return pdrive_at(g, raw, mask, blend, anyMask, jy + g.Ny * jx); };
-        const double pc = p(ix, iy);
-        pd[c] = pc;
-        double gx, gy;
-        if (g.perx) gx = (p(wrapi(ix + 1, g.Nx), iy) - p(wrapi(ix - 1, g.Nx), iy)) / (2.0 * dx);
-        else if (ix == 0) gx = (p(ix + 1, iy) - pc) / dx;
-        else if (ix == g.Nx - 1) gx = (pc - p(ix - 1, iy)) / dx;
-        else gx = (p(ix + 1, iy) - p(ix - 1, iy)) / (2.0 * dx);
-        if (g.pery) gy = (p(ix, wrapi(iy + 1, g.Ny)) - p(ix, wrapi(iy - 1, g.Ny))) / (2.0 * dy);
-        else if (iy == 0) gy = (p(ix, iy + 1) - pc) / dy;
-        else if (iy == g.Ny - 1) gy = (pc - p(ix, iy - 1)) / dy;
-        else gy = (p(ix, iy + 1) - p(ix, iy - 1)) / (2.0 * dy);
-        ex[c] = -dtOverRho * gx * betaEOS;
-        ey[c] = -dtOverRho * gy * betaEOS;
+        pd[c] = pdrive_at(g, raw, mask, blend, anyMask, c);
     }
     s0[threadIdx.x] = num;
     s1[threadIdx.x] = den;
@@ -1621,12 +1584,34 @@ __device__ inline void beta_from_sums(double* scal, int useOptimal, double betaR
     scal[3] = app;
 }
 
-/* the repair sums and beta in one block (thread 0 wrote the sums) */
-__global__ void __launch_bounds__(TPB) k_reduce_beta(const double* __restrict__ part, int np, double* scal,
-                                                     int useOptimal, double betaRepair, const int* gate = nullptr) {
+/* duEOS = -(dt/rhoT) * grad(pdrive) * betaEOS (liquid_closure.cpp:243-295, :424-430),
+ * and in one more block the repair sums and beta, which nothing here waits
+ * for */
+__global__ void __launch_bounds__(TPB) k_eos_beta(Geom g, const double* __restrict__ p, double dtOverRho, double betaEOS,
+                                                  double* __restrict__ ex, double* __restrict__ ey,
+                                                  const double* __restrict__ part, int np, double* scal, int useOptimal,
+                                                  double betaRepair, const int* gate) {
     if (gated_off(gate)) return;
-    reduce_parts_block(part, np, 2, scal);
-    if (threadIdx.x == 0) beta_from_sums(scal, useOptimal, betaRepair);
+    if (blockIdx.x == gridDim.x - 1) {
+        reduce_parts_block(part, np, 2, scal);
+        if (threadIdx.x == 0) beta_from_sums(scal, useOptimal, betaRepair);
+        return;
+    }
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= g.Nc) return;
+    const int ix = c / g.Ny, iy = c - ix * g.Ny;
+    const double dx = g.dxc, dy = g.dyc;
+    double gx, gy;
+    if (g.perx) gx = (p[iy + g.Ny * wrapi(ix + 1, g.Nx)] - p[iy + g.Ny * wrapi(ix - 1, g.Nx)]) / (2.0 * dx);
+    else if (ix == 0) gx = (p[iy + g.Ny * (ix + 1)] - p[c]) / dx;
+    else if (ix == g.Nx - 1) gx = (p[c] - p[iy + g.Ny * (ix - 1)]) / dx;
+    else gx = (p[iy + g.Ny * (ix + 1)] - p[iy + g.Ny * (ix - 1)]) / (2.0 * dx);
+    if (g.pery) gy = (p[wrapi(iy + 1, g.Ny) + g.Ny * ix] - p[wrapi(iy - 1, g.Ny) + g.Ny * ix]) / (2.0 * dy);
+    else if (iy == 0) gy = (p[(iy + 1) + g.Ny * ix] - p[c]) / dy;
+    else if (iy == g.Ny - 1) gy = (p[c] - p[(iy - 1) + g.Ny * ix]) / dy;
+    else gy = (p[(iy + 1) + g.Ny * ix] - p[(iy - 1) + g.Ny * ix]) / (2.0 * dy);
+    ex[c] = -dtOverRho * gx * betaEOS;
+    ey[c] = -dtOverRho * gy * betaEOS;
 }
 
 /* The closure's kick: repair (scaled by beta) then EOS correction. */
@@ -2429,7 +2414,7 @@ struct mpcd_gpu_sim {
 
     /* exclusive scan of in + in2 - sub over m entries; zero cleared beside it */
     void scan(const int* in, int m, int* out, const int* in2, int* zero, const int* sub) {
-        if (m <= ONE_TILES * 4 * ONE_TPB) {
+        if (m <= ONE_MAX) {
             hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(ONE_TPB), 0, stream, in, m, out, in2, zero, sub);
             return;
         }
@@ -2833,11 +2818,11 @@ struct mpcd_gpu_sim {
         const int nbc = (int)nblk(Nc);
         /* the counters the fused kick fills are cleared beside */
         const bool clr = fuseNext >= 0;
-        hipLaunchKernelGGL(k_closure_grids, dim3(nbc), dim3(TPB), 0, stream, ca, g, pdriveRaw, mask,
-                           p.smoothPdriveInterzoneBlend, anyMask, p.dt / rho_target(), p.betaEOS, pdrive, duEX, duEY,
-                           clr ? bin.cntS : (int*)nullptr, clr ? bin.cnt : (int*)nullptr);
-        hipLaunchKernelGGL(k_reduce_beta, dim3(1), dim3(TPB), 0, stream, part, nbc, scal, p.useOptimalBetaRepair,
-                           p.betaRepair, gate);
+        hipLaunchKernelGGL(k_closure_repair, dim3(nbc), dim3(TPB), 0, stream, ca, g, pdriveRaw, mask,
+                           p.smoothPdriveInterzoneBlend, anyMask, pdrive, clr ? bin.cntS : (int*)nullptr,
+                           clr ? bin.cnt : (int*)nullptr);
+        hipLaunchKernelGGL(k_eos_beta, dim3(nbc + 1), dim3(TPB), 0, stream, g, pdrive, p.dt / rho_target(), p.betaEOS,
+                           duEX, duEY, part, nbc, scal, p.useOptimalBetaRepair, p.betaRepair, gate);
         check_launch();
     }
 
