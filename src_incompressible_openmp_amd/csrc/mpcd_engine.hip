@@ -321,8 +321,8 @@ __global__ void __launch_bounds__(ONE_TPB) k_scan_one(const int* __restrict__ in
         const int y = __shfl_up(x, o, 64);
         if (lane >= o) x += y;
     }
-    __syncthreads();
     if (lane == 63) ws[wave] = x;
+    __syncthreads();
     int run = x - own;
     for (int w = 0; w < ONE_TPB / 64; ++w) run += w < wave ? ws[w] : 0;
     for (int k = 0; k < 4; ++k) {
@@ -330,8 +330,8 @@ __global__ void __launch_bounds__(ONE_TPB) k_scan_one(const int* __restrict__ in
             out[b + k] = run;
             if (zero) zero[b + k] = 0;
         }
-    }
         run += v[k];
+    }
 }
 
 /* Scatter (pid, slot) keys into their cell's run: one returning atomic per
