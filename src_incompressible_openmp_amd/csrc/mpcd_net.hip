@@ -72,20 +72,40 @@ struct Grid {
     long long tpitch; /* pitch of the transposed copies: total rounded up to 16 */
 };
 
-/* neighbour (dx, dy) of cell index q, or -1 outside the padded domain */
-__device__ inline long long neighbour(const Grid& g, long long q, int dx, int dy) {
-    const long long s = q / g.Nc;
-    const int c = (int)(q - s * g.Nc);
-    int jx = c / g.Ny + dx, jy = c % g.Ny + dy;
-    if (jx < 0 || jx >= g.Nx) {
-        if (!g.perx) return -1;
-        jx = (jx + g.Nx) % g.Nx;
+/* The place of cell index q: its sample's first cell, and its column and row.
+ * Taken once per cell; the nine taps' neighbours follow by additions (a
+ * division per tap, in 64 bits, was most of the convolutions' time: 60 us per
+ * 32 -> 32 layer of 524,288 cells, whose traffic takes 28). */
+struct CellAt {
+    long long s0; /* -1: no cell */
+    int ix, iy;
+};
+__device__ inline CellAt cell_at(const Grid& g, long long q) {
+    CellAt p{-1, 0, 0};
+    if (q >= g.total) return p;
+    int c;
+    if (g.total <= 0x7fffffffLL) {
+        const unsigned qq = (unsigned)q, s = g.B > 1 ? qq / (unsigned)g.Nc : 0u;
+        p.s0 = (long long)(s * (unsigned)g.Nc);
+        c = (int)(qq - s * (unsigned)g.Nc);
+    } else {
+        const long long s = q / g.Nc;
+        p.s0 = s * g.Nc;
+        c = (int)(q - p.s0);
     }
-    if (jy < 0 || jy >= g.Ny) {
-        if (!g.pery) return -1;
-        jy = (jy + g.Ny) % g.Ny;
-    }
-    return s * g.Nc + jy + (long long)g.Ny * jx;
+    p.ix = (int)((unsigned)c / (unsigned)g.Ny);
+    p.iy = c - p.ix * g.Ny;
+    return p;
+}
+/* the cell at (dx, dy) of p, |dx|, |dy| <= 1, or -1 outside the padded domain */
+__device__ inline long long neighbour(const Grid& g, const CellAt& p, int dx, int dy) {
+    int jx = p.ix + dx, jy = p.iy + dy;
+    bool in = p.s0 >= 0;
+    if (g.perx) jx = jx < 0 ? jx + g.Nx : (jx >= g.Nx ? jx - g.Nx : jx);
+    else in = in & (jx >= 0) & (jx < g.Nx);
+    if (g.pery) jy = jy < 0 ? jy + g.Ny : (jy >= g.Ny ? jy - g.Ny : jy);
+    else in = in & (jy >= 0) & (jy < g.Ny);
+    return in ? p.s0 + jy + (long long)g.Ny * jx : -1;
 }
 
 enum { EPI_RELU = 0, EPI_LINEAR = 1, EPI_MASK = 2 };
@@ -124,8 +144,7 @@ __global__ void __launch_bounds__(NTPB) k_conv(ConvArgs a) {
     const Grid& g = a.g;
     for (long long t0 = (long long)blockIdx.x * 64; t0 < g.total; t0 += (long long)gridDim.x * 64) {
         const long long cell0 = t0 + 16 * wv;
-        const long long q = cell0 + row;
-        const bool valid = q < g.total;
+        const CellAt at = cell_at(g, cell0 + row);
         f32x4 acc[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -133,10 +152,8 @@ __global__ void __launch_bounds__(NTPB) k_conv(ConvArgs a) {
         for (int s = 0; s < NS; ++s) {
             const int gblk = 4 * s + kb, tap = gblk / BPT, chb = gblk % BPT;
             bf16x8 av = zero8();
-            if (valid && tap < 9) {
-                const long long nbq = neighbour(g, q, tap / 3 - 1, tap % 3 - 1);
-                if (nbq >= 0) av = ld8(a.in + nbq * CIN + chb * 8);
-            }
+            const long long nbq = neighbour(g, at, tap / 3 - 1, tap % 3 - 1);
+            if (tap < 9 && nbq >= 0) av = ld8(a.in + nbq * CIN + chb * 8);
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bw[s][nb], acc[nb], 0, 0, 0);
         }
@@ -220,34 +237,42 @@ __global__ void __launch_bounds__(NTPB) k_conv_wgrad(Grid g, const u16* __restri
     f32x4 acc[9];
 #pragma unroll
     for (int t = 0; t < 9; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float bsum = 0.0f; /* threads 0..31: co */
+    static_assert(NTPB % WG_PITCH == 0 && NTPB == 8 * 32, "one cell per thread, eight threads per bias");
+    float bsum = 0.0f; /* threads 8 co ..: co's */
     const long long nblkTot = (g.total + WG_PITCH - 1) / WG_PITCH;
     for (long long bk = blockIdx.x; bk < nblkTot; bk += gridDim.x) {
         const long long c0 = bk * WG_PITCH;
-        for (int e = threadIdx.x; e < 32 * WG_PITCH; e += NTPB) {
-            const int co = e / WG_PITCH, k = e % WG_PITCH;
-            const long long q = c0 + k;
+        /* thread t holds cell t % WG_PITCH of the tile: its place once, its
+         * neighbour once per tap, whatever the channel */
+        const int k = (int)threadIdx.x % WG_PITCH, r0 = (int)threadIdx.x / WG_PITCH;
+        const long long q = c0 + k;
+        const CellAt at = cell_at(g, q);
+#pragma unroll
+        for (int j = 0; j < 32 * WG_PITCH / NTPB; ++j) {
+            const int co = r0 + (NTPB / WG_PITCH) * j;
             sg[co][k] = (co < gRows && q < g.total) ? gT[(size_t)co * g.tpitch + q] : (u16)0;
         }
         __syncthreads();
-        if (threadIdx.x < 32) {
+        {
+            /* eight threads per output channel, sixteen cells each */
+            const int co = (int)threadIdx.x >> 3, part8 = (int)threadIdx.x & 7;
             float s = 0.0f;
-            for (int k = 0; k < WG_PITCH; ++k) s += bf2f(sg[threadIdx.x][k]);
+            for (int u = 0; u < WG_PITCH / 8; ++u) s += bf2f(sg[co][part8 * (WG_PITCH / 8) + u]);
+            s += __shfl_xor(s, 1, 64);
+            s += __shfl_xor(s, 2, 64);
+            s += __shfl_xor(s, 4, 64);
             bsum += s;
         }
 #pragma unroll
         for (int tap = 0; tap < 9; ++tap) {
             const int dx = tap / 3 - 1, dy = tap % 3 - 1;
-            for (int e = threadIdx.x; e < CIN * WG_PITCH; e += NTPB) {
-                const int ci = e / WG_PITCH, k = e % WG_PITCH;
-                const long long q = c0 + k;
-                u16 v = 0;
-                if (q < g.total) {
-                    const long long nq = neighbour(g, q, dx, dy);
-                    if (nq >= 0) v = inT[(size_t)ci * g.tpitch + nq];
-                }
-                si[ci][k] = v;
-            }
+            const long long nq = neighbour(g, at, dx, dy);
+            u16 v[CIN * WG_PITCH / NTPB];
+#pragma unroll
+            for (int j = 0; j < CIN * WG_PITCH / NTPB; ++j)
+                v[j] = nq >= 0 ? inT[(size_t)(r0 + (NTPB / WG_PITCH) * j) * g.tpitch + nq] : (u16)0;
+#pragma unroll
+            for (int j = 0; j < CIN * WG_PITCH / NTPB; ++j) si[r0 + (NTPB / WG_PITCH) * j][k] = v[j];
             __syncthreads();
             if (active) {
 #pragma unroll
@@ -273,24 +298,49 @@ __global__ void __launch_bounds__(NTPB) k_conv_wgrad(Grid g, const u16* __restri
                 pb[((size_t)co * 9 + tap) * 32 + ci] = acc[tap][r];
             }
     }
-    if (threadIdx.x < 32) bpart[(size_t)blockIdx.x * 32 + threadIdx.x] = bsum;
+    if ((threadIdx.x & 7) == 0) bpart[(size_t)blockIdx.x * 32 + (threadIdx.x >> 3)] = bsum;
 }
 
-/* Sums the per-block partials in block order into the flat gradient of
- * one layer (W[co][tap][ci] for the real channels, then b[co]). */
-__global__ void k_wgrad_reduce(const float* __restrict__ part, const float* __restrict__ bpart, int nparts, int co,
-                               int ci, double* __restrict__ grad) {
+/* Sums the per-block partials in a fixed order into the flat gradient of one
+ * layer (W[co][tap][ci] for the real channels, then b[co]): 64 entries per
+ * block, sixteen threads per entry, each its sixteenth of the partials in
+ * order, then the sixteen in order (one thread per entry walked up to 512
+ * partials alone: 124 us per layer). */
+constexpr int WR_E = 64, WR_G = 16;
+__global__ void __launch_bounds__(WR_E * WR_G) k_wgrad_reduce(const float* __restrict__ part,
+                                                              const float* __restrict__ bpart, int nparts, int co, int ci,
+                                                              double* __restrict__ grad) {
+    __shared__ double sh[WR_G][WR_E];
     const int nW = co * 9 * ci;
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nW + co) return;
+    const int e = blockIdx.x * WR_E + (int)threadIdx.x % WR_E, gi = (int)threadIdx.x / WR_E;
     double s = 0.0;
-    if (e < nW) {
-        const int o = e / (9 * ci), t = (e / ci) % 9, i = e % ci;
-        for (int b = 0; b < nparts; ++b) s += (double)part[(size_t)b * (32 * 9 * 32) + ((size_t)o * 9 + t) * 32 + i];
-    } else {
-        for (int b = 0; b < nparts; ++b) s += (double)bpart[(size_t)b * 32 + (e - nW)];
+    if (e < nW + co) {
+        const int per = (nparts + WR_G - 1) / WR_G, b0 = gi * per, b1 = min(nparts, b0 + per);
+        const float* src;
+        size_t stride;
+        if (e < nW) {
+            const int o = e / (9 * ci), t = (e / ci) % 9, i = e % ci;
+            src = part + ((size_t)o * 9 + t) * 32 + i;
+            stride = 32 * 9 * 32;
+        } else {
+            src = bpart + (e - nW);
+            stride = 32;
+        }
+        for (int b = b0; b < b1; b += 8) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = b + u < b1 ? src[(size_t)(b + u) * stride] : 0.0f;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += (double)v[u];
+        }
     }
-    grad[e] = s;
+    sh[gi][threadIdx.x % WR_E] = s;
+    __syncthreads();
+    if (gi == 0 && e < nW + co) {
+        double t = 0.0;
+        for (int k = 0; k < WR_G; ++k) t += sh[k][threadIdx.x];
+        grad[e] = t;
+    }
 }
 
 /* features (float [cell][4]) -> bfloat16 [cell][8] and its transpose */
@@ -554,8 +604,8 @@ struct mpcd_gpu_net {
                 hipLaunchKernelGGL((k_conv_wgrad<32, 2>), dim3(np), dim3(NTPB), 0, stream, g, inT, gT, gRows, part,
                                    bpart);
             const int nW = CH[l + 1] * 9 * CH[l] + CH[l + 1];
-            hipLaunchKernelGGL(k_wgrad_reduce, dim3(nb(nW)), dim3(NTPB), 0, stream, part, bpart, (int)np, CH[l + 1],
-                               CH[l], grad + offset(l));
+            hipLaunchKernelGGL(k_wgrad_reduce, dim3(nb(nW, WR_E)), dim3(WR_E * WR_G), 0, stream, part, bpart, (int)np,
+                               CH[l + 1], CH[l], grad + offset(l));
             if (l == 0) break;
             /* input gradient of layer l, masked by the forward activation */
             ConvArgs c{};
