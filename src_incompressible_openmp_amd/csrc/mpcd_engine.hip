@@ -23,6 +23,7 @@
 #include "mpcd_core.h"
 #include "mpcd_hip_util.h"
 #include "mpcd_host.h"
+#include "mpcd_transfer.h"
 
 using namespace mpcdk;
 
@@ -2042,6 +2043,7 @@ struct mpcd_gpu_sim {
     Geom g{};
     int n = 0, Nc = 0;
     hipStream_t stream = nullptr;
+    HostCopy copy;
     double *x = nullptr, *y = nullptr, *vx = nullptr, *vy = nullptr;
     double *vx2 = nullptr, *vy2 = nullptr; /* zone-pass output velocities (swapped after each pass) */
     double *x2 = nullptr, *y2 = nullptr;   /* reorder targets */
@@ -2370,15 +2372,14 @@ struct mpcd_gpu_sim {
 
     /* ---- transfers ---- */
     void upload_xy(const double* h, double* dx_, double* dy_) {
-        HIP_OK(hipMemcpyAsync(stage, h, 2 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, stream));
+        copy.upload(stage, h, 2 * (size_t)n * sizeof(double), stream);
         hipLaunchKernelGGL(k_deinterleave, dim3(nblk(n)), dim3(TPB), 0, stream, stage, n, dx_, dy_);
         check_launch();
     }
     void download_xy(const double* dx_, const double* dy_, double* h) {
         hipLaunchKernelGGL(k_interleave, dim3(nblk(n)), dim3(TPB), 0, stream, dx_, dy_, pid, n, stage);
         check_launch();
-        HIP_OK(hipMemcpyAsync(h, stage, 2 * (size_t)n * sizeof(double), hipMemcpyDeviceToHost, stream));
-        HIP_OK(hipStreamSynchronize(stream));
+        copy.download(h, stage, 2 * (size_t)n * sizeof(double), stream);
     }
     /* Slots are reset to particle-id order (pid = iota).  An array the
      * caller does not upload (null) is kept: it is first scattered from the
@@ -2787,8 +2788,7 @@ struct mpcd_gpu_sim {
         hipLaunchKernelGGL(k_repaired_velocity, dim3(nblk(n)), dim3(TPB), 0, stream, g, x2, y2, vx2, vy2, pid2, duRX,
                            duRY, scal, stage);
         check_launch();
-        HIP_OK(hipMemcpyAsync(hv, stage, 2 * (size_t)n * sizeof(double), hipMemcpyDeviceToHost, stream));
-        HIP_OK(hipStreamSynchronize(stream));
+        copy.download(hv, stage, 2 * (size_t)n * sizeof(double), stream);
     }
 
     ClosureArgs closure_args() {
@@ -3258,7 +3258,7 @@ int mpcd_gpu_sim_cell_fields(mpcd_gpu_sim* s, double rhoTarget, mpcd_cell_fields
         if (s->streamed >= 0) throw ApiError(MPCD_E_INVALID, "internal: a fused stream was left unused");
         s->fields_current();
         const size_t C = (size_t)s->Nc;
-        if (out->N) HIP_OK(hipMemcpyAsync(out->N, s->outN, C * sizeof(int), hipMemcpyDeviceToHost, s->stream));
+        if (out->N) s->copy.download(out->N, s->outN, C * sizeof(int), s->stream);
         double* hs[9] = {out->Ux, out->Uy, out->Px, out->Py, out->T, out->rho, out->Pkin, out->Pvir, out->P};
         for (int k = 0; k < 9; ++k)
             if (hs[k])
@@ -3359,8 +3359,7 @@ int mpcd_gpu_srd_cell_id_with_random_shift(const mpcd_params* p, const double* x
         hipLaunchKernelGGL(k_shift_cells, dim3(nblk(s.n)), dim3(TPB), 0, s.stream, s.g, s.x, s.y, sx, sy, s.xmax,
                            s.ymax, s.cid);
         s.check_launch();
-        HIP_OK(hipMemcpyAsync(cid, s.cid, (size_t)s.n * sizeof(int), hipMemcpyDeviceToHost, s.stream));
-        HIP_OK(hipStreamSynchronize(s.stream));
+        s.copy.download(cid, s.cid, (size_t)s.n * sizeof(int), s.stream);
     });
 }
 
@@ -3371,7 +3370,7 @@ int mpcd_gpu_srd_collision_step(const mpcd_params* p, double* v, const int32_t* 
             if (cid[i] < 0 || cid[i] >= p->Nc) throw ApiError(MPCD_E_INVALID, "srd_collision_step: cell id out of range");
         auto& s = scratch_sim(*p);
         s.set_state(nullptr, v);
-        HIP_OK(hipMemcpyAsync(s.cid, cid, (size_t)s.n * sizeof(int), hipMemcpyHostToDevice, s.stream));
+        s.copy.upload(s.cid, cid, (size_t)s.n * sizeof(int), s.stream);
         s.bin_cells(s.cid);
         s.collide(rng_seed);
         s.get_state(nullptr, v);

@@ -431,6 +431,7 @@ __global__ void __launch_bounds__(TPB) k_ens_flow_acc(const EnsRep* __restrict__
 /* ===================================================================== */
 
 struct mpcd_gpu_ensemble {
+    HostCopy copy;
     int R = 0, N = 0, C = 0, B = 0; /* replicas, particles, cells, closure blocks */
     int Z[2] = {0, 0};
     std::vector<mpcd_params> prm;
@@ -967,12 +968,11 @@ struct mpcd_gpu_ensemble {
         check_replica(r);
         const int n = prm[(size_t)r].n, o = hreps[(size_t)r].poff;
         if (hx) {
-            HIP_OK(hipMemcpyAsync(stage, hx, 2 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, stream));
+            copy.upload(stage, hx, 2 * (size_t)n * sizeof(double), stream);
             hipLaunchKernelGGL(k_deinterleave, dim3(nblk(n)), dim3(TPB), 0, stream, stage, n, x + o, y + o);
         }
         if (hv) {
-            HIP_OK(hipMemcpyAsync(stage + (hx ? 0 : 0), hv, 2 * (size_t)n * sizeof(double), hipMemcpyHostToDevice,
-                                  stream));
+            copy.upload(stage, hv, 2 * (size_t)n * sizeof(double), stream);
             hipLaunchKernelGGL(k_deinterleave, dim3(nblk(n)), dim3(TPB), 0, stream, stage, n, vx + o, vy + o);
         }
         hipLaunchKernelGGL(k_iota, dim3(nblk(n)), dim3(TPB), 0, stream, pid + o, n);
@@ -990,8 +990,7 @@ struct mpcd_gpu_ensemble {
             hipLaunchKernelGGL(k_interleave, dim3(nblk(n)), dim3(TPB), 0, stream, src[k][0], src[k][1], pid + o, n,
                                stage);
             check_launch();
-            HIP_OK(hipMemcpyAsync(dst[k], stage, 2 * (size_t)n * sizeof(double), hipMemcpyDeviceToHost, stream));
-            HIP_OK(hipStreamSynchronize(stream));
+            copy.download(dst[k], stage, 2 * (size_t)n * sizeof(double), stream);
         }
     }
 };

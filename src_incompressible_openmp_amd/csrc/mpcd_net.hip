@@ -30,6 +30,7 @@
 
 #include "mpcd_gpu.h"
 #include "mpcd_hip_util.h"
+#include "mpcd_transfer.h"
 #include "mpcd_rng.h"
 
 using namespace mpcdk;
@@ -435,6 +436,7 @@ struct mpcd_gpu_net {
     Grid g{};
     int maxB = 0;
     hipStream_t stream = nullptr;
+    HostCopy copy;
     int nParts = 0;
     /* parameters */
     double *theta = nullptr, *mom = nullptr, *vel = nullptr, *grad = nullptr;
@@ -703,12 +705,9 @@ int mpcd_gpu_net_forward(mpcd_gpu_net* net, const float* feat, int B, float* out
     return guarded([&] {
         if (!net || !feat || !out) throw ApiError(MPCD_E_INVALID, "null argument");
         net->set_batch(B);
-        HIP_OK(hipMemcpyAsync(net->feat, feat, (size_t)net->g.total * 4 * sizeof(float), hipMemcpyHostToDevice,
-                              net->stream));
+        net->copy.upload(net->feat, feat, (size_t)net->g.total * 4 * sizeof(float), net->stream);
         net->forward(false);
-        HIP_OK(hipMemcpyAsync(out, net->pred, (size_t)net->g.total * 2 * sizeof(float), hipMemcpyDeviceToHost,
-                              net->stream));
-        HIP_OK(hipStreamSynchronize(net->stream));
+        net->copy.download(out, net->pred, (size_t)net->g.total * 2 * sizeof(float), net->stream);
     });
 }
 
@@ -717,10 +716,8 @@ int mpcd_gpu_net_loss_grad(mpcd_gpu_net* net, const float* feat, const float* ta
     return guarded([&] {
         if (!net || !feat || !target) throw ApiError(MPCD_E_INVALID, "null argument");
         net->set_batch(B);
-        HIP_OK(hipMemcpyAsync(net->feat, feat, (size_t)net->g.total * 4 * sizeof(float), hipMemcpyHostToDevice,
-                              net->stream));
-        HIP_OK(hipMemcpyAsync(net->tgt, target, (size_t)net->g.total * 2 * sizeof(float), hipMemcpyHostToDevice,
-                              net->stream));
+        net->copy.upload(net->feat, feat, (size_t)net->g.total * 4 * sizeof(float), net->stream);
+        net->copy.upload(net->tgt, target, (size_t)net->g.total * 2 * sizeof(float), net->stream);
         net->forward(true);
         net->backward_enqueue();
         const double l = net->read_loss();
@@ -757,10 +754,8 @@ int mpcd_gpu_net_train(mpcd_gpu_net* net, const float* feat, const float* target
             net->setT = dalloc<float>((size_t)nSamples * nc * 2);
             net->setN = nSamples;
         }
-        HIP_OK(hipMemcpyAsync(net->setF, feat, (size_t)nSamples * nc * 4 * sizeof(float), hipMemcpyHostToDevice,
-                              net->stream));
-        HIP_OK(hipMemcpyAsync(net->setT, target, (size_t)nSamples * nc * 2 * sizeof(float), hipMemcpyHostToDevice,
-                              net->stream));
+        net->copy.upload(net->setF, feat, (size_t)nSamples * nc * 4 * sizeof(float), net->stream);
+        net->copy.upload(net->setT, target, (size_t)nSamples * nc * 2 * sizeof(float), net->stream);
         for (int it = 0; it < iters; ++it) {
             /* mini-batch of samples drawn with the counter generator */
             for (int b = 0; b < batch; ++b) {

@@ -79,11 +79,9 @@ class Net:
         f = _f32(feat, 4).reshape(-1, self.Nc, 4)
         out = np.zeros((f.shape[0], self.Nc, 2), np.float32)
         for b0 in range(0, f.shape[0], self.max_batch):
-            fb = np.ascontiguousarray(f[b0:b0 + self.max_batch])
-            ob = np.zeros((fb.shape[0], self.Nc, 2), np.float32)
+            fb, ob = f[b0:b0 + self.max_batch], out[b0:b0 + self.max_batch]  # contiguous: whole samples
             gpu._check(_lib().mpcd_gpu_net_forward(self._h, fb.ctypes.data_as(_fp), fb.shape[0],
                                                    ob.ctypes.data_as(_fp)))
-            out[b0:b0 + fb.shape[0]] = ob
         return out
 
     def loss_grad(self, feat: np.ndarray, target: np.ndarray):
