@@ -3102,16 +3102,15 @@ namespace {
 
 /* Scratch of mpcd_gpu_compute_cell_fields_noalloc: a file-scope device
  * array (each GPU the library runs on holds its own copy until the process
- * ends).  Regions, each 256-byte aligned: vx, vy (f64), cid, pid, list
- * (i32) and the sort keys (u64) per particle; counts, starts, cursors (i32)
- * per cell + 1; the scan's tile totals. */
+ * ends).  Regions, each 256-byte aligned: vx, vy (f64), cid, rank, list
+ * (i32) and the sort keys (u64) per particle; counts, starts (i32) per cell
+ * + 1; the scan's tile totals. */
 constexpr size_t NA_N = MPCD_NOALLOC_MAX_PARTICLES, NA_C = (size_t)MPCD_NOALLOC_MAX_CELLS + 1;
 constexpr size_t na_al(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t NA_VX = 0, NA_VY = NA_VX + na_al(8 * NA_N), NA_CID = NA_VY + na_al(8 * NA_N),
-                 NA_PID = NA_CID + na_al(4 * NA_N), NA_LIST = NA_PID + na_al(4 * NA_N),
+                 NA_RANK = NA_CID + na_al(4 * NA_N), NA_LIST = NA_RANK + na_al(4 * NA_N),
                  NA_KEY = NA_LIST + na_al(4 * NA_N), NA_CNT = NA_KEY + na_al(8 * NA_N),
-                 NA_START = NA_CNT + na_al(4 * NA_C), NA_CUR = NA_START + na_al(4 * NA_C),
-                 NA_TILE = NA_CUR + na_al(4 * NA_C),
+                 NA_START = NA_CNT + na_al(4 * NA_C), NA_TILE = NA_START + na_al(4 * NA_C),
                  NA_BYTES = NA_TILE + na_al(4 * ((NA_C + SCAN_TILE - 1) / SCAN_TILE));
 
 static __device__ __align__(256) unsigned char scratch[NA_BYTES];
@@ -3136,10 +3135,47 @@ unsigned char* noalloc_scratch() {
     return g_na_ptr[dev];
 }
 
-/* unshifted cells of interleaved positions (common_grid.cpp:9-19) */
-__global__ void k_cells_xy(Geom g, const double* __restrict__ xy, int* __restrict__ cid) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < g.n) cid[i] = cell_of(g, xy[2 * (size_t)i], xy[2 * (size_t)i + 1]);
+/* The scratch's binning is launch-bound (50x50x10: eleven launches took 60 us,
+ * of which the histogram and the scatter, whose key groups need a caller's
+ * particles in cell order to be few, 34; these six take 25), so one kernel
+ * clears, one does all that is done per particle before the scan, and the
+ * histogram's atomics give each particle its place in the cell's run. */
+__global__ void __launch_bounds__(TPB) k_na_clear(int* __restrict__ cnt, int Nc, double* __restrict__ rhoOut,
+                                                  double rhoTarget) {
+    const int c = blockIdx.x * TPB + threadIdx.x;
+    if (c <= Nc) cnt[c] = 0;
+    if (rhoOut && c < Nc) rhoOut[c] = rhoTarget;
+}
+/* unshifted cells (common_grid.cpp:9-19), ranks in the cells' runs (in no
+ * order: the runs are sorted afterwards) and velocities by component */
+__global__ void __launch_bounds__(TPB) k_na_cells(Geom g, const double* __restrict__ xy, const double* __restrict__ v,
+                                                  int* __restrict__ cid, int* __restrict__ rank,
+                                                  double* __restrict__ vx, double* __restrict__ vy,
+                                                  int* __restrict__ cnt) {
+    const int i = blockIdx.x * TPB + threadIdx.x, lane = __lane_id();
+    const bool in = i < g.n;
+    const size_t j = 2 * (size_t)(in ? i : g.n - 1);
+    const int c = in ? cell_of(g, xy[j], xy[j + 1]) : -1;
+    /* lanes of one cell in a row take one atomic, their first's */
+    const int before = __shfl_up(c, 1, 64);
+    const unsigned long long heads = __ballot(lane == 0 || before != c);
+    const int head = 63 - __clzll((long long)(heads & (~0ull >> (63 - lane))));
+    const unsigned long long later = lane == 63 ? 0ull : heads & (~0ull << (lane + 1));
+    const int end = later ? __ffsll((long long)later) - 1 : 64;
+    int base = 0;
+    if (in && lane == head) base = atomicAdd(&cnt[c], end - head);
+    base = __shfl(base, head, 64);
+    if (!in) return;
+    rank[i] = base + lane - head;
+    vx[i] = v[j];
+    vy[i] = v[j + 1];
+    cid[i] = c;
+}
+__global__ void __launch_bounds__(TPB) k_na_scatter(const int* __restrict__ cid, const int* __restrict__ rank, int n,
+                                                    const int* __restrict__ start,
+                                                    unsigned long long* __restrict__ key) {
+    const int i = blockIdx.x * TPB + threadIdx.x;
+    if (i < n) key[start[cid[i]] + rank[i]] = ((unsigned long long)(unsigned)i << 32) | (unsigned)i;
 }
 
 }  // namespace
@@ -3423,39 +3459,33 @@ int mpcd_gpu_compute_cell_fields_noalloc(const mpcd_params* p, const double* x, 
         double* vx = (double*)(b + NA_VX);
         double* vy = (double*)(b + NA_VY);
         int* cid = (int*)(b + NA_CID);
-        int* pid = (int*)(b + NA_PID);
+        int* rank = (int*)(b + NA_RANK);
         int* list = (int*)(b + NA_LIST);
         unsigned long long* key = (unsigned long long*)(b + NA_KEY);
         int* cnt = (int*)(b + NA_CNT);
         int* start = (int*)(b + NA_START);
-        int* cursor = (int*)(b + NA_CUR);
         int* tileSum = (int*)(b + NA_TILE);
         const int nTiles = (int)((Nc + 1 + SCAN_TILE - 1) / SCAN_TILE);
         /* the scratch keeps the last call's contents: everything read is
-         * written first (counts cleared by a fill kernel, not a memset) */
-        if (n > 0) {
-            hipLaunchKernelGGL(k_deinterleave, dim3(nblk(n)), dim3(TPB), 0, st, v, n, vx, vy);
-            hipLaunchKernelGGL(k_cells_xy, dim3(nblk(n)), dim3(TPB), 0, st, g, x, cid);
-            hipLaunchKernelGGL(k_iota, dim3(nblk(n)), dim3(TPB), 0, st, pid, n);
+         * written first (counts cleared by a kernel, not a memset) */
+        hipLaunchKernelGGL(k_na_clear, dim3(nblk(Nc + 1)), dim3(TPB), 0, st, cnt, Nc, out->rhoTarget, rhoTarget);
+        hipLaunchKernelGGL(k_na_cells, dim3(nblk(n)), dim3(TPB), 0, st, g, x, v, cid, rank, vx, vy, cnt);
+        if (Nc + 1 <= ONE_MAX) {
+            hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(ONE_TPB), 0, st, cnt, Nc + 1, start, (const int*)nullptr,
+                               (int*)nullptr, (const int*)nullptr);
+        } else {
+            hipLaunchKernelGGL(k_scan_tiles, dim3(nTiles), dim3(TPB), 0, st, cnt, Nc + 1, start, tileSum);
+            hipLaunchKernelGGL(k_scan_add_prefix, dim3(nblk(Nc + 1)), dim3(TPB), 0, st, start, Nc + 1, tileSum);
         }
-        hipLaunchKernelGGL(k_fill_int, dim3(nblk(Nc + 1)), dim3(TPB), 0, st, cnt, Nc + 1, 0);
-        if (n > 0) hipLaunchKernelGGL(k_hist, dim3(bin_blocks(n)), dim3(TPB), 0, st, cid, n, cnt);
-        hipLaunchKernelGGL(k_scan_tiles, dim3(nTiles), dim3(TPB), 0, st, cnt, Nc + 1, start, tileSum,
-                           (const int*)nullptr, cursor);
-        hipLaunchKernelGGL(k_scan_add_prefix, dim3(nblk(Nc + 1)), dim3(TPB), 0, st, start, Nc + 1, tileSum);
-        if (n > 0) {
-            hipLaunchKernelGGL(k_scatter, dim3(bin_blocks(n)), dim3(TPB), 0, st, cid, pid, n, start, cursor, key);
-            hipLaunchKernelGGL(k_segsort, dim3(nblk(Nc, SEG_CELLS)), dim3(SEG_CELLS), 0, st, start, Nc, key, list,
-                               (int)(n < (1 << 27)), 0);
-        }
+        hipLaunchKernelGGL(k_na_scatter, dim3(nblk(n)), dim3(TPB), 0, st, cid, rank, n, start, key);
+        hipLaunchKernelGGL(k_segsort, dim3(nblk(Nc, SEG_CELLS)), dim3(SEG_CELLS), 0, st, start, Nc, key, list,
+                           (int)(n < (1 << 27)), 0);
         const double mean = (double)n / (double)std::max(Nc, 1) * CELL_BLK;
         const int cap = (int)std::min(4096.0, std::max(256.0, 1.15 * mean + 2.0 * CELL_BLK));
         FieldsOut f{out->N, out->Ux, out->Uy, out->Px, out->Py, out->T, out->rho, out->Pkin, out->Pvir, out->P};
         const double vc = (p->Lx / (double)p->Nx) * (p->Ly / (double)p->Ny);
         hipLaunchKernelGGL(k_cell_fields, dim3(nblk(Nc, CELL_BLK)), dim3(CELL_BLK), cap * 2 * sizeof(double), st,
                            start, list, Nc, vx, vy, vc, p->Kvirial, rhoTarget, f, cap);
-        if (out->rhoTarget)
-            hipLaunchKernelGGL(k_fill_double, dim3(nblk(Nc)), dim3(TPB), 0, st, out->rhoTarget, Nc, rhoTarget);
         HIP_OK(hipGetLastError());
     });
 }
