@@ -74,9 +74,10 @@ struct Grid {
 };
 
 /* The place of cell index q: its sample's first cell, and its column and row.
- * Taken once per cell; the nine taps' neighbours follow by additions (a
- * division per tap, in 64 bits, was most of the convolutions' time: 60 us per
- * 32 -> 32 layer of 524,288 cells, whose traffic takes 28). */
+ * Taken once per cell; the nine taps' neighbours follow by additions instead
+ * of a 64-bit division each: a 32 -> 32 layer of 524,288 cells takes 50 us
+ * instead of 60 (its traffic alone 14; what is left is the chain from the
+ * gathers to the products), the weight gradient's gathers most of their time. */
 struct CellAt {
     long long s0; /* -1: no cell */
     int ix, iy;
@@ -244,7 +245,9 @@ __global__ void __launch_bounds__(NTPB) k_conv_wgrad(Grid g, const u16* __restri
     for (long long bk = blockIdx.x; bk < nblkTot; bk += gridDim.x) {
         const long long c0 = bk * WG_PITCH;
         /* thread t holds cell t % WG_PITCH of the tile: its place once, its
-         * neighbour once per tap, whatever the channel */
+         * neighbour once per tap, whatever the channel, and a tap's loads all
+         * issued before the first is stored (131,072 cells, 32 -> 32: 151 us
+         * with a division per element, 38 now) */
         const int k = (int)threadIdx.x % WG_PITCH, r0 = (int)threadIdx.x / WG_PITCH;
         const long long q = c0 + k;
         const CellAt at = cell_at(g, q);
@@ -306,7 +309,7 @@ __global__ void __launch_bounds__(NTPB) k_conv_wgrad(Grid g, const u16* __restri
  * layer (W[co][tap][ci] for the real channels, then b[co]): 64 entries per
  * block, sixteen threads per entry, each its sixteenth of the partials in
  * order, then the sixteen in order (one thread per entry walked up to 512
- * partials alone: 124 us per layer). */
+ * partials alone: 124 us per layer of 131,072 cells, 11.5 now). */
 constexpr int WR_E = 64, WR_G = 16;
 __global__ void __launch_bounds__(WR_E * WR_G) k_wgrad_reduce(const float* __restrict__ part,
                                                               const float* __restrict__ bpart, int nparts, int co, int ci,

@@ -1,7 +1,6 @@
 /*
  * mpcd_zone.h -- one zone of the snapshot zone redistribution
- * (zone_pass.cpp:62-973) on one wavefront, shared by the gfx950 kernel in
- * mpcd_engine.hip and the host logic check in tests/ (ZHD code).
+ * (zone_pass.cpp:62-973), shared by the gfx950 kernels in mpcd_engine.hip and the host logic check in tests/ (ZHD code).
  *
  * The reference's zone kernel is sequential: a shuffled list of dense cells,
  * each of which mutates the counts its successors read.  That order is kept;
@@ -15,8 +14,9 @@
  * the barrier to nothing.  A move only records, per particle, the dense pass
  * or the sparse phase that moved it last; the momentum correction, which
  * visits every particle in its final cell, writes the new positions from
- * that record.  On the device the correction runs in a kernel of its own
- * (the zone's state handed over in global memory, see ZoneState).
+ * that record.  The fused kernel (zones with 16-bit indices) runs the passes
+ * on four wavefronts and the correction behind them, the zone's state staying
+ * in LDS; the two-kernel form hands it over in global memory (ZoneState).
  *
  * Memory.  Cell arrays are indexed by the zone-local cell
  * lc = (ix-xs)*zh + (iy-ys) (ascending global cell id); particles by the
