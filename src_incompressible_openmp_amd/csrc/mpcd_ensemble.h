@@ -236,7 +236,7 @@ __global__ void __launch_bounds__(TPB) k_ens_closure_repair(const EnsRep* __rest
     }
 }
 
-/* beta of every replica: block r reduces replica r's partials (k_reduce_beta) */
+/* beta of every replica: block r reduces replica r's partials */
 __global__ void __launch_bounds__(TPB) k_ens_reduce_beta(const EnsRep* __restrict__ reps,
                                                          const double* __restrict__ part, double* __restrict__ scal) {
     const EnsRep& e = reps[blockIdx.x];
