@@ -179,7 +179,12 @@ inline ZoneParams make_zone_params(const mpcd_params& p) {
             const int ax = std::abs(a % 5 - 2), ay = std::abs(a / 5 - 2), bx = std::abs(b % 5 - 2), by = std::abs(b / 5 - 2);
             if (std::max(ax, ay) == std::max(bx, by) && ax * ax + ay * ay == bx * bx + by * by) apart = false;
         }
-    zp.quadBins = !zp.dedupe && apart && *std::max_element(perBin, perBin + 8) <= 3;
+    /* on a periodic axis of one or two cells an offset leads back to the cell
+     * itself, a target once the low threshold lies above the high one */
+    const bool own = ((p.bc_left == MPCD_BC_PERIODIC && p.bc_right == MPCD_BC_PERIODIC && p.Nx < 3) ||
+                      (p.bc_bottom == MPCD_BC_PERIODIC && p.bc_top == MPCD_BC_PERIODIC && p.Ny < 3)) &&
+                     zp.lowThrBulk > zp.highThr;
+    zp.quadBins = !own && apart && *std::max_element(perBin, perBin + 8) <= 3;
     return zp;
 }
 

@@ -133,8 +133,8 @@ struct ZoneParams {
     double lowLoc1, highLoc1; /* empty-cell thresholds for fluid fraction 1 */
     int useLocal, maxPasses, corrEnabled;
     int dedupe; /* a periodic axis narrower than 5 cells: wrapped neighbours can repeat */
-    int quadBins; /* no dedupe, at most 3 neighbour offsets per angular bin, no two of a bin equally far: the
-                   * wavefront form's lane layout, in which no tie is left to a draw */
+    int quadBins; /* at most 3 neighbour offsets per angular bin, no two of a bin equally far (the wavefront form's
+                   * lane layout, in which no tie is left to a draw), and no dense cell its own target */
     /* angular bin (3 bits) of (dx,dy) in [-2,2]^2 at index (dy+2)*5+(dx+2):
      * indices 0..20 in binLo, 21..24 in binHi (registers, not an array that
      * a dynamic index would send to private memory) */
@@ -1172,6 +1172,16 @@ ZHD bool zone_wrap_y(const Z& z) {
 }
 /* zone-relative coordinate t taken once around an axis of n cells */
 ZHD int wrap_near(int t, int n) { return t < 0 ? t + n : (t >= n ? t - n : t); }
+/* Offset d to the (not yet wrapped) coordinate t is min_step's on a periodic
+ * axis of n cells.  Below five cells several offsets lead to one cell, and
+ * this one alone stands for it: the candidates come out as the general form's
+ * dedupe leaves them, whose keys are those of the shortest step.  (On one
+ * wavefront in the general form a launch of 4 x 1024 x 20 took 216 us, on the
+ * four 56; one of 5 x 1024 x 20 takes 60.) */
+ZHD bool shortest_step(int d, int t, int n) {
+    const int a = 2 * (d < 0 ? -d : d);
+    return a < n || (a == n && (unsigned)t < (unsigned)n);
+}
 
 /* A dense cell's surplus over its high threshold (an occupied cell's is the
  * bulk one), and its start bins of both phases. */
@@ -1331,9 +1341,16 @@ template <class Z>
 ZHD int dense_cell_wave(Z& z, const DenseLane& dl, int c, int cx, int cy, int need, unsigned bins, int pass, int lane) {
     typedef typename Z::idx_t IT;
     int tx = cx + dl.dx, ty = cy + dl.dy;
-    if (zone_wrap_x(z)) tx = wrap_near(tx, z.g.Nx);
-    if (zone_wrap_y(z)) ty = wrap_near(ty, z.g.Ny);
-    const bool in = (dl.code >= 0) & ((unsigned)tx < (unsigned)z.zw) & ((unsigned)ty < (unsigned)z.zh);
+    bool in = dl.code >= 0;
+    if (zone_wrap_x(z)) {
+        if (z.zp.dedupe) in = in & shortest_step(dl.dx, tx, z.g.Nx);
+        tx = wrap_near(tx, z.g.Nx);
+    }
+    if (zone_wrap_y(z)) {
+        if (z.zp.dedupe) in = in & shortest_step(dl.dy, ty, z.g.Ny);
+        ty = wrap_near(ty, z.g.Ny);
+    }
+    in = in & ((unsigned)tx < (unsigned)z.zw) & ((unsigned)ty < (unsigned)z.zh);
     const int l = in ? tx * z.zh + ty : c;
     const ZCell<IT> S = z.cell[c];
     const unsigned fS = (unsigned)S.fl;
@@ -2010,9 +2027,16 @@ __device__ __forceinline__ int sparse_neighbour(const Z& z, int cx, int cy, int 
     dy = f / 3 - 1;
     dx = f - 3 * (f / 3) - 1;
     int tx = cx + dx, ty = cy + dy;
-    if (zone_wrap_x(z)) tx = wrap_near(tx, z.g.Nx);
-    if (zone_wrap_y(z)) ty = wrap_near(ty, z.g.Ny);
-    const bool in = (o < 8) & ((unsigned)tx < (unsigned)z.zw) & ((unsigned)ty < (unsigned)z.zh);
+    bool in = o < 8;
+    if (zone_wrap_x(z)) {
+        if (z.zp.dedupe) in = in & shortest_step(dx, tx, z.g.Nx);
+        tx = wrap_near(tx, z.g.Nx);
+    }
+    if (zone_wrap_y(z)) {
+        if (z.zp.dedupe) in = in & shortest_step(dy, ty, z.g.Ny);
+        ty = wrap_near(ty, z.g.Ny);
+    }
+    in = in & ((unsigned)tx < (unsigned)z.zw) & ((unsigned)ty < (unsigned)z.zh);
     return in ? tx * z.zh + ty : -1;
 }
 
@@ -2107,7 +2131,7 @@ __device__ __forceinline__ void zone_sparse_pass_mw(Z& z, int wave, int lane) {
     volatile IT* vlix = z.lix;
     double* const score = z.duG; /* 8 per low cell of the segment */
     const int SEG = imax(1, z.C / 4);
-    const bool noSeg = z.C < 4 || z.zp.dedupe != 0;
+    const bool noSeg = z.C < 4;
     for (int s0 = 0; s0 < m; s0 += SEG) {
         const int s1 = imin(m, s0 + SEG);
         /* scores: eight lanes per low cell */
