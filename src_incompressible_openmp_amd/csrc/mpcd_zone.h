@@ -1189,6 +1189,15 @@ template <class Z>
 ZHD int dense_need(const Z& z, int nc) {
     return imax(0, (int)MPCD_CEIL((double)nc - z.zp.highThr));
 }
+/* The cell's movers fit the wavefront form, min(need + 1, count) <= 64, and
+ * so does the need itself (it exceeds the count where the high threshold lies
+ * below zero); a cell that was empty when the pass took its thresholds has
+ * another than dense_need's. */
+template <class Z>
+ZHD bool dense_fits(const Z& z, int c, int nc) {
+    const int need = dense_need(z, nc);
+    return need > 0 && need <= ZONE_MAX_MOVE && imin(need + 1, nc) <= ZONE_MAX_MOVE && fget(z, c, ZF_BULK0);
+}
 template <class Z>
 ZHD unsigned dense_bins(const Z& z, int c, int pass) {
     const uint32_t gc = (uint32_t)lc_gc(z, c);
@@ -1516,7 +1525,7 @@ ZHD void zone_dense_passes(Z& z, int lane, int nl) {
             if ((double)nc <= hl) continue;
             const int needOut = imax(0, (int)MPCD_CEIL((double)nc - hl));
 #if defined(__HIP_DEVICE_COMPILE__)
-            if (z.zp.quadBins && needOut > 0 && imin(needOut + 1, nc) <= ZONE_MAX_MOVE) {
+            if (z.zp.quadBins && dense_fits(z, c, nc)) {
                 ++nHighW;
                 const int cx = lc_col(z, c);
                 movedW += dense_cell_wave(z, dlane, c, cx, c - cx * z.zh, needOut, dense_bins(z, c, pass), pass, lane);
@@ -1653,7 +1662,7 @@ __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
                 pos[lc] = (IT)NONE;
                 const int nc = cnt_of(z, lc);
                 f = (double)nc > high_thr(z, lc) && !fget(z, lc, ZF_OUT);
-                one = one || (f && (nc <= 0 || imin(dense_need(z, nc) + 1, nc) > ZONE_MAX_MOVE));
+                one = one || (f && !dense_fits(z, lc, nc));
             }
             const unsigned long long msk = wave_ballot(f);
             if (lane == 0) chunkMask[ch] = msk;
@@ -1728,8 +1737,8 @@ __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
                 const double hl = high_thr(z, c);
                 if (nc <= 0 || (double)nc <= hl) continue;
                 ++nHighW;
-                const int needOut = dense_need(z, nc);
-                if (z.zp.quadBins && imin(needOut + 1, nc) <= ZONE_MAX_MOVE) {
+                const int needOut = imax(0, (int)MPCD_CEIL((double)nc - hl));
+                if (z.zp.quadBins && dense_fits(z, c, nc)) {
                     movedW += dense_cell_wave(z, dlane, c, cx, cy, needOut, dense_bins(z, c, pass), pass, lane);
                 } else {
                     /* the one-lane form (serial lists only: wavefront 0, the

@@ -131,3 +131,21 @@ def test_narrow_axis_takes_the_scheduled_form(gpu):
         sim.close()
         best[Nx] = min(t)
     assert best[4] <= 1.15 * best[5], best
+
+
+@pytest.mark.parametrize("floor", [3.0, -3.0])
+def test_high_threshold_below_zero(gpu, oracle, floor):
+    """Every occupied cell is dense, with a surplus past seven bits however few
+    particles it has, and the empty ones receive; with the empty cells'
+    threshold below zero too, they are dense in turn once they have."""
+    p = to_struct(poiseuille_params(Nx=40, Ny=30, gamma=2.0, coef=-80.0, lowThrBulkOverride=-500.0, lowThrFloor=5.0,
+                                    highThrFloor=floor))
+    for layout in (LAYOUT_BASE, LAYOUT_SHIFTED):
+        x, v = state(p, False)
+        xo, vo = x.copy(), v.copy()
+        m, _ = oracle.zone_pass(CTR, p, xo, vo, layout, 88172645463325252)
+        g, _ = gpu.zone_pass(p, x, v, layout, 88172645463325252)
+        assert m["nParticlesMovedDense"] > 2000
+        assert g["nParticlesMovedDense"] == m["nParticlesMovedDense"], layout
+        assert x.tobytes() == xo.tobytes(), layout
+        assert v.tobytes() == vo.tobytes(), layout
