@@ -1,12 +1,14 @@
 """Host arrays to the device and back around the size where a copy is cut into
 chunks (8 MiB: 524,288 particles of two doubles), at sizes that leave partial
 chunks, from one thread and from several with an object each: every byte."""
+import ctypes
 import threading
 
 import numpy as np
 import pytest
 
 from src_incompressible_openmp_amd.params import poiseuille_params, to_struct
+from tests.test_zz_no_alloc import hip_runtime
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +49,40 @@ def test_several_threads():
     for t in th:
         t.join()
     assert bad == [0] * 4
+
+
+@pytest.mark.parametrize("up", ["pageable", "pinned"])
+@pytest.mark.parametrize("down", ["pageable", "pinned"])
+def test_each_direction_alone(up, down):
+    """Pinned arrays are copied in one piece and pageable ones in chunks, so
+    with one of each only one direction is cut into chunks."""
+    from src_incompressible_openmp_amd import gpu
+
+    n = 600001
+    p = to_struct(poiseuille_params(Nx=64, Ny=32, gamma=n / 2048.0))
+    p.n = n
+    rng = np.random.default_rng(5)
+    x = rng.random((n, 2)) * np.array([p.Lx, p.Ly]) * 0.999
+    v = rng.normal(size=(n, 2))
+    hip = hip_runtime(gpu)
+    pinned = []
+
+    def new(kind):
+        if kind == "pageable":
+            return np.zeros((n, 2))
+        q = ctypes.c_void_p()
+        assert hip.hipHostMalloc(ctypes.byref(q), ctypes.c_size_t(16 * n), ctypes.c_uint(0)) == 0
+        pinned.append(q)
+        return np.ctypeslib.as_array(ctypes.cast(q, ctypes.POINTER(ctypes.c_double)), shape=(n, 2))
+
+    hx, hv, x2, v2 = new(up), new(up), new(down), new(down)
+    hx[:], hv[:], x2[:], v2[:] = x, v, 0.0, 0.0
+    ptr = lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+    sim = gpu.Sim(p)
+    sim.set_state(hx, hv)
+    gpu._check(gpu.load().mpcd_gpu_sim_get_state(sim._h, ptr(x2), ptr(v2)))
+    sim.close()
+    same = np.array_equal(x2, x) and np.array_equal(v2, v)
+    for q in pinned:
+        assert hip.hipHostFree(q) == 0
+    assert same
