@@ -3294,12 +3294,11 @@ int mpcd_gpu_sim_cell_fields(mpcd_gpu_sim* s, double rhoTarget, mpcd_cell_fields
         if (s->streamed >= 0) throw ApiError(MPCD_E_INVALID, "internal: a fused stream was left unused");
         s->fields_current();
         const size_t C = (size_t)s->Nc;
-        if (out->N) s->copy.download(out->N, s->outN, C * sizeof(int), s->stream);
+        /* one wait for all ten grids (a wait of N's own cost 20 us of 50 x 50's 0.21 ms) */
+        if (out->N) s->copy.download_later(out->N, s->outN, C * sizeof(int), s->stream);
         double* hs[9] = {out->Ux, out->Uy, out->Px, out->Py, out->T, out->rho, out->Pkin, out->Pvir, out->P};
         for (int k = 0; k < 9; ++k)
-            if (hs[k])
-                HIP_OK(hipMemcpyAsync(hs[k], s->outF + (size_t)k * C, C * sizeof(double), hipMemcpyDeviceToHost,
-                                      s->stream));
+            if (hs[k]) s->copy.download_later(hs[k], s->outF + (size_t)k * C, C * sizeof(double), s->stream);
         HIP_OK(hipStreamSynchronize(s->stream));
         if (out->rhoTarget)
             for (size_t c = 0; c < C; ++c) out->rhoTarget[c] = rhoTarget;
@@ -3431,10 +3430,10 @@ int mpcd_gpu_compute_cell_fields(const mpcd_params* p, const double* x, const do
                            s.cellCap);
         s.check_launch();
         const size_t nb = (size_t)s.Nc * sizeof(double);
-        if (out->N) HIP_OK(hipMemcpyAsync(out->N, dN, (size_t)s.Nc * sizeof(int), hipMemcpyDeviceToHost, s.stream));
+        if (out->N) s.copy.download_later(out->N, dN, (size_t)s.Nc * sizeof(int), s.stream);
         double* hs[9] = {out->Ux, out->Uy, out->Px, out->Py, out->T, out->rho, out->Pkin, out->Pvir, out->P};
         for (int k = 0; k < 9; ++k)
-            if (hs[k]) HIP_OK(hipMemcpyAsync(hs[k], d[k], nb, hipMemcpyDeviceToHost, s.stream));
+            if (hs[k]) s.copy.download_later(hs[k], d[k], nb, s.stream);
         HIP_OK(hipStreamSynchronize(s.stream));
         if (out->rhoTarget)
             for (int c = 0; c < s.Nc; ++c) out->rhoTarget[c] = rhoTarget;

@@ -90,10 +90,15 @@ class HostCopy {
 
     /* device to host, complete on return */
     void download(void* dst, const void* src, size_t bytes, hipStream_t st) {
-        if (!staged(dst, const_cast<void*>(src), bytes, st, false)) {
-            HIP_OK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
-            HIP_OK(hipStreamSynchronize(st));
-        }
+        if (!download_later(dst, src, bytes, st)) HIP_OK(hipStreamSynchronize(st));
+    }
+    /* the same for one of several arrays that share one wait: complete at the
+     * latest once the caller has waited for the stream; true if it is on
+     * return */
+    bool download_later(void* dst, const void* src, size_t bytes, hipStream_t st) {
+        if (staged(dst, const_cast<void*>(src), bytes, st, false)) return true;
+        HIP_OK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+        return false;
     }
     /* host to device, ordered on the stream: a pageable array may change on
      * return, a pinned one once the stream has got there (every caller waits

@@ -86,3 +86,26 @@ def test_each_direction_alone(up, down):
     for q in pinned:
         assert hip.hipHostFree(q) == 0
     assert same
+
+
+@pytest.mark.parametrize("grid", [(1024, 1023), (1025, 1024), (2048, 1025)])
+def test_large_field_grids(oracle, grid):
+    """Field grids of doubles just below and above the size that is cut, and
+    one whose counts are cut too, from both entry points that return them."""
+    from src_incompressible_openmp_amd import gpu
+
+    nx, ny = grid
+    p = to_struct(poiseuille_params(Nx=nx, Ny=ny, gamma=0.25))
+    p.n = 200003
+    rng = np.random.default_rng(7)
+    x = (rng.random((p.n, 2)) * np.array([p.Lx, p.Ly]) * 0.999).reshape(-1)
+    v = rng.normal(size=2 * p.n)
+    rt = p.gamma / ((p.Lx / p.Nx) * (p.Ly / p.Ny))
+    want = oracle.cell_fields(p, x, v, rt)
+    sim = gpu.Sim(p)
+    sim.set_state(x, v)
+    both = gpu.compute_cell_fields(p, x, v, rt), sim.cell_fields(rt)
+    sim.close()
+    bits = lambda a: np.ascontiguousarray(a).view(np.uint8)
+    differ = [k for got in both for k in want if not np.array_equal(bits(got[k]), bits(want[k]))]
+    assert not differ

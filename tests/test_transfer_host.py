@@ -38,7 +38,7 @@ def one():
     return run
 
 
-@pytest.mark.parametrize("up", [1, 0], ids=["upload", "download"])
+@pytest.mark.parametrize("up", [1, 0, -1], ids=["upload", "download", "download_later"])
 @pytest.mark.parametrize("n", [1, CUT_FROM - 1, CUT_FROM, CUT_FROM + 1, 5 * CHUNK, 7 * CHUNK + 12345, 33 * CHUNK - 8])
 def test_pageable(one, n, up):
     for strict in (0, 1):
@@ -47,7 +47,7 @@ def test_pageable(one, n, up):
         assert copies == (1 if n < CUT_FROM else -(-n // CHUNK))
 
 
-@pytest.mark.parametrize("up", [1, 0], ids=["upload", "download"])
+@pytest.mark.parametrize("up", [1, 0, -1], ids=["upload", "download", "download_later"])
 @pytest.mark.parametrize("kind", [PINNED, DEVICE], ids=["pinned", "device"])
 def test_registered_goes_direct(one, kind, up):
     for n in (CUT_FROM - 1, CUT_FROM, 9 * CHUNK + 77):

@@ -7,14 +7,15 @@ namespace mpcdk {
 void set_last_error(const std::string&) {}
 }  // namespace mpcdk
 
-/* One copy of n bytes (up: host to device).  type: the host array's
+/* One copy of n bytes (up 1: host to device, 0: back, -1: back with the wait
+ * left to the caller).  type: the host array's
  * (hipMemoryType), strict: an unregistered pointer is an error to ask about.
  * Returns the number of wrong bytes once the stream has been waited for;
  * *copies: how many copies the runtime was given. */
 extern "C" long long transfer_one(long long n, int up, int type, int strict, long long* copies) {
     std::vector<unsigned char> host((size_t)n + 64), dev((size_t)n + 64);
-    std::vector<unsigned char>& src = up ? host : dev;
-    std::vector<unsigned char>& dst = up ? dev : host;
+    std::vector<unsigned char>& src = up > 0 ? host : dev;
+    std::vector<unsigned char>& dst = up > 0 ? dev : host;
     uint64_t r = 88172645463325252ull;
     for (long long i = 0; i < n; ++i) {
         r ^= r << 13;
@@ -36,13 +37,15 @@ extern "C" long long transfer_one(long long n, int up, int type, int strict, lon
     FakeStream st;
     {
         mpcdk::HostCopy copy;
-        if (up) {
+        if (up > 0) {
             copy.upload(dev.data(), host.data(), (size_t)n, &st);
             /* pageable memory may change on return */
             if (type == hipMemoryTypeUnregistered && st.queued > 1) std::fill(host.begin(), host.end(), 0);
         } else {
-            copy.download(host.data(), dev.data(), (size_t)n, &st);
-            if (st.done != st.queued) return -1; /* complete on return */
+            const bool later = up < 0;
+            const bool whole = later && copy.download_later(host.data(), dev.data(), (size_t)n, &st);
+            if (!later) copy.download(host.data(), dev.data(), (size_t)n, &st);
+            if ((st.done == st.queued) != (!later || whole)) return -1; /* complete on return, and only then */
         }
         (void)hipStreamSynchronize(&st);
     }
