@@ -5,7 +5,7 @@
  * The runtime's own staged copies reach 9-10 GB/s into a pageable destination
  * and 28 GB/s out of one here, a fraction of the link's rate: one download of
  * 10.5 million particles (336 MB) took 32 ms, 37 into fresh pages, as long as
- * 20 time steps.  A copy of COPY_MIN bytes or more is cut into chunks instead,
+ * 20 time steps.  A copy of UP_MIN or DOWN_MIN bytes or more is cut into chunks instead,
  * which a few threads move: each owns two pinned chunks, so its copy on one
  * side runs beside the device's on the other, and the page faults of a fresh
  * destination are shared.  The same download takes 9.7 ms (10.0 fresh), the
@@ -78,10 +78,12 @@ class PinnedChunks {
 /* Held by every object that copies; the copies themselves. */
 class HostCopy {
    public:
-    /* two threads' worth of chunks: a copy of 8 MiB takes the same either way
-     * (an evaluation of 524,288 cells 0.729 ms chunked, 0.732 not), one of
-     * 10 MiB a fifth less chunked */
-    static constexpr size_t COPY_MIN = 4 * PinnedChunks::BYTES;
+    /* Down, two threads' worth of chunks: 8 MiB take 0.35 ms chunked, 0.51 not
+     * (the threads' start costs what is gained below).  The runtime's uploads
+     * are three times as fast, so chunks pay later: 8 MiB take 0.30 ms
+     * chunked, 0.25 not, 10 MiB 0.35 and 0.32, 12 MiB 0.41 and 0.40, 16 MiB
+     * 0.52 and 0.56. */
+    static constexpr size_t DOWN_MIN = 4 * PinnedChunks::BYTES, UP_MIN = 8 * PinnedChunks::BYTES;
 
     HostCopy() { PinnedChunks::instance().lease(); }
     ~HostCopy() { PinnedChunks::instance().release(); }
@@ -117,7 +119,7 @@ class HostCopy {
     }
 
     bool staged(void* host, void* dev, size_t bytes, hipStream_t st, bool up) {
-        if (bytes < COPY_MIN || !pageable(host)) return false;
+        if (bytes < (up ? UP_MIN : DOWN_MIN) || !pageable(host)) return false;
         PinnedChunks& pc = PinnedChunks::instance();
         std::unique_lock<std::mutex> lk(pc.busy(), std::try_to_lock);
         if (!lk.owns_lock()) return false;

@@ -1,6 +1,7 @@
-"""Host arrays to the device and back around the size where a copy is cut into
-chunks (8 MiB: 524,288 particles of two doubles), at sizes that leave partial
-chunks, from one thread and from several with an object each: every byte."""
+"""Host arrays to the device and back around the sizes where a copy is cut into
+chunks (8 MiB down, 16 MiB up: 524,288 and 1,048,576 particles of two doubles),
+at sizes that leave partial chunks, from one thread and from several with an
+object each: every byte."""
 import ctypes
 import threading
 
@@ -58,7 +59,7 @@ def test_each_direction_alone(up, down):
     with one of each only one direction is cut into chunks."""
     from src_incompressible_openmp_amd import gpu
 
-    n = 600001
+    n = 1200001
     p = to_struct(poiseuille_params(Nx=64, Ny=32, gamma=n / 2048.0))
     p.n = n
     rng = np.random.default_rng(5)
