@@ -1189,14 +1189,19 @@ template <class Z>
 ZHD int dense_need(const Z& z, int nc) {
     return imax(0, (int)MPCD_CEIL((double)nc - z.zp.highThr));
 }
-/* The cell's movers fit the wavefront form, min(need + 1, count) <= 64, and
- * so does the need itself (it exceeds the count where the high threshold lies
- * below zero); a cell that was empty when the pass took its thresholds has
- * another than dense_need's. */
+/* The movers of a dense cell of nc particles fit the wavefront form,
+ * min(need + 1, nc) <= 64, and so does the need itself (it exceeds the count
+ * where the high threshold lies below zero). */
+template <class Z>
+ZHD bool dense_count_fits(const Z& z, int nc) {
+    const int need = dense_need(z, nc);
+    return need > 0 && need <= ZONE_MAX_MOVE && imin(need + 1, nc) <= ZONE_MAX_MOVE;
+}
+/* (a cell that was empty when the pass took its thresholds has another than
+ * dense_need's) */
 template <class Z>
 ZHD bool dense_fits(const Z& z, int c, int nc) {
-    const int need = dense_need(z, nc);
-    return need > 0 && need <= ZONE_MAX_MOVE && imin(need + 1, nc) <= ZONE_MAX_MOVE && fget(z, c, ZF_BULK0);
+    return dense_count_fits(z, nc) && fget(z, c, ZF_BULK0);
 }
 template <class Z>
 ZHD unsigned dense_bins(const Z& z, int c, int pass) {
@@ -1615,9 +1620,12 @@ __device__ __forceinline__ int zone_compact_mw(Z& z, const unsigned long long* c
  * each wait is bounded all the same (past DS_WAIT_MAX polls it records
  * schedWait, which the kernel reports as an error, and goes on).  A list with
  * a cell that needs the one-lane form (its movers exceed a wavefront, or the
- * grid has no quadBins), thresholds that let a dense cell receive (low above
- * high) or list an empty one, or a list that leaves ext no room for pos and
- * done runs on wavefront 0 alone, in list order.
+ * grid has no quadBins) or an empty one, or a list that leaves ext no room for
+ * pos and done runs on wavefront 0 alone, in list order.  With the low
+ * threshold above the high one a dense cell receives too, up to the low
+ * threshold: it takes its surplus after its wait, and the list is scheduled
+ * if a cell of that many particles fits a wavefront (200 x 100 x 12 with 16
+ * above 13.2: 898 us a step, 1328 on one wavefront).
  *
  * What a cell writes lies in LDS, whose accesses the release and acquire
  * order; a zone whose links spill to its global region orders those too. */
@@ -1651,6 +1659,8 @@ __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
     IT* const pos = z.ext;
     volatile IT* const done = z.ext + z.C;
     unsigned long long* const chunkMask = reinterpret_cast<unsigned long long*>(z.scr->cand); /* idle here */
+    const bool late = z.zp.lowThrBulk > z.zp.highThr;
+    const bool form = z.zp.quadBins && (!late || dense_count_fits(z, (int)MPCD_CEIL(z.zp.lowThrBulk)));
     for (int pass = 1; pass <= z.zp.maxPasses; ++pass) {
         /* thresholds and the list: chunk ch of 64 cells on wavefront ch % 4 */
         bool one = false;
@@ -1668,7 +1678,7 @@ __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
             if (lane == 0) chunkMask[ch] = msk;
         }
         for (int k = z.C + tid; k < nExt; k += NT) z.ext[k] = (IT)0;
-        bool serial = __syncthreads_or(one) || !z.zp.quadBins || z.zp.lowThrBulk > z.zp.highThr;
+        bool serial = __syncthreads_or(one) || !form;
         const int m = zone_compact_mw(z, chunkMask, wave, lane);
         serial = serial || m + z.C > nExt;
         __syncthreads();
@@ -1727,7 +1737,8 @@ __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
                         __builtin_amdgcn_s_sleep(1);
                     }
                     sched_acquire(z);
-                    movedW += dense_cell_wave(z, dlane, c, cx, cy, (int)(nb & 127u), nb >> 7, pass, lane);
+                    const int need = late ? uniform(dense_need(z, cnt_of(z, c))) : (int)(nb & 127u);
+                    movedW += dense_cell_wave(z, dlane, c, cx, cy, need, nb >> 7, pass, lane);
                     sched_release(z);
                     if (lane == 0) done[k] = (IT)1;
                     ZWSYNC();

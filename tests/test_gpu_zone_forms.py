@@ -149,3 +149,20 @@ def test_high_threshold_below_zero(gpu, oracle, floor):
         assert g["nParticlesMovedDense"] == m["nParticlesMovedDense"], layout
         assert x.tobytes() == xo.tobytes(), layout
         assert v.tobytes() == vo.tobytes(), layout
+
+
+@pytest.mark.parametrize("crowded", [False, True], ids=["uniform", "crowded"])
+@pytest.mark.parametrize("low", [12.3, 12.7, 16.0, 40.0, 63.0, 64.0, 65.5, 90.0, 1e6])
+def test_low_threshold_above_high(gpu, oracle, low, crowded):
+    """Dense cells that receive before their turn, up to a low threshold just
+    above the high one (12.24), and around the most a wavefront takes."""
+    p = to_struct(poiseuille_params(Nx=60, Ny=50, gamma=12.0, coef=0.02, lowThrBulkOverride=low, maxRedistribPasses=3))
+    for layout in (LAYOUT_BASE, LAYOUT_SHIFTED):
+        x, v = state(p, crowded)
+        xo, vo = x.copy(), v.copy()
+        m, _ = oracle.zone_pass(CTR, p, xo, vo, layout, 88172645463325252)
+        g, _ = gpu.zone_pass(p, x, v, layout, 88172645463325252)
+        assert g["nParticlesMovedDense"] == m["nParticlesMovedDense"], layout
+        assert g["nParticlesMovedSparse"] == m["nParticlesMovedSparse"], layout
+        assert x.tobytes() == xo.tobytes(), layout
+        assert v.tobytes() == vo.tobytes(), layout
