@@ -158,7 +158,7 @@ enum {
     MPCD_PROF_ZONE_KERNEL = 5, /* the zone kernel launches (passes, and the correction when fused; 2 per step) */
     MPCD_PROF_CLOSURE = 6,     /* closure: fields, beta, stencil, kick */
     MPCD_PROF_KICK = 7,        /* the closure's per-particle kick alone */
-    MPCD_PROF_ZONE_FINISH = 8, /* the separate momentum correction kernel (zones the fused kernel does not take) */
+    MPCD_PROF_ZONE_FINISH = 8, /* passes and correction of the zones the fused kernel does not take */
     MPCD_PROF_KICK_STREAM = 9, /* the kick fused with the next step's stream (steps of one call) */
     MPCD_PROF_CLASSES = 10
 };

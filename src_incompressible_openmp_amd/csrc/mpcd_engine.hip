@@ -303,9 +303,9 @@ __global__ void __launch_bounds__(TPB) k_scan_add_prefix(int* __restrict__ out, 
 
 /* The whole scan by one block of 1024 threads, four entries each: a grid of
  * up to 4,095 cells pays one launch instead of two, four times a step (at
- * 2,501 entries 4.5 us against 8.9; with nine entries' loads per thread a
- * block of its own took 29 us at 32,769 entries against 9.7, so larger scans
- * keep the two kernels). */
+ * 2,501 entries 4.5 us against 8.9; one block with nine groups of four entries
+ * per thread took 29 us at 32,769 entries against 9.7, so larger scans keep
+ * the two kernels). */
 constexpr int ONE_TPB = 1024, ONE_MAX = 4 * ONE_TPB;
 __global__ void __launch_bounds__(ONE_TPB) k_scan_one(const int* __restrict__ in, int m, int* __restrict__ out,
                                                       const int* __restrict__ in2, int* __restrict__ zero,
@@ -1018,7 +1018,7 @@ __global__ void __launch_bounds__(CELL_BLK) k_cell_fields(const int* __restrict_
     if (f.P) f.P[c] = s.P;
 }
 
-/* ---- zone pass: one workgroup (one wavefront) per zone ---- */
+/* ---- zone pass: one workgroup per zone ---- */
 
 struct ZoneArgs {
     ZoneIn in;
@@ -1072,8 +1072,7 @@ __device__ __forceinline__ const ZoneIn& zone_in_of(const ZoneArgs& a, int zi, i
     }
 }
 
-/* particles of each zone: its columns' runs of the binning list */
-/* One wavefront per zone (block nZ writes the terminating zero): each lane
+/* particles of each zone: its columns' runs of the binning list.  One wavefront per zone (block nZ writes the terminating zero): each lane
  * takes columns of the zone, whose cells are one run of the binning. */
 __global__ void __launch_bounds__(64) k_zone_sizes(const ZoneRect* __restrict__ rects, int nZ,
                                                    const int* __restrict__ start, int Ny, int* __restrict__ sizes) {
@@ -1090,12 +1089,10 @@ __global__ void __launch_bounds__(64) k_zone_sizes(const ZoneRect* __restrict__ 
     if (lane == 0) sizes[zi] = P;
 }
 
-/* One zone per workgroup of one wavefront.  IT = uint16_t keeps the working
- * set in LDS at four zones per CU; IT = int serves zones of 65535 particles
- * or more (and the single-zone layout), in LDS or in global scratch. */
 /* The passes of zone zi by one wavefront (lanes 0..63): set-up, the dense
  * and sparse phases, the state hand-over to the correction.  The zone code
- * synchronises its lanes with wavefront-level barriers only. */
+ * synchronises its lanes with wavefront-level barriers only.  kLds: the
+ * working set in LDS (else in the zone's global scratch). */
 template <class IT, bool kLds>
 __device__ __forceinline__ void zone_pass_body(const ZoneArgs& a, int zi, long long off, int lane,
                                                unsigned char* lds, ZoneShared* sh) {
@@ -1124,8 +1121,6 @@ __device__ __forceinline__ void zone_pass_body(const ZoneArgs& a, int zi, long l
     }
 }
 
-/* A workgroup takes zones blockIdx.x, + gridDim.x, ... (the grid is
- * smaller than the zone count when few zones need this form). */
 /* The zones block b takes, b + gridDim.x * k, 64 at a time: each lane reads
  * one zone's size and a ballot names the zones in this launch's range (the
  * others go to another launch), so a small grid finds its few zones in one
@@ -1145,34 +1140,13 @@ __device__ inline bool next_zone(const ZoneArgs& a, int& k0, unsigned long long&
     return true;
 }
 
-template <class IT, bool kLds>
-__global__ void __launch_bounds__(ZONE_TPB) k_zone(ZoneArgs a) {
-    extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ ZoneShared sh;
-    const int lane = threadIdx.x;
-    int k0 = 0, zi = 0;
-    unsigned long long todo = 0ull;
-    while (next_zone(a, k0, todo, zi)) {
-        const int P = a.zsize[zi];
-        const long long off = a.zoff[zi];
-        if (off + (long long)P > a.scratchCap) {
-            if (lane == 0) atomicOr(a.err, 2);
-            continue;
-        }
-        zone_pass_body<IT, kLds>(a, zi, off, lane, lds, &sh);
-        ZBAR(); /* the next zone reuses the working set */
-    }
-}
-
-/* The momentum correction of the zones k_zone left (zone_pass.cpp:870-922),
- * FINISH_TPB threads per zone: a group of FIN_G lanes per cell for the
- * input-run sums and for the final lists' sums and writes (the sums in list
- * order), then one wavefront for the ordered stats. */
 constexpr int FINISH_TPB = 256;
-constexpr int FINISH_LDS = 40 * 1024; /* cell arrays, column map and as many links as fit */
-/* The correction of zone zi by TPB threads (zones of more than CPT x TPB
- * cells take the two-sweep form); lds/ldsBytes: the staging space (kLds) of
- * the zone state k_zone left in global memory. */
+/* The momentum correction of a zone zone_pass_body left (zone_pass.cpp:870-922)
+ * by TPB threads: a group of FIN_G lanes per cell for the input-run sums and
+ * for the final lists' sums and writes (the sums in list order), then one
+ * wavefront for the ordered stats; zones of more than CPT x TPB cells take the
+ * two-sweep form.  lds/ldsBytes: the staging space (kLds) of the zone state in
+ * global memory. */
 template <class IT, bool kLds, int TPB, int CPT>
 __device__ __forceinline__ void zone_finish_body(const ZoneArgs& a, const ZoneIn& in, int zid, uint64_t seed, int zi,
                                                  long long off, int tid, unsigned char* lds, long long ldsBytes,
@@ -1282,30 +1256,6 @@ __device__ __forceinline__ void zone_finish_body(const ZoneArgs& a, const ZoneIn
     }
 }
 
-template <class IT, bool kLds>
-__global__ void __launch_bounds__(FINISH_TPB) k_zone_finish(ZoneArgs a) {
-    extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ int queue[FINISH_TPB];
-    int k0 = 0, zi = 0;
-    unsigned long long todo = 0ull; /* the same in every wavefront of the block */
-    while (next_zone(a, k0, todo, zi)) {
-        const int P = a.zsize[zi];
-        const long long off = a.zoff[zi];
-        if (off + (long long)P > a.scratchCap) continue;
-        int zid;
-        uint64_t seed;
-        const ZoneIn& in = zone_in_of<false>(a, zi, zid, seed);
-        zone_finish_body<IT, kLds, FINISH_TPB, 4>(a, in, zid, seed, zi, off, (int)threadIdx.x, lds, FINISH_LDS, queue);
-        __syncthreads(); /* the next zone reuses the staging */
-    }
-}
-
-/* The passes and the correction of a zone in one workgroup of FUSED_TPB
- * threads (four wavefronts of at most 128 registers, so four zones share a
- * CU): all four wavefronts run the set-up, the scheduled dense and sparse
- * phases, then the correction, which takes the zone over in LDS where the
- * passes left it.  A zone's correction starts as soon as its own passes
- * end, beside the passes of slower zones. */
 /* a value every lane holds alike, in scalar registers */
 template <class T>
 __device__ __forceinline__ T uniform_value(T v) {
@@ -1335,9 +1285,10 @@ __device__ __forceinline__ void zone_uniform(Z& z) {
                  z.dgCnt);
 }
 
-/* The zones of more particles than 16-bit indices take: the passes on the
- * first wavefront, then the correction on all four (one launch: as a rule it
- * finds no such zone, and only its launch costs). */
+/* The zones k_zone_fused does not take (more particles or cells than 16-bit
+ * indices or its LDS hold): the passes on the first wavefront, then the
+ * correction on all four (one launch: as a rule it finds no such zone, and
+ * only its launch costs). */
 template <bool kLds>
 __global__ void __launch_bounds__(FINISH_TPB) k_zone_wide(ZoneArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
@@ -1373,6 +1324,12 @@ __device__ __forceinline__ void zone_region_done(const ZoneArgs& a) {
     }
 }
 
+/* The passes and the correction of a zone in one workgroup of FUSED_TPB
+ * threads (four wavefronts of at most 128 registers, so four zones share a
+ * CU): all four wavefronts run the set-up, the scheduled dense and sparse
+ * phases, then the correction, which takes the zone over in LDS where the
+ * passes left it.  A zone's correction starts as soon as its own passes
+ * end, beside the passes of slower zones. */
 constexpr int FUSED_TPB = 256;
 template <class IT, bool kEns = false>
 __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 waves per SIMD: four zones per CU */
@@ -1407,6 +1364,7 @@ __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 
     z.duG = a.duG + (size_t)zi * (size_t)a.duStride;
     zone_carve(z, lds, a.ldsBytes);
     static_assert(FUSED_TPB == 256, "the set-up and the phases take four wavefronts");
+    static_assert(ZONE_LDS_FAST / (sizeof(ZCell<uint16_t>) + 3 * sizeof(uint16_t)) <= 64 * 64, "zone_compact_mw's chunks");
     zone_setup_columns(z, wave, lane);
     __syncthreads();
     z.P = sh.P;
@@ -2586,11 +2544,7 @@ struct mpcd_gpu_sim {
                    const unsigned char* zmask = nullptr, bool stats = true) {
         const size_t fix16 = zone_fixed_bytes<uint16_t>(maxC, maxW, zp.useLocal);
         const bool fast = maxC < 65535 && fix16 + 2048 <= (size_t)ZONE_LDS_FAST;
-        /* LDS staging of the correction: the cell arrays and the column map leave room for links */
-        const size_t cellB16 = (size_t)maxC * (sizeof(ZCell<uint16_t>) + sizeof(uint16_t)) + 8 * (size_t)maxW + 16;
-        /* passes and correction in one kernel when the correction fits the passes' LDS */
-        const bool fused = fast && cellB16 + 4096 <= (size_t)ZONE_LDS_FAST;
-        if (!fused) { /* the fused kernel finds its zones' sizes and regions itself */
+        if (!fast) { /* the fused kernel finds its zones' sizes and regions itself */
             hipLaunchKernelGGL(k_zone_sizes, dim3(nZ + 1), dim3(64), 0, stream, rectsDev, nZ, bin.start, p.Ny, zsize);
             const int nt = (nZ + 1 + SCAN_TILE - 1) / SCAN_TILE;
             hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(TPB), 0, stream, zsize, nZ + 1, zoff, tileSum,
@@ -2664,22 +2618,10 @@ struct mpcd_gpu_sim {
             a.pMin = 0;
             a.pMax = 65534;
             a.ldsBytes = ZONE_LDS_FAST;
-            if (fused)
-                hipLaunchKernelGGL((k_zone_fused<uint16_t>), dim3(nZ), dim3(FUSED_TPB), ZONE_LDS_FAST, stream, a);
-            else
-                hipLaunchKernelGGL((k_zone<uint16_t, true>), dim3(nZ), dim3(ZONE_TPB), ZONE_LDS_FAST, stream, a);
+            hipLaunchKernelGGL((k_zone_fused<uint16_t>), dim3(nZ), dim3(FUSED_TPB), ZONE_LDS_FAST, stream, a);
             check_launch();
         }
         pend(MPCD_PROF_ZONE_KERNEL);
-        if (fast && !fused) {
-            pbeg(MPCD_PROF_ZONE_FINISH);
-            if (cellB16 + 4096 <= (size_t)FINISH_LDS)
-                hipLaunchKernelGGL((k_zone_finish<uint16_t, true>), dim3(nZ), dim3(FINISH_TPB), FINISH_LDS, stream, a);
-            else
-                hipLaunchKernelGGL((k_zone_finish<uint16_t, false>), dim3(nZ), dim3(FINISH_TPB), 0, stream, a);
-            pend(MPCD_PROF_ZONE_FINISH);
-            check_launch();
-        }
         /* zones the 16-bit path does not take, passes and correction in one
          * launch: none, as a rule, and none at all in a state of fewer
          * particles than such a zone has (a small grid strides over the zones;

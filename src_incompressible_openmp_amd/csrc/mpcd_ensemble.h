@@ -245,7 +245,7 @@ __global__ void __launch_bounds__(TPB) k_ens_reduce_beta(const EnsRep* __restric
     if (threadIdx.x == 0) beta_from_sums(sc, e.useOptimal, e.betaRepair);
 }
 
-/* pdrive with the interzone cross smoothing (k_pdrive per replica) */
+/* pdrive with the interzone cross smoothing (pdrive_at per replica) */
 __global__ void __launch_bounds__(TPB) k_ens_pdrive(const EnsRep* __restrict__ reps, const int* __restrict__ coff,
                                                     int R, int C, const double* __restrict__ raw,
                                                     const int* __restrict__ mask, double* __restrict__ pd) {
@@ -278,7 +278,7 @@ __global__ void __launch_bounds__(TPB) k_ens_pdrive(const EnsRep* __restrict__ r
     pd[c] = v;
 }
 
-/* duEOS (k_eos per replica) */
+/* duEOS (k_eos_beta's, per replica) */
 __global__ void __launch_bounds__(TPB) k_ens_eos(const EnsRep* __restrict__ reps, const int* __restrict__ coff, int R,
                                                  int C, const double* __restrict__ pdr, double* __restrict__ exo,
                                                  double* __restrict__ eyo) {
@@ -452,8 +452,8 @@ struct mpcd_gpu_ensemble {
     unsigned long long* key = nullptr;
     int *startB = nullptr, *listB = nullptr;
     unsigned long long* keyB = nullptr;
-    /* the passes' record of moved particles: departures and arrivals per cell,
-     * each arrival's rank (-1 for every slot between updates) */
+    /* the passes' record of moved particles: departures and arrivals per cell
+     * (zero between updates, as the length of the list of arrivals) */
     int *dout = nullptr, *inc = nullptr, *arrN = nullptr;
     int2* arr = nullptr; /* the arrivals a pass listed, arrN of them */
     unsigned long long* zcur = nullptr; /* k_zone_fused's region counter */
@@ -578,8 +578,7 @@ struct mpcd_gpu_ensemble {
         narrow = maxN < (1 << 27) ? 1 : 0;
         /* the fused zone kernel on 16-bit working sets must take every zone */
         const size_t fix16 = zone_fixed_bytes<uint16_t>(maxC, maxW, anyLocal);
-        const size_t cellB16 = (size_t)maxC * (sizeof(ZCell<uint16_t>) + sizeof(uint16_t)) + 8 * (size_t)maxW + 16;
-        if (!(maxC < 65535 && fix16 + 2048 <= (size_t)ZONE_LDS_FAST && cellB16 + 4096 <= (size_t)ZONE_LDS_FAST))
+        if (!(maxC < 65535 && fix16 + 2048 <= (size_t)ZONE_LDS_FAST))
             throw ApiError(MPCD_E_INVALID, "ensemble zones must fit the fused zone kernel (zone tiles too large)");
         HIP_OK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         /* tables */

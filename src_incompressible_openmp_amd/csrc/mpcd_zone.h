@@ -1,6 +1,7 @@
 /*
  * mpcd_zone.h -- one zone of the snapshot zone redistribution
- * (zone_pass.cpp:62-973), shared by the gfx950 kernels in mpcd_engine.hip and the host logic check in tests/ (ZHD code).
+ * (zone_pass.cpp:62-973), shared by the gfx950 kernels in mpcd_engine.hip and
+ * the host logic check in tests/ (ZHD code).
  *
  * The reference's zone kernel is sequential: a shuffled list of dense cells,
  * each of which mutates the counts its successors read.  That order is kept;
@@ -16,7 +17,8 @@
  * visits every particle in its final cell, writes the new positions from
  * that record.  The fused kernel (zones with 16-bit indices) runs the passes
  * on four wavefronts and the correction behind them, the zone's state staying
- * in LDS; the two-kernel form hands it over in global memory (ZoneState).
+ * in LDS; the form with 32-bit indices runs the passes on one wavefront and
+ * hands the state over in global memory (ZoneState) to the correction on four.
  *
  * Memory.  Cell arrays are indexed by the zone-local cell
  * lc = (ix-xs)*zh + (iy-ys) (ascending global cell id); particles by the
@@ -1103,12 +1105,6 @@ ZHD int spread(Z& z, int src, int needOut, int pass, int* rv, int& nr) {
 
 /* value held by lane src (per-lane src) */
 ZHD int lane_get(int v, int src) { return __shfl(v, src, 64); }
-ZHD double lane_get_d(double v, int src) { return __shfl(v, src, 64); }
-ZHD unsigned long long lane_get_u64(unsigned long long v, int src) {
-    const unsigned lo = (unsigned)__shfl((int)(unsigned)v, src, 64);
-    const unsigned hi = (unsigned)__shfl((int)(unsigned)(v >> 32), src, 64);
-    return ((unsigned long long)hi << 32) | lo;
-}
 /* every lane's v to lane dst (dst a permutation of the lanes) */
 ZHD int lane_put(int v, int dst) { return __builtin_amdgcn_ds_permute(dst << 2, v); }
 ZHD double lane_put_d(double v, int dst) {
@@ -1614,7 +1610,7 @@ __device__ __forceinline__ int zone_compact_mw(Z& z, const unsigned long long* c
  * cell sets its word in done (both in ext, idle in the dense passes).
  * Conflicting cells thus keep the list order and the result is the serial
  * loop's bit for bit, while a wavefront waits only for the cells its own
- * depends on, after everything that does not depend on them (dense_prep).
+ * depends on, after everything that does not depend on them.
  * Cells are taken in increasing order and wait only on smaller positions,
  * which are taken already, so the smallest unfinished cell can always run;
  * each wait is bounded all the same (past DS_WAIT_MAX polls it records
@@ -2826,18 +2822,6 @@ ZHD void fin_write(Z& z, int sl, unsigned short ow, bool corr, double vx, double
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)
-/* Phase 2 for changed, occupied cell lc on a group of FIN_G consecutive
- * lanes (r: the lane's rank; every lane of the group passes the same cell).
- * Every entry's link is set to lc, its final cell, once the walk has read
- * it: phase 3 reads the links of the moved particles, and nothing reads the
- * others.
- * The group takes the final list FIN_G * FIN_L entries at a time, lane r
- * entries [FIN_L r, FIN_L (r + 1)) of each chunk, so a list of up to
- * FIN_G * FIN_L entries has each slot and velocity loaded once instead of
- * once per pass.  The momentum sums keep the list order: lane r adds its
- * entries to the running sum lane r - 1 hands on.  A linked list is walked by
- * the whole group in step.  pbx, pby: the cell's input-run momentum.  Returns
- * |du|^2 (the same on every lane of the group). */
 /* Phase 1 for changed, occupied cell lc on a group of FIN_G lanes: the
  * momentum of its input run (the particles binned into it, before the
  * passes), FIN_G * FIN_L entries at a time, summed in run order as
@@ -2905,6 +2889,18 @@ __device__ __forceinline__ void fin_group_entries(const Z& z, FinWalk& w, int m,
     }
 }
 
+/* Phase 2 for changed, occupied cell lc on a group of FIN_G consecutive
+ * lanes (r: the lane's rank; every lane of the group passes the same cell).
+ * Every entry's link is set to lc, its final cell, once the walk has read
+ * it: phase 3 reads the links of the moved particles, and nothing reads the
+ * others.
+ * The group takes the final list FIN_G * FIN_L entries at a time, lane r
+ * entries [FIN_L r, FIN_L (r + 1)) of each chunk, so a list of up to
+ * FIN_G * FIN_L entries has each slot and velocity loaded once instead of
+ * once per pass.  The momentum sums keep the list order: lane r adds its
+ * entries to the running sum lane r - 1 hands on.  A linked list is walked by
+ * the whole group in step.  pbx, pby: the cell's input-run momentum.  Returns
+ * |du|^2 (the same on every lane of the group). */
 template <class Z>
 __device__ __forceinline__ double fin_cell_group(Z& z, int lc, int r, int lane, double pbx, double pby) {
     constexpr int CH = FIN_G * FIN_L;

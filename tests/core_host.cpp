@@ -93,7 +93,7 @@ extern "C" int core_collide(const mpcd_params* p, double* va, const int32_t* cid
     return 0;
 }
 
-/* One zone of a pass, as k_zone runs it, with working-set index type IT and
+/* One zone of a pass, as the kernels run it, with working-set index type IT and
  * `bytes` of working set (links beyond it go to the zone's global region). */
 template <class IT>
 void run_zone(const ZoneIn& in, ZoneRect r, int zid, uint64_t seed, size_t bytes, std::vector<IT>& nxG,
