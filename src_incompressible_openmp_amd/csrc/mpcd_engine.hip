@@ -1279,7 +1279,7 @@ __device__ __forceinline__ void zone_uniform(Z& z) {
     make_uniform(z.g.Nx, z.g.Ny, z.g.Nc, z.g.n, z.g.perx, z.g.pery, z.g.Lx, z.g.Ly, z.g.a0, z.g.dxc, z.g.dyc);
     make_uniform(z.zp.highThr, z.zp.lowThrBulk, z.zp.lowFrac, z.zp.highFrac, z.zp.gamma, z.zp.fluidFracGain,
                  z.zp.lowThrFloor, z.zp.highThrFloor, z.zp.lowLoc1, z.zp.highLoc1, z.zp.useLocal, z.zp.maxPasses,
-                 z.zp.corrEnabled, z.zp.dedupe, z.zp.quadBins, z.zp.binLo, z.zp.binHi);
+                 z.zp.corrEnabled, z.zp.dedupe, z.zp.odd, z.zp.quadBins, z.zp.binLo, z.zp.binHi);
     make_uniform(z.xs, z.xe, z.ys, z.ye, z.zw, z.zh, z.C, z.zhM, z.zid, z.seed, z.gcnt, z.gstart, z.glist, z.gkey, z.x,
                  z.y, z.vx, z.vy, z.vsx, z.vsy, z.gchg, z.inPx, z.inPy, z.dcid, z.dout, z.dinc, z.darr, z.darrN, z.cellOff, z.dgCell,
                  z.dgCnt);
@@ -1329,9 +1329,12 @@ __device__ __forceinline__ void zone_region_done(const ZoneArgs& a) {
  * CU): all four wavefronts run the set-up, the scheduled dense and sparse
  * phases, then the correction, which takes the zone over in LDS where the
  * passes left it.  A zone's correction starts as soon as its own passes
- * end, beside the passes of slower zones. */
+ * end, beside the passes of slower zones.
+ * kOdd: narrow periodic axes and unordered thresholds (ZoneParams::odd) are
+ * looked for; the ordinary form drops what that takes (a step of
+ * 106 x 76 x 5 948 us with it, by scalar spills, and 905 without). */
 constexpr int FUSED_TPB = 256;
-template <class IT, bool kEns = false>
+template <class IT, bool kEns = false, bool kOdd = false>
 __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 waves per SIMD: four zones per CU */
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ ZoneShared sh;
@@ -1361,6 +1364,10 @@ __global__ void __launch_bounds__(FUSED_TPB, 4) k_zone_fused(ZoneArgs a) { /* 4 
     const ZoneIn& in = *inp;
     zone_init(z, in, a.rects[zi], zid, seed, &sh);
     if constexpr (kEns) zone_uniform(z);
+    if constexpr (!kOdd) {
+        z.zp.odd = z.zp.dedupe = 0;
+        z.zp.quadBins = 1;
+    }
     z.duG = a.duG + (size_t)zi * (size_t)a.duStride;
     zone_carve(z, lds, a.ldsBytes);
     static_assert(FUSED_TPB == 256, "the set-up and the phases take four wavefronts");
@@ -2618,7 +2625,10 @@ struct mpcd_gpu_sim {
             a.pMin = 0;
             a.pMax = 65534;
             a.ldsBytes = ZONE_LDS_FAST;
-            hipLaunchKernelGGL((k_zone_fused<uint16_t>), dim3(nZ), dim3(FUSED_TPB), ZONE_LDS_FAST, stream, a);
+            if (zp.odd)
+                hipLaunchKernelGGL((k_zone_fused<uint16_t, false, true>), dim3(nZ), dim3(FUSED_TPB), ZONE_LDS_FAST, stream, a);
+            else
+                hipLaunchKernelGGL((k_zone_fused<uint16_t>), dim3(nZ), dim3(FUSED_TPB), ZONE_LDS_FAST, stream, a);
             check_launch();
         }
         pend(MPCD_PROF_ZONE_KERNEL);

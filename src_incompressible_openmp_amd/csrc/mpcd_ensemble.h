@@ -458,6 +458,7 @@ struct mpcd_gpu_ensemble {
     int2* arr = nullptr; /* the arrivals a pass listed, arrN of them */
     unsigned long long* zcur = nullptr; /* k_zone_fused's region counter */
     int nTiles = 0, narrow = 1, cellCap = 256;
+    int anyOdd = 0; /* a replica needs the zone kernel's kOdd form, whose other replicas it serves alike */
     /* cells */
     double *refPx = nullptr, *refPy = nullptr, *refUx = nullptr, *refUy = nullptr, *pdriveRaw = nullptr;
     double *redPx = nullptr, *redPy = nullptr, *redUx = nullptr, *redUy = nullptr;
@@ -553,7 +554,9 @@ struct mpcd_gpu_ensemble {
             b += e.nbc;
             maxN = std::max(maxN, p.n);
             maxPpc = std::max(maxPpc, (double)p.n / (double)p.Nc);
-            anyLocal |= make_zone_params(p).useLocal;
+            const ZoneParams zp = make_zone_params(p);
+            anyLocal |= zp.useLocal;
+            anyOdd |= zp.odd;
             for (int L = 0; L < 2; ++L) {
                 std::vector<int32_t> own;
                 lr[L].push_back(layout_rects(p, L == 0 ? MPCD_LAYOUT_BASE : MPCD_LAYOUT_SHIFTED, &own));
@@ -824,7 +827,10 @@ struct mpcd_gpu_ensemble {
         a.ensIn = ensIn[parity][L];
         a.ensSeed = zseed + (size_t)L * R;
         a.ensZoneOff = zoneOff[L];
-        hipLaunchKernelGGL((k_zone_fused<uint16_t, true>), dim3(nz), dim3(FUSED_TPB), ZONE_LDS_FAST, stream, a);
+        if (anyOdd)
+            hipLaunchKernelGGL((k_zone_fused<uint16_t, true, true>), dim3(nz), dim3(FUSED_TPB), ZONE_LDS_FAST, stream, a);
+        else
+            hipLaunchKernelGGL((k_zone_fused<uint16_t, true>), dim3(nz), dim3(FUSED_TPB), ZONE_LDS_FAST, stream, a);
         check_launch();
         pendCopy = nOver[L] > 0 ? CopybackArgs{overCells[L], nOver[L], chg, start, list, vx2, vy2, vx, vy} : CopybackArgs{};
     }

@@ -185,6 +185,9 @@ inline ZoneParams make_zone_params(const mpcd_params& p) {
                       (p.bc_bottom == MPCD_BC_PERIODIC && p.bc_top == MPCD_BC_PERIODIC && p.Ny < 3)) &&
                      zp.lowThrBulk > zp.highThr;
     zp.quadBins = !own && apart && *std::max_element(perBin, perBin + 8) <= 3;
+    /* (negated, so that a NaN counts as odd) */
+    zp.odd = zp.dedupe || !zp.quadBins || !(zp.lowThrBulk <= zp.highThr) || !(zp.highThr >= 0.0) || !(zp.highLoc1 >= 0.0) ||
+             !(zp.highFrac >= 0.0 || zp.highThrFloor >= 0.0);
     return zp;
 }
 

@@ -135,6 +135,7 @@ struct ZoneParams {
     double lowLoc1, highLoc1; /* empty-cell thresholds for fluid fraction 1 */
     int useLocal, maxPasses, corrEnabled;
     int dedupe; /* a periodic axis narrower than 5 cells: wrapped neighbours can repeat */
+    int odd;    /* dedupe, or thresholds below zero or the low one above the high one: k_zone_fused's kOdd form */
     int quadBins; /* at most 3 neighbour offsets per angular bin, no two of a bin equally far (the wavefront form's
                    * lane layout, in which no tie is left to a draw), and no dense cell its own target */
     /* angular bin (3 bits) of (dx,dy) in [-2,2]^2 at index (dy+2)*5+(dx+2):
@@ -1128,6 +1129,35 @@ ZHD unsigned long long quad_rot64(unsigned long long v) {
 }
 ZHD int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+/* a periodic axis whose wrapped range-2 neighbours can lie in the zone */
+template <class Z>
+ZHD bool zone_wrap_x(const Z& z) {
+    return z.g.perx && z.zw >= z.g.Nx - 1;
+}
+template <class Z>
+ZHD bool zone_wrap_y(const Z& z) {
+    return z.g.pery && z.zh >= z.g.Ny - 1;
+}
+/* zone-relative coordinate t taken once around an axis of n cells */
+ZHD int wrap_near(int t, int n) { return t < 0 ? t + n : (t >= n ? t - n : t); }
+/* Below five cells several offsets lead to one cell of a periodic axis, and
+ * min_step's alone stands for it: the candidates come out as the general
+ * form's dedupe leaves them, whose keys are those of the shortest step.  An
+ * offset past half the axis never is; one that wraps is if it is under half
+ * (at half of it the one that stays on the axis).  (On one wavefront in the
+ * general form a launch of 4 x 1024 x 20 took 216 us, on the four 56; one of
+ * 5 x 1024 x 20 takes 60.) */
+template <class Z>
+ZHD bool past_half(const Z& z, int dx, int dy) {
+    return z.zp.odd && ((z.g.perx && 2 * (dx < 0 ? -dx : dx) > z.g.Nx) || (z.g.pery && 2 * (dy < 0 ? -dy : dy) > z.g.Ny));
+}
+template <class Z>
+ZHD bool wrap_step(const Z& z, int d, int& t, int n) {
+    const int t0 = t;
+    t = wrap_near(t, n);
+    return !z.zp.odd || t == t0 || 2 * (d < 0 ? -d : d) < n;
+}
+
 /* A dense cell's ranking lives in lanes by angular bin: lanes 4 b + m and
  * 32 + 4 b + m (m < 3) hold the m-th neighbour offset of bin b, the first for
  * the low thresholds (phase 0), the second for the high ones (phase 1).  A
@@ -1149,34 +1179,13 @@ ZHD DenseLane dense_lane(const Z& z, int lane) {
             d.dy = idx / 5 - 2;
             const int ax = d.dx < 0 ? -d.dx : d.dx, ay = d.dy < 0 ? -d.dy : d.dy;
             d.code = (imax(ax, ay) << 4) | (ax * ax + ay * ay);
+            if (past_half(z, d.dx, d.dy)) d.code = -1;
         }
         ++seen;
     }
     d.thB = lane < 32 ? z.zp.lowThrBulk : z.zp.highThr;
     d.thE = lane < 32 ? z.zp.lowLoc1 : z.zp.highLoc1;
     return d;
-}
-
-/* a periodic axis whose wrapped range-2 neighbours can lie in the zone */
-template <class Z>
-ZHD bool zone_wrap_x(const Z& z) {
-    return z.g.perx && z.zw >= z.g.Nx - 1;
-}
-template <class Z>
-ZHD bool zone_wrap_y(const Z& z) {
-    return z.g.pery && z.zh >= z.g.Ny - 1;
-}
-/* zone-relative coordinate t taken once around an axis of n cells */
-ZHD int wrap_near(int t, int n) { return t < 0 ? t + n : (t >= n ? t - n : t); }
-/* Offset d to the (not yet wrapped) coordinate t is min_step's on a periodic
- * axis of n cells.  Below five cells several offsets lead to one cell, and
- * this one alone stands for it: the candidates come out as the general form's
- * dedupe leaves them, whose keys are those of the shortest step.  (On one
- * wavefront in the general form a launch of 4 x 1024 x 20 took 216 us, on the
- * four 56; one of 5 x 1024 x 20 takes 60.) */
-ZHD bool shortest_step(int d, int t, int n) {
-    const int a = 2 * (d < 0 ? -d : d);
-    return a < n || (a == n && (unsigned)t < (unsigned)n);
 }
 
 /* A dense cell's surplus over its high threshold (an occupied cell's is the
@@ -1191,24 +1200,30 @@ ZHD int dense_need(const Z& z, int nc) {
 template <class Z>
 ZHD bool dense_count_fits(const Z& z, int nc) {
     const int need = dense_need(z, nc);
-    return need > 0 && need <= ZONE_MAX_MOVE && imin(need + 1, nc) <= ZONE_MAX_MOVE;
+    return imin(need + 1, nc) <= ZONE_MAX_MOVE && (!z.zp.odd || (need > 0 && need <= ZONE_MAX_MOVE));
 }
 /* (a cell that was empty when the pass took its thresholds has another than
  * dense_need's) */
 template <class Z>
 ZHD bool dense_fits(const Z& z, int c, int nc) {
-    return dense_count_fits(z, nc) && fget(z, c, ZF_BULK0);
+    return dense_count_fits(z, nc) && (!z.zp.odd || fget(z, c, ZF_BULK0));
 }
 template <class Z>
 ZHD unsigned dense_bins(const Z& z, int c, int pass) {
     const uint32_t gc = (uint32_t)lc_gc(z, c);
     return (unsigned)mpcd_draw_start_bin(z.seed, pass, 0, gc) | ((unsigned)mpcd_draw_start_bin(z.seed, pass, 1, gc) << 3);
 }
+/* a dense cell can receive: the low threshold lies above the high one */
+template <class Z>
+ZHD bool dense_receives(const Z& z) {
+    return z.zp.odd && z.zp.lowThrBulk > z.zp.highThr;
+}
 /* both in the cell's lix entry (the surplus of a cell whose movers fit the
- * wavefront is below 64) */
+ * wavefront is 1 to 64; 0: it can still grow and is taken later) */
 template <class Z>
 ZHD void dense_word(Z& z, int c, int pass) {
-    z.lix[c] = (typename Z::idx_t)((unsigned)dense_need(z, cnt_of(z, c)) | (dense_bins(z, c, pass) << 7));
+    const int need = dense_receives(z) ? 0 : dense_need(z, cnt_of(z, c));
+    z.lix[c] = (typename Z::idx_t)((unsigned)need | (dense_bins(z, c, pass) << 7));
 }
 
 /* lanes of `half` set in a ballot, as 32 bits */
@@ -1352,14 +1367,8 @@ ZHD int dense_cell_wave(Z& z, const DenseLane& dl, int c, int cx, int cy, int ne
     typedef typename Z::idx_t IT;
     int tx = cx + dl.dx, ty = cy + dl.dy;
     bool in = dl.code >= 0;
-    if (zone_wrap_x(z)) {
-        if (z.zp.dedupe) in = in & shortest_step(dl.dx, tx, z.g.Nx);
-        tx = wrap_near(tx, z.g.Nx);
-    }
-    if (zone_wrap_y(z)) {
-        if (z.zp.dedupe) in = in & shortest_step(dl.dy, ty, z.g.Ny);
-        ty = wrap_near(ty, z.g.Ny);
-    }
+    if (zone_wrap_x(z)) in = in & wrap_step(z, dl.dx, tx, z.g.Nx);
+    if (zone_wrap_y(z)) in = in & wrap_step(z, dl.dy, ty, z.g.Ny);
     in = in & ((unsigned)tx < (unsigned)z.zw) & ((unsigned)ty < (unsigned)z.zh);
     const int l = in ? tx * z.zh + ty : c;
     const ZCell<IT> S = z.cell[c];
@@ -1655,8 +1664,6 @@ __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
     IT* const pos = z.ext;
     volatile IT* const done = z.ext + z.C;
     unsigned long long* const chunkMask = reinterpret_cast<unsigned long long*>(z.scr->cand); /* idle here */
-    const bool late = z.zp.lowThrBulk > z.zp.highThr;
-    const bool form = z.zp.quadBins && (!late || dense_count_fits(z, (int)MPCD_CEIL(z.zp.lowThrBulk)));
     for (int pass = 1; pass <= z.zp.maxPasses; ++pass) {
         /* thresholds and the list: chunk ch of 64 cells on wavefront ch % 4 */
         bool one = false;
@@ -1674,7 +1681,8 @@ __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
             if (lane == 0) chunkMask[ch] = msk;
         }
         for (int k = z.C + tid; k < nExt; k += NT) z.ext[k] = (IT)0;
-        bool serial = __syncthreads_or(one) || !form;
+        bool serial = __syncthreads_or(one) || !z.zp.quadBins ||
+                      (dense_receives(z) && !dense_count_fits(z, (int)MPCD_CEIL(z.zp.lowThrBulk)));
         const int m = zone_compact_mw(z, chunkMask, wave, lane);
         serial = serial || m + z.C > nExt;
         __syncthreads();
@@ -1733,7 +1741,8 @@ __device__ __forceinline__ void zone_dense_passes_mw(Z& z, int wave, int lane) {
                         __builtin_amdgcn_s_sleep(1);
                     }
                     sched_acquire(z);
-                    const int need = late ? uniform(dense_need(z, cnt_of(z, c))) : (int)(nb & 127u);
+                    int need = (int)(nb & 127u);
+                    if (z.zp.odd && need == 0) need = uniform(dense_need(z, cnt_of(z, c)));
                     movedW += dense_cell_wave(z, dlane, c, cx, cy, need, nb >> 7, pass, lane);
                     sched_release(z);
                     if (lane == 0) done[k] = (IT)1;
@@ -2044,14 +2053,8 @@ __device__ __forceinline__ int sparse_neighbour(const Z& z, int cx, int cy, int 
     dx = f - 3 * (f / 3) - 1;
     int tx = cx + dx, ty = cy + dy;
     bool in = o < 8;
-    if (zone_wrap_x(z)) {
-        if (z.zp.dedupe) in = in & shortest_step(dx, tx, z.g.Nx);
-        tx = wrap_near(tx, z.g.Nx);
-    }
-    if (zone_wrap_y(z)) {
-        if (z.zp.dedupe) in = in & shortest_step(dy, ty, z.g.Ny);
-        ty = wrap_near(ty, z.g.Ny);
-    }
+    if (zone_wrap_x(z)) in = in & wrap_step(z, dx, tx, z.g.Nx);
+    if (zone_wrap_y(z)) in = in & wrap_step(z, dy, ty, z.g.Ny);
     in = in & ((unsigned)tx < (unsigned)z.zw) & ((unsigned)ty < (unsigned)z.zh);
     return in ? tx * z.zh + ty : -1;
 }

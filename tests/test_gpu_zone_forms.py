@@ -166,3 +166,27 @@ def test_low_threshold_above_high(gpu, oracle, low, crowded):
         assert g["nParticlesMovedSparse"] == m["nParticlesMovedSparse"], layout
         assert x.tobytes() == xo.tobytes(), layout
         assert v.tobytes() == vo.tobytes(), layout
+
+
+def test_both_instantiations_agree(gpu):
+    """One replica with a narrow axis sends an ensemble to the zone kernel's
+    form that looks for it: its other replicas, local thresholds and wrapped
+    zones among them, follow their single simulations, which take the other."""
+    forms = [dict(Nx=4, Ny=30, gamma=10.0), dict(Nx=60, Ny=40, gamma=5.0), dict(FORMS["wrap_gap_of_one"]),
+             dict(FORMS["local_thresholds"]), dict(FORMS["low_above_high"]), dict(FORMS["wrap_full_axis"])]
+    ps = [to_struct(poiseuille_params(**f)) for f in forms]
+    st = [state(p, False) for p in ps]
+    ens = gpu.Ensemble(ps, list(range(len(ps))))
+    for r, (x, v) in enumerate(st):
+        ens.set_state(r, x, v)
+    ens.step(1, 3)
+    got = [ens.get_state(r) for r in range(len(ps))]
+    ens.close()
+    for r, p in enumerate(ps):
+        sim = gpu.Sim(p)
+        sim.set_seed_key(r)
+        sim.set_state(*st[r])
+        sim.step(1, 3)
+        x, v = sim.get_state()
+        sim.close()
+        assert np.array_equal(got[r][0], x) and np.array_equal(got[r][1], v), r
