@@ -80,10 +80,13 @@ class HostCopy {
    public:
     /* Down, two threads' worth of chunks: 8 MiB take 0.35 ms chunked, 0.51 not
      * (the threads' start costs what is gained below).  The runtime's uploads
-     * are three times as fast, so chunks pay later: 8 MiB take 0.30 ms
-     * chunked, 0.25 not, 10 MiB 0.35 and 0.32, 12 MiB 0.41 and 0.40, 16 MiB
-     * 0.52 and 0.56. */
-    static constexpr size_t DOWN_MIN = 4 * PinnedChunks::BYTES, UP_MIN = 8 * PinnedChunks::BYTES;
+     * are three times as fast, so chunks pay later.  Arrays uploaded again and
+     * again: 8 MiB take 0.30 ms chunked, 0.25 not, 10 MiB 0.34 and 0.30, 14 MiB
+     * 0.46 and 0.42, 16 MiB 0.51 both, 20 MiB 0.62 and 0.69.  New arrays at each
+     * call, the program that calls the stages one by one: a step with arrays of
+     * 8.2 MiB takes 11.2 ms chunked, 10.8 not, of 10 MiB 12.0 and 12.2, of 14.3
+     * MiB 17.1 and 17.3.  The line is the latter's. */
+    static constexpr size_t DOWN_MIN = 4 * PinnedChunks::BYTES, UP_MIN = 5 * PinnedChunks::BYTES;
 
     HostCopy() { PinnedChunks::instance().lease(); }
     ~HostCopy() { PinnedChunks::instance().release(); }

@@ -1,5 +1,5 @@
 """Host arrays to the device and back around the sizes where a copy is cut into
-chunks (8 MiB down, 16 MiB up: 524,288 and 1,048,576 particles of two doubles),
+chunks (8 MiB down, 10 MiB up: 524,288 and 655,360 particles of two doubles),
 at sizes that leave partial chunks, from one thread and from several with an
 object each: every byte."""
 import ctypes
