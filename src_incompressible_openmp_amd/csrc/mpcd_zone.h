@@ -836,8 +836,8 @@ ZHD void zone_shuffle(T* a, int m, int lane, int nl, ShufDraw draw) {
     if (m <= 128) {
         /* elements q and 64 + q in lane q's registers: a swap is two reads
          * and two writes of single lanes.  (A list in LDS instead makes each
-         * swap two dependent accesses of one lane, about 250 cycles against
-         * 40; a zone of 25 x 25 cells has 50 to 80 dense cells.) */
+         * swap two dependent accesses of one lane, 259 cycles against 31;
+         * a zone of 25 x 25 cells has 50 to 80 dense cells.) */
         int v0 = lane < m ? (int)a[lane] : 0, v1 = 0, j1 = 0;
         const int j0 = (lane >= 1 && lane < m) ? (int)draw((uint32_t)lane) : 0;
         if (m > 64) {
